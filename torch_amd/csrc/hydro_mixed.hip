@@ -640,8 +640,13 @@ __global__ void mixed_scale_rotate_kernel(StepState* st) {
 }
 
 // Largest density and pressure (after the floors of fixPrimitives) over the
-// grid into qmax_next, one atomicMax per wave.
+// grid into qmax_next.  Bound by reading U (56 B per cell).  Atomics on one
+// address retire about one per 12 ns here, and one pair per wave (16,384
+// waves) took 378 us on a 1.7 M-cell grid whatever its size: each block now
+// reduces in LDS and thread 0 only issues an atomicMax that can raise the
+// record (a stale read costs an extra atomic, never a lost maximum).
 __global__ __launch_bounds__(256) void state_max_kernel(HydroGeom g, const double* __restrict__ U, StepState* st) {
+    __shared__ unsigned int red[4][2];
     unsigned int mr = 0, mp = 0;
     for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < g.ncell;
          c += (long long)gridDim.x * blockDim.x) {
@@ -659,8 +664,15 @@ __global__ __launch_bounds__(256) void state_max_kernel(HydroGeom g, const doubl
         mp = max(mp, (unsigned int)__shfl_xor((int)mp, off, 64));
     }
     if ((threadIdx.x & 63) == 0) {
-        if (mr) atomicMax(&st->qmax_next[0], mr);
-        if (mp) atomicMax(&st->qmax_next[1], mp);
+        red[threadIdx.x >> 6][0] = mr;
+        red[threadIdx.x >> 6][1] = mp;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const int j = threadIdx.x;
+        const unsigned int m = max(max(red[0][j], red[1][j]), max(red[2][j], red[3][j]));
+        if (m > __hip_atomic_load(&st->qmax_next[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(&st->qmax_next[j], m);
     }
 }
 
@@ -668,7 +680,7 @@ hipError_t launch_mixed_scale_seed(const HydroGeom& g, const double* U, StepStat
     // clear the record, reduce the grid into it, make it the scale
     hipLaunchKernelGGL(mixed_scale_rotate_kernel, dim3(1), dim3(1), 0, stream, st);
     long long nb = (g.ncell + 255) / 256;
-    if (nb > 4096) nb = 4096;
+    if (nb > 2048) nb = 2048;
     hipLaunchKernelGGL(state_max_kernel, dim3((unsigned)nb), dim3(256), 0, stream, g, U, st);
     hipLaunchKernelGGL(mixed_scale_rotate_kernel, dim3(1), dim3(1), 0, stream, st);
     return hipGetLastError();
