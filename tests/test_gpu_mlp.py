@@ -14,7 +14,7 @@ from torch_amd import cooling_inputs
 pytestmark = pytest.mark.gpu
 
 
-def _setup(seed=0, B=512):
+def _setup(seed=0, B=512, max_batch=4096):
     import torch
 
     from torch_amd import surrogate as sg
@@ -25,7 +25,7 @@ def _setup(seed=0, B=512):
     f = np.zeros((B, 8), np.float32)
     f[:, :6] = rng.normal(0, 1, (B, 6))
     t = rng.normal(0, 1, (B, 3)).astype(np.float32)
-    m = sg.MLP(max_batch=4096)
+    m = sg.MLP(max_batch=max_batch)
     m.set_params(W, b)
     Ws, bs = sg.unpack(W, b)
     p = {f"W{L + 1}": Ws[L] for L in range(5)}
@@ -47,6 +47,28 @@ def test_mlp_gradients_match_cpu_reference(gpu):
             ref = g[name]
             err = np.linalg.norm(got - ref) / max(np.linalg.norm(ref), 1e-30)
             assert err < 1e-3, (name, err)
+
+
+@pytest.mark.parametrize("B", [1, 16, 17, 33, 4096 + 31, 32768 + 129])
+def test_mlp_kernels_at_tile_edges(gpu, B):
+    """Batches around the 16-cell tiles, the 32-cell blocks of the weight
+    gradients and (last) more tiles than waves in flight.  An operand that the
+    FP32 and the FP64 sums round to different bfloat16 neighbours is off by
+    2^-8 of itself; with one cell it can be a whole row of a gradient."""
+    from torch_amd import surrogate as sg
+
+    m, p, f, t, fd, td = _setup(seed=11, B=B, max_batch=B)
+    y = m.forward(fd).cpu().numpy()
+    yr, _ = omlp.forward(p, f.astype(np.float64))
+    assert np.abs(y - yr).max() / np.abs(yr).max() < 2.0 ** -8
+    loss, gW, gb = m.loss_grad(fd, td)
+    ref_loss, g, _ = omlp.loss_and_grads(p, f.astype(np.float64), t.astype(np.float64), np.ones(3))
+    assert abs(loss - ref_loss) / ref_loss < 2.0 ** -8
+    Ws, bs = sg.unpack(gW, gb)
+    for L in range(5):
+        for name, got in ((f"W{L + 1}", Ws[L]), (f"b{L + 1}", bs[L])):
+            err = np.linalg.norm(got - g[name]) / max(np.linalg.norm(g[name]), 1e-30)
+            assert err < 2.0 ** -8, (name, err)
 
 
 def test_mlp_fused_inference_matches_reference(gpu):

@@ -999,7 +999,7 @@ static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 
 // the MLP handle is defined in mlp_api.cpp; the cooling operator only needs
 // its device weights
-extern "C" int torchgpu_mlp_device_weights(torchgpu_mlp* m, const uint16_t** w16, const float** b);
+extern "C" int torchgpu_mlp_device_weights(torchgpu_mlp* m, const uint16_t** packed, const float** b);
 
 namespace {
 
