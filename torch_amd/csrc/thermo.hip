@@ -61,8 +61,7 @@ struct CellState {
 // cell's heating rate and pre-step RATE as this function computed them on
 // the same state (pre_rate[pidx], pre_rate[pn + pidx]; thermo_timestep_kernel
 // stores them), taken instead of evaluating them again.
-__device__ __forceinline__ bool thermo_init(const ThermoConsts& t, const double* sx, const double* sy,
-                                            const double* sy2, const double* in, long long stride, long long cell,
+__device__ __forceinline__ bool thermo_init(const ThermoConsts& t, const double* tab, const double* in, long long stride, long long cell,
                                             CellState& s, unsigned int* err, const double* pre_rate = nullptr,
                                             long long pidx = 0, long long pn = 0) {
     const double den = in[0 * stride + cell], pre = in[1 * stride + cell], hii = in[2 * stride + cell];
@@ -84,15 +83,15 @@ __device__ __forceinline__ bool thermo_init(const ThermoConsts& t, const double*
     const double T = (pre / den) * (1.0 / mu_inv) / t.spec_gas_const;  // Fluid::calcTemperature
     const double Av = 1.086 * t.dust_xsec * col_den;
     s.T0 = T;
-    s.cc = cooling_cell(t, nH, x);
+    s.cc = cooling_cell(t, tab, nH, x);
     double RATE;
     if (pre_rate) {
         s.heat = pre_rate[pidx];
         RATE = pre_rate[pn + pidx];
     } else {
-        double rate = heating(t, nH, Av, F);
+        double rate = heating(t, tab, nH, Av, F);
         s.heat = rate;
-        rate = subtract_cooling(t, s.cc, sx, sy, sy2, rate, T);
+        rate = subtract_cooling(t, s.cc, tab, rate, T);
         rate = soft_landing(rate, T, T_min);
         RATE = t.heating_amplification * rate;
     }
@@ -129,9 +128,8 @@ __device__ __forceinline__ bool thermo_init(const ThermoConsts& t, const double*
 }
 
 // One subcycle, :314-330.
-__device__ __forceinline__ void thermo_substep(const ThermoConsts& t, const double* sx, const double* sy,
-                                               const double* sy2, CellState& s) {
-    double r = subtract_cooling(t, s.cc, sx, sy, sy2, s.heat, s.subT);
+__device__ __forceinline__ void thermo_substep(const ThermoConsts& t, const double* tab, CellState& s) {
+    double r = subtract_cooling(t, s.cc, tab, s.heat, s.subT);
     r = t.heating_amplification * soft_landing(r, s.subT, s.T_min);
     double pressure = s.pressure + r * s.rate2dpre;
     double subT = pressure * s.pre2temp;
@@ -173,7 +171,15 @@ __device__ __forceinline__ long long wave_append(bool pred, unsigned long long* 
     return pred ? base + __popcll(mask & ((1ull << lane) - 1ull)) : -1;
 }
 
-__device__ __forceinline__ void load_tables(const double* tables, double* sx, double* sy, double* sy2) {
+// The rate tables (behind the spline's x, y, y2 in `tables`) into LDS; every
+// thread of the block calls it.
+__device__ __forceinline__ void load_tables(const double* __restrict__ tables, double* tab) {
+    for (int i = threadIdx.x; i < TT_N; i += blockDim.x) tab[i] = tables[78 + i];
+    __syncthreads();
+}
+
+// The spline's knots and second derivatives, as heating_terms reads them.
+__device__ __forceinline__ void load_spline(const double* __restrict__ tables, double* sx, double* sy, double* sy2) {
     if (threadIdx.x < 26) {
         sx[threadIdx.x] = tables[threadIdx.x];
         sy[threadIdx.x] = tables[26 + threadIdx.x];
@@ -191,10 +197,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
                                                           const double* __restrict__ in, double* __restrict__ out,
                                                           unsigned long long* __restrict__ counters,
                                                           unsigned int* __restrict__ err, unsigned char* path) {
-    __shared__ double sx[26], sy[26], sy2[26];
+    __shared__ double tab[TT_N];
     if (count_dev) count = (long long)*count_dev;
     if (count <= 0) return;  // an empty queue (the grid is sized for a full one)
-    load_tables(tables, sx, sy, sy2);
+    load_tables(tables, tab);
     const int lane = threadIdx.x & 63;
     bool active = false, exhausted = false;
     long long cell = 0;
@@ -211,7 +217,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
                 const long long idx = base + __popcll(need & ((1ull << lane) - 1ull));
                 if (idx < count) {
                     cell = order ? order[idx] : idx;
-                    active = thermo_init(t, sx, sy, sy2, in, stride, cell, s, err);
+                    active = thermo_init(t, tab, in, stride, cell, s, err);
                     if (path) path[cell] = order ? 2 : 0;
                     if (!active) thermo_finish(s, out, stride, cell);
                 } else {
@@ -221,7 +227,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
         }
         if (!__any(active) && !__any(!exhausted)) break;
         if (active) {
-            thermo_substep(t, sx, sy, sy2, s);
+            thermo_substep(t, tab, s);
             if (s.remaining <= 0) {
                 thermo_finish(s, out, stride, cell);
                 nsub_total += (unsigned long long)s.nsub;
@@ -268,9 +274,8 @@ __device__ __forceinline__ double residual_scale(long long nsub) { return 0.01 /
 
 // Rate of one subcycle step at temperature T (Thermodynamics.cpp:314-320),
 // as dp per subcycle.
-__device__ __forceinline__ double substep_dp(const ThermoConsts& t, const double* sx, const double* sy,
-                                             const double* sy2, const CellState& s, double T) {
-    const double r = subtract_cooling(t, s.cc, sx, sy, sy2, s.heat, T);
+__device__ __forceinline__ double substep_dp(const ThermoConsts& t, const double* tab, const CellState& s, double T) {
+    const double r = subtract_cooling(t, s.cc, tab, s.heat, T);
     return t.heating_amplification * soft_landing(r, T, s.T_min) * s.rate2dpre;
 }
 
@@ -283,15 +288,14 @@ __device__ __forceinline__ double substep_dp(const ThermoConsts& t, const double
 // long subcycles (the explicit steps resolve the evolution) this is close to
 // the subcycle's own result; what remains is learned by the network.
 constexpr int COARSE_STEPS = 512;
-__device__ __forceinline__ double coarse_end_temperature(const ThermoConsts& t, const double* sx, const double* sy,
-                                                         const double* sy2, const CellState& s) {
+__device__ __forceinline__ double coarse_end_temperature(const ThermoConsts& t, const double* tab, const CellState& s) {
     double p = s.pressure;
     double kleft = (double)s.remaining;
     for (int it = 0; it < COARSE_STEPS && kleft > 0.0; ++it) {
-        const double r0 = substep_dp(t, sx, sy, sy2, s, p * s.pre2temp);
+        const double r0 = substep_dp(t, tab, s, p * s.pre2temp);
         if (r0 == 0.0) break;
         const double eps = 1.0e-4 * p;
-        const double r1 = substep_dp(t, sx, sy, sy2, s, (p + eps) * s.pre2temp);
+        const double r1 = substep_dp(t, tab, s, (p + eps) * s.pre2temp);
         const double J = (r1 - r0) / eps;
         double dk = fmin(kleft, fmax(1.0, 0.02 * p / fabs(r0)));
         if (J > 0.0) dk = fmin(dk, fmax(1.0, 1.0 / J));
@@ -396,11 +400,10 @@ __device__ __forceinline__ void apply_cell(const HydroGeom& g, double u[7], doub
 // A cell whose subcycle is longer than the exact limit: the coarse end
 // temperature, its raw features and the training-envelope test, which
 // route it to the network (to_mlp) or the FP64 fallback (to_fb).
-__device__ __forceinline__ void route_active(const ThermoConsts& t, const double* sx, const double* sy,
-                                             const double* sy2, const SurrogateConsts& sc, const double* cin,
+__device__ __forceinline__ void route_active(const ThermoConsts& t, const double* tab, const SurrogateConsts& sc, const double* cin,
                                              long long cstride, long long ccell, const CellState& s, double& Tc,
                                              double u[8], bool& to_mlp, bool& to_fb) {
-    Tc = coarse_end_temperature(t, sx, sy, sy2, s);
+    Tc = coarse_end_temperature(t, tab, s);
     raw_features(t, cin, cstride, ccell, s, Tc, u);
     // the bounds are [min, max] of the training set's features, which were
     // stored as floats: compare the float-rounded features, so that a cell
@@ -488,8 +491,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 
                                                                double* Uw, float* __restrict__ qf,
                                                                StepState* stw, long long* __restrict__ long_list,
                                                                const double* __restrict__ pre_rate) {
-    __shared__ double sx[26], sy[26], sy2[26];
-    load_tables(tables, sx, sy, sy2);
+    __shared__ double tab[TT_N];
+    load_tables(tables, tab);
     const double gdt = GRID ? grid_dt(gs) : 0.0;
     const bool halted = GRID && gs.dt < 0.0 && gs.st->halted;
     const long long nloop = ((n + blockDim.x - 1) / blockDim.x) * blockDim.x;  // uniform trip count per wave
@@ -510,9 +513,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 
             ccell = 0;
         }
         if (valid) {
-            bool active = thermo_init(t, sx, sy, sy2, cin, cstride, ccell, s, err, GRID ? pre_rate : nullptr, cell, n);
+            bool active = thermo_init(t, tab, cin, cstride, ccell, s, err, GRID ? pre_rate : nullptr, cell, n);
             if (active && s.remaining < sc.nexact) {
-                while (s.remaining > 0) thermo_substep(t, sx, sy, sy2, s);
+                while (s.remaining > 0) thermo_substep(t, tab, s);
                 active = false;
             }
             if (!active) {
@@ -526,7 +529,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 
                 if (path) path[cell] = 0;
             } else {
                 if (DEFER) defer = true;
-                else route_active(t, sx, sy, sy2, sc, cin, cstride, ccell, s, Tc, u, to_mlp, to_fb);
+                else route_active(t, tab, sc, cin, cstride, ccell, s, Tc, u, to_mlp, to_fb);
                 if (GRID) {
 #pragma unroll
                     for (int k = 0; k < 9; ++k) in[k * n + cell] = lin[k];
@@ -559,11 +562,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void su
     unsigned char* path, long long* __restrict__ mlp_list, float* __restrict__ feat, SurrCell* __restrict__ sdata,
     long long* __restrict__ fb_list, unsigned long long* __restrict__ counters,
     const long long* __restrict__ long_list, unsigned int* __restrict__ err) {
-    __shared__ double sx[26], sy[26], sy2[26];
+    __shared__ double tab[TT_N];
     const long long nfront = (long long)counters[4];
     const long long count = nfront + (long long)counters[5];
     if ((long long)blockIdx.x * blockDim.x >= count) return;  // uniform per block, before the table load's barrier
-    load_tables(tables, sx, sy, sy2);
+    load_tables(tables, tab);
     const long long nloop = ((count + blockDim.x - 1) / blockDim.x) * blockDim.x;  // uniform trip count per wave
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i - threadIdx.x < nloop;
          i += (long long)gridDim.x * blockDim.x) {
@@ -574,8 +577,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void su
         long long cell = 0;
         if (i < count) {
             cell = i < nfront ? long_list[i] : long_list[n - 1 - (i - nfront)];
-            (void)thermo_init(t, sx, sy, sy2, in, n, cell, s, err);
-            route_active(t, sx, sy, sy2, sc, in, n, cell, s, Tc, u, to_mlp, to_fb);
+            (void)thermo_init(t, tab, in, n, cell, s, err);
+            route_active(t, tab, sc, in, n, cell, s, Tc, u, to_mlp, to_fb);
         }
         queue_cell(to_mlp, to_fb, cell, u, s, Tc, sc, path, mlp_list, feat, sdata, nullptr, fb_list, counters);
     }
@@ -703,9 +706,9 @@ __global__ __launch_bounds__(256) void thermo_timestep_kernel(ThermoConsts t, co
                                                              unsigned long long* __restrict__ dtmin_bits,
                                                              unsigned int* __restrict__ err, GridSrc gs,
                                                              StepState* cfl_st, double* __restrict__ rate_out) {
-    __shared__ double sx[26], sy[26], sy2[26];
+    __shared__ double tab[TT_N];
     __shared__ double red[4], redc[4];
-    load_tables(tables, sx, sy, sy2);
+    load_tables(tables, tab);
     double m = __longlong_as_double(0x7fefffffffffffffll);
     double mc = 0.0;
     for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (long long)gridDim.x * blockDim.x) {
@@ -725,7 +728,7 @@ __global__ __launch_bounds__(256) void thermo_timestep_kernel(ThermoConsts t, co
                 if (it >= 0.0) mc = fmax(mc, it);
             }
         }
-        (void)thermo_init(t1, sx, sy, sy2, cin, cstride, ccell, s, err);
+        (void)thermo_init(t1, tab, cin, cstride, ccell, s, err);
         if (GRID && rate_out) {
             rate_out[c] = s.heat;
             rate_out[n + c] = s.rate_pre;
@@ -799,7 +802,7 @@ __global__ __launch_bounds__(256) void fill_heating_kernel(HydroGeom g, ThermoCo
                                                            long long excluded, double* __restrict__ heat,
                                                            double* __restrict__ H) {
     __shared__ double sx[26], sy[26], sy2[26];
-    load_tables(tables, sx, sy, sy2);
+    load_spline(tables, sx, sy, sy2);
     const long long n = g.ncell;
     for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (long long)gridDim.x * blockDim.x) {
         const int ijk[3] = {(int)(c % g.nx), (int)((c / g.nx) % g.ny), (int)(c / ((long long)g.nx * g.ny))};
@@ -857,16 +860,16 @@ __global__ __launch_bounds__(256) void lpt_bucket_kernel(ThermoConsts t, const d
                                                         unsigned char* __restrict__ bucket,
                                                         unsigned long long* __restrict__ hist,
                                                         unsigned int* __restrict__ err) {
-    __shared__ double sx[26], sy[26], sy2[26];
+    __shared__ double tab[TT_N];
     __shared__ unsigned int h[LPT_NB];
     if (threadIdx.x < LPT_NB) h[threadIdx.x] = 0;
-    load_tables(tables, sx, sy, sy2);
+    load_tables(tables, tab);
     if (count_dev) count = (long long)*count_dev;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count;
          i += (long long)gridDim.x * blockDim.x) {
         const long long cell = list ? list[i] : i;
         CellState s;
-        thermo_init(t, sx, sy, sy2, in, stride, cell, s, err);
+        thermo_init(t, tab, in, stride, cell, s, err);
         const int b = s.remaining > 0 ? 64 - __clzll(s.remaining) : 0;
         bucket[i] = (unsigned char)b;
         atomicAdd(&h[b], 1u);
@@ -882,12 +885,12 @@ __global__ __launch_bounds__(256) void lpt_bucket_kernel(ThermoConsts t, const d
 __global__ __launch_bounds__(256) void subcycle_count_kernel(ThermoConsts t, const double* __restrict__ tables,
                                                             long long n, const double* __restrict__ in,
                                                             long long* __restrict__ count) {
-    __shared__ double sx[26], sy[26], sy2[26];
-    load_tables(tables, sx, sy, sy2);
+    __shared__ double tab[TT_N];
+    load_tables(tables, tab);
     for (long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x; cell < n;
          cell += (long long)gridDim.x * blockDim.x) {
         CellState s;
-        thermo_init(t, sx, sy, sy2, in, n, cell, s, nullptr);
+        thermo_init(t, tab, in, n, cell, s, nullptr);
         count[cell] = s.remaining;
     }
 }
@@ -936,7 +939,7 @@ struct torchgpu_cooling {
     torchgpu_thermo_params p;
     tg::ThermoConsts t;
     hipStream_t stream = nullptr;
-    double* tables = nullptr;                 // spline x, y, y2 (78 doubles)
+    double* tables = nullptr;                 // spline x, y, y2 (78 doubles), then the rate tables (TT_N)
     unsigned long long* counters = nullptr;   // [0] work, [1] subcycles, [2] surrogate queue, [3] fallback queue,
                                               // [4], [5] cells the surrogate prepass deferred (long, short)
     unsigned int* err = nullptr;
@@ -1012,6 +1015,45 @@ namespace {
         }                                            \
     } while (0)
 
+}  // namespace
+
+namespace tg {
+
+// The tables of thermo_math.hpp (exp2, logarithm, spline pieces) from the
+// operator's spline, in extended precision.
+static void fill_rate_tables(const torchgpu_thermo_params& p, double* tab) {
+    for (int j = 0; j < 128; ++j) {
+        tab[TT_EXP + j] = (double)exp2l(j / 128.0L);
+        tab[TT_EXP_LO + j] = (double)(exp2l(j / 128.0L) - (long double)tab[TT_EXP + j]);
+        const double c = (float)(1.0L / (0.5L + (j + 0.5L) / 256.0L));
+        const long double l = -logl((long double)c);
+        const double hi = (double)(rintl(ldexpl(l, 40)) / 1099511627776.0L);
+        tab[TT_C + j] = c;
+        tab[TT_LHI + j] = hi;
+        tab[TT_LLO + j] = (double)(l - (long double)hi);
+    }
+    const double *x = p.spl_x, *y = p.spl_y, *y2 = p.spl_y2;
+    const auto piece = [tab](int k, double x0, double a, long double b, long double c, long double d) {
+        double* q = tab + TT_SPL + k;
+        q[0] = x0;
+        q[TT_NSPL] = a;
+        q[2 * TT_NSPL] = (double)b;
+        q[3 * TT_NSPL] = (double)c;
+        q[4 * TT_NSPL] = (double)d;
+    };
+    piece(0, x[0], y[0], p.spl_min_slope, 0.0L, 0.0L);
+    for (int k = 0; k < 25; ++k) {
+        const long double h = (long double)x[k + 1] - x[k];
+        piece(k + 1, x[k], y[k], ((long double)y[k + 1] - y[k]) / h - h * (2.0L * y2[k] + y2[k + 1]) / 6.0L,
+              y2[k] / 2.0L, ((long double)y2[k + 1] - y2[k]) / (6.0L * h));
+    }
+    piece(26, x[25], y[25], p.spl_max_slope, 0.0L, 0.0L);
+}
+
+}  // namespace tg
+
+namespace {
+
 tg::ThermoConsts to_consts(const torchgpu_thermo_params& p) {
     tg::ThermoConsts t{};
     t.thermo_hii_switch = p.thermo_hii_switch;
@@ -1030,6 +1072,7 @@ tg::ThermoConsts to_consts(const torchgpu_thermo_params& p) {
     t.crh = p.crh;
     t.spl_min_slope = p.spl_min_slope;
     t.spl_max_slope = p.spl_max_slope;
+    t.icxhi = 1.0 / p.cxhi_damp;
     t.subcycling = p.subcycling;
     return t;
 }
@@ -1172,8 +1215,9 @@ int torchgpu_cooling_create(const torchgpu_thermo_params* p, void* stream, torch
     c->p = *p;
     c->t = to_consts(*p);
     c->stream = (hipStream_t)stream;  // NULL: the null (default) stream
-    double tab[78];
+    double tab[78 + tg::TT_N];
     for (int i = 0; i < 26; ++i) { tab[i] = p->spl_x[i]; tab[26 + i] = p->spl_y[i]; tab[52 + i] = p->spl_y2[i]; }
+    tg::fill_rate_tables(*p, tab + 78);
     hipDeviceProp_t prop;
     int dev = 0;
     if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
