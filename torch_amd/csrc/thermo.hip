@@ -196,10 +196,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
                                                           const long long* __restrict__ order,
                                                           const double* __restrict__ in, double* __restrict__ out,
                                                           unsigned long long* __restrict__ counters,
-                                                          unsigned int* __restrict__ err, unsigned char* path) {
+                                                          unsigned int* __restrict__ err, unsigned char* path,
+                                                          int path_mark) {
     __shared__ double tab[TT_N];
     if (count_dev) count = (long long)*count_dev;
-    if (count <= 0) return;  // an empty queue (the grid is sized for a full one)
+    // a block past the queue (the grid is sized for a full one)
+    if ((long long)blockIdx.x * blockDim.x >= count) return;
     load_tables(tables, tab);
     const int lane = threadIdx.x & 63;
     bool active = false, exhausted = false;
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
                 if (idx < count) {
                     cell = order ? order[idx] : idx;
                     active = thermo_init(t, tab, in, stride, cell, s, err);
-                    if (path) path[cell] = order ? 2 : 0;
+                    if (path) path[cell] = (unsigned char)path_mark;
                     if (!active) thermo_finish(s, out, stride, cell);
                 } else {
                     exhausted = true;
@@ -243,8 +245,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
     if (lane == 0) atomicAdd(&counters[1], nsub_total);
 }
 
-__global__ void zero_u64_kernel(unsigned long long* p, int n) {
+__global__ void zero_u64_kernel(unsigned long long* p, int n, unsigned long long* q, int m) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
+    if ((int)threadIdx.x < m) q[threadIdx.x] = 0ull;
 }
 
 // ---------------------------------------------------------------------------
@@ -478,7 +481,11 @@ constexpr int COARSE_LONG = 64;
 // the routing is done here.  The GRID instance (which also forms the inputs
 // and applies the update) runs at three waves per SIMD with a few spilled
 // registers: measured faster than two without spills and four with ~50.
-template <bool GRID, bool DEFER>
+//
+// FALLBACK (a grid's FP64 step): every cell past nexact goes to the fallback
+// list.
+enum PrepassMode { PRE_ROUTE, PRE_DEFER, PRE_FALLBACK };
+template <bool GRID, PrepassMode MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 4))) void surrogate_prepass_kernel(ThermoConsts t, const double* __restrict__ tables,
                                                                SurrogateConsts sc, long long n,
                                                                double* __restrict__ in, double* __restrict__ out,
@@ -528,7 +535,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 
                 }
                 if (path) path[cell] = 0;
             } else {
-                if (DEFER) defer = true;
+                if (MODE == PRE_DEFER) defer = true;
+                else if (MODE == PRE_FALLBACK) to_fb = true;
                 else route_active(t, tab, sc, cin, cstride, ccell, s, Tc, u, to_mlp, to_fb);
                 if (GRID) {
 #pragma unroll
@@ -536,7 +544,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 
                 }
             }
         }
-        if (DEFER) {
+        if (MODE == PRE_FALLBACK) {
+            const long long fslot = wave_append(to_fb, &counters[3]);
+            if (to_fb) {
+                fb_list[fslot] = cell;
+                path[cell] = 2;
+            }
+        } else if (MODE == PRE_DEFER) {
             // cells of many remaining subcycles from the front of long_list,
             // the others from its back, so that the former share waves
             const bool lng = defer && s.remaining > COARSE_LONG;
@@ -849,33 +863,52 @@ __global__ __launch_bounds__(256) void fill_heating_kernel(HydroGeom g, ThermoCo
 // factor of two of the exact order), so the launch ends near
 // max(longest cell, total work / throughput).  Results do not depend on the
 // order: every cell is integrated independently.
+//
+// Cells of at most SHORT_STEPS subcycles, most of a batch and all of a grid's
+// at the time step the operator allows, are finished by the bucket pass and
+// get no place in the order: the persistent kernel spent a refill of its
+// wave, with its rate set-up evaluated again, on each of them (0.6 ms for 2 M
+// such cells, beside 0.1 ms to order them).
 // ---------------------------------------------------------------------------
 constexpr int LPT_NB = 64;
+constexpr unsigned char LPT_DONE = 255;
+constexpr int SHORT_STEPS = 8;
 
-__global__ __launch_bounds__(256) void lpt_bucket_kernel(ThermoConsts t, const double* __restrict__ tables,
-                                                        long long stride, long long count,
-                                                        const unsigned long long* __restrict__ count_dev,
-                                                        const long long* __restrict__ list,
-                                                        const double* __restrict__ in,
-                                                        unsigned char* __restrict__ bucket,
-                                                        unsigned long long* __restrict__ hist,
-                                                        unsigned int* __restrict__ err) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lpt_bucket_kernel(
+    ThermoConsts t, const double* __restrict__ tables, long long stride, long long count,
+    const unsigned long long* __restrict__ count_dev, const long long* __restrict__ list, const double* __restrict__ in,
+    double* __restrict__ out, unsigned char* path, unsigned char* __restrict__ bucket,
+    unsigned long long* __restrict__ hist, unsigned long long* __restrict__ counters, unsigned int* __restrict__ err) {
     __shared__ double tab[TT_N];
-    __shared__ unsigned int h[LPT_NB];
-    if (threadIdx.x < LPT_NB) h[threadIdx.x] = 0;
-    load_tables(tables, tab);
+    __shared__ unsigned int h[LPT_NB], done_steps;
     if (count_dev) count = (long long)*count_dev;
+    if ((long long)blockIdx.x * blockDim.x >= count) return;
+    if (threadIdx.x < LPT_NB) h[threadIdx.x] = 0;
+    if (threadIdx.x == LPT_NB) done_steps = 0;
+    load_tables(tables, tab);
+    unsigned int steps = 0;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count;
          i += (long long)gridDim.x * blockDim.x) {
         const long long cell = list ? list[i] : i;
         CellState s;
-        thermo_init(t, tab, in, stride, cell, s, err);
-        const int b = s.remaining > 0 ? 64 - __clzll(s.remaining) : 0;
-        bucket[i] = (unsigned char)b;
-        atomicAdd(&h[b], 1u);
+        const bool active = thermo_init(t, tab, in, stride, cell, s, err);
+        if (active && s.remaining > SHORT_STEPS) {
+            const int b = 64 - __clzll(s.remaining);
+            bucket[i] = (unsigned char)b;
+            atomicAdd(&h[b], 1u);
+        } else {
+            while (s.remaining > 0) thermo_substep(t, tab, s);
+            thermo_finish(s, out, stride, cell);
+            steps += (unsigned int)s.nsub;
+            bucket[i] = LPT_DONE;
+            if (path) path[cell] = list ? 2 : 0;
+        }
     }
+    for (int off = 32; off > 0; off >>= 1) steps += __shfl_xor(steps, off, 64);
+    if ((threadIdx.x & 63) == 0 && steps) atomicAdd(&done_steps, steps);
     __syncthreads();
     if (threadIdx.x < LPT_NB && h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], (unsigned long long)h[threadIdx.x]);
+    if (threadIdx.x == LPT_NB && done_steps) atomicAdd(&counters[1], (unsigned long long)done_steps);
 }
 
 // Subcycle count of each cell (the explicit steps integrate() takes after
@@ -895,14 +928,16 @@ __global__ __launch_bounds__(256) void subcycle_count_kernel(ThermoConsts t, con
     }
 }
 
-// cursor[b] = number of items in buckets above b (longest first)
-__global__ void lpt_offsets_kernel(const unsigned long long* __restrict__ hist, unsigned long long* __restrict__ cursor) {
+// cursor[b] = number of items in buckets above b (longest first); hist[0]
+// (no item has bucket 0) becomes their number.
+__global__ void lpt_offsets_kernel(unsigned long long* __restrict__ hist, unsigned long long* __restrict__ cursor) {
     if (threadIdx.x != 0) return;
     unsigned long long off = 0;
-    for (int b = LPT_NB - 1; b >= 0; --b) {
+    for (int b = LPT_NB - 1; b > 0; --b) {
         cursor[b] = off;
         off += hist[b];
     }
+    hist[0] = off;
 }
 
 __global__ __launch_bounds__(256) void lpt_scatter_kernel(long long count, const unsigned long long* __restrict__ count_dev,
@@ -916,19 +951,16 @@ __global__ __launch_bounds__(256) void lpt_scatter_kernel(long long count, const
     const int tid = threadIdx.x;
     // the trip count is uniform over the block (barriers inside)
     for (long long i0 = (long long)blockIdx.x * blockDim.x; i0 < count; i0 += (long long)gridDim.x * blockDim.x) {
-        if (tid < LPT_NB) h[tid] = 0;
-        __syncthreads();
         const long long i = i0 + tid;
-        int b = -1;
+        const int b = i < count ? bucket[i] : LPT_DONE;
+        if (tid < LPT_NB) h[tid] = 0;
+        if (!__syncthreads_or(b != LPT_DONE)) continue;
         unsigned int rank = 0;
-        if (i < count) {
-            b = bucket[i];
-            rank = atomicAdd(&h[b], 1u);
-        }
+        if (b != LPT_DONE) rank = atomicAdd(&h[b], 1u);
         __syncthreads();
         if (tid < LPT_NB && h[tid]) base[tid] = atomicAdd(&cursor[tid], (unsigned long long)h[tid]);
         __syncthreads();
-        if (b >= 0) order[base[b] + rank] = list ? list[i] : i;
+        if (b != LPT_DONE) order[base[b] + rank] = list ? list[i] : i;
         __syncthreads();
     }
 }
@@ -952,6 +984,7 @@ struct torchgpu_cooling {
     long long cap = 0;                        // capacity of the queues below
     long long* mlp_list = nullptr;
     long long* fb_list = nullptr;
+    long long fb_cap = 0;                     // capacity of fb_list
     long long* long_list = nullptr;           // the surrogate prepass's deferred cells
     float* feat = nullptr;
     float* y = nullptr;
@@ -1078,49 +1111,48 @@ tg::ThermoConsts to_consts(const torchgpu_thermo_params& p) {
 }
 
 int zero_counters(torchgpu_cooling* c) {
-    hipLaunchKernelGGL(tg::zero_u64_kernel, dim3(1), dim3(64), 0, c->stream, c->counters, 6);
+    hipLaunchKernelGGL(tg::zero_u64_kernel, dim3(1), dim3(64), 0, c->stream, c->counters, 6,
+                       (unsigned long long*)nullptr, 0);
     HIP_OK(hipGetLastError());
     return TORCHGPU_OK;
 }
 
-int launch_fp64(torchgpu_cooling* c, long long stride, long long count, const unsigned long long* count_dev,
-                const long long* order, const double* in, double* out, unsigned char* path) {
-    long long blocks = (long long)c->nsm * 8;  // 32 waves per CU
-    if (!count_dev && blocks * 256 > count) blocks = (count + 255) / 256;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(tg::thermo_cells_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, c->t, c->tables,
-                       stride, count, count_dev, order, in, out, c->counters, c->err, path);
-    HIP_OK(hipGetLastError());
-    return TORCHGPU_OK;
-}
-
-// Work order (longest cells first) of `count` items (count_dev: on the
-// device) that are cells list[i] (list == NULL: i), into `order` [count],
-// with the per-item buckets in `bucket` [count] and the histogram and
-// cursors in `hist` [2 LPT_NB] (cleared here by a kernel).
-int lpt_order_into(torchgpu_cooling* c, long long stride, long long count, const unsigned long long* count_dev,
-                   const long long* list, const double* in, long long* order, unsigned char* bucket,
-                   unsigned long long* hist) {
-    hipLaunchKernelGGL(tg::zero_u64_kernel, dim3(1), dim3(2 * tg::LPT_NB), 0, c->stream, hist, 2 * tg::LPT_NB);
+// The FP64 integrator on `count` items (count_dev: on the device, at most
+// count) that are cells list[i] (list == NULL: i): the short ones in the
+// bucket pass, the rest by the persistent kernel, longest first.  order
+// [count], bucket [count] and hist [2 LPT_NB] (cleared here by a kernel) are
+// the work order's scratch; counters [1] gets the subcycles.
+int integrate(torchgpu_cooling* c, long long stride, long long count, const unsigned long long* count_dev,
+              const long long* list, const double* in, double* out, unsigned char* path, long long* order,
+              unsigned char* bucket, unsigned long long* hist) {
+    hipLaunchKernelGGL(tg::zero_u64_kernel, dim3(1), dim3(2 * tg::LPT_NB), 0, c->stream, hist, 2 * tg::LPT_NB,
+                       c->counters, 2);
     HIP_OK(hipGetLastError());
     long long blocks = (count + 255) / 256;
-    if (blocks > (long long)c->nsm * 16) blocks = (long long)c->nsm * 16;
+    const long long most = (long long)c->nsm * 16;
+    if (blocks > most) blocks = most;
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(tg::lpt_bucket_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, c->t, c->tables,
-                       stride, count, count_dev, list, in, bucket, hist, c->err);
+                       stride, count, count_dev, list, in, out, path, bucket, hist, c->counters, c->err);
     HIP_OK(hipGetLastError());
     hipLaunchKernelGGL(tg::lpt_offsets_kernel, dim3(1), dim3(64), 0, c->stream, hist, hist + tg::LPT_NB);
     HIP_OK(hipGetLastError());
     hipLaunchKernelGGL(tg::lpt_scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, count, count_dev,
                        list, bucket, hist + tg::LPT_NB, order);
     HIP_OK(hipGetLastError());
+    blocks = (count + 255) / 256;
+    if (blocks > (long long)c->nsm * 8) blocks = (long long)c->nsm * 8;  // 32 waves per CU
+    if (blocks < 1) blocks = 1;
+    hipLaunchKernelGGL(tg::thermo_cells_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, c->t, c->tables,
+                       stride, count, (const unsigned long long*)hist, order, in, out, c->counters, c->err, path,
+                       list ? 2 : 0);
+    HIP_OK(hipGetLastError());
     return TORCHGPU_OK;
 }
 
-// lpt_order_into on the handle's own buffers (grown as needed); returns
-// c->lpt_order.
-int lpt_order(torchgpu_cooling* c, long long stride, long long count, const unsigned long long* count_dev,
-              const long long* list, const double* in, const long long** order) {
+// integrate() on the handle's own scratch (grown as needed).
+int integrate_own(torchgpu_cooling* c, long long stride, long long count, const unsigned long long* count_dev,
+                  const long long* list, const double* in, double* out, unsigned char* path) {
     if (count > c->lpt_cap) {
         (void)hipStreamSynchronize(c->stream);
         if (c->lpt_order) (void)hipFree(c->lpt_order);
@@ -1133,12 +1165,8 @@ int lpt_order(torchgpu_cooling* c, long long stride, long long count, const unsi
         c->lpt_cap = count;
     }
     if (!c->lpt_hist) HIP_OK(hipMalloc(&c->lpt_hist, 2 * tg::LPT_NB * sizeof(unsigned long long)));
-    int rc = lpt_order_into(c, stride, count, count_dev, list, in, c->lpt_order, c->lpt_bucket, c->lpt_hist);
-    if (rc) return rc;
-    *order = c->lpt_order;
-    return TORCHGPU_OK;
+    return integrate(c, stride, count, count_dev, list, in, out, path, c->lpt_order, c->lpt_bucket, c->lpt_hist);
 }
-
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
 std::mutex noalloc_mu;
@@ -1164,21 +1192,32 @@ int noalloc_setup(torchgpu_cooling* c, int dev) {
     return TORCHGPU_OK;
 }
 
+int ensure_fallback(torchgpu_cooling* c, long long n) {
+    if (n <= c->fb_cap) return TORCHGPU_OK;
+    (void)hipStreamSynchronize(c->stream);
+    if (c->fb_list) (void)hipFree(c->fb_list);
+    c->fb_list = nullptr;
+    c->fb_cap = 0;
+    HIP_OK(hipMalloc(&c->fb_list, n * sizeof(long long)));
+    c->fb_cap = n;
+    return TORCHGPU_OK;
+}
+
 int ensure_queues(torchgpu_cooling* c, long long n) {
     if (n <= c->cap) return TORCHGPU_OK;
+    int rc;
     (void)hipStreamSynchronize(c->stream);
     if (c->mlp_list) (void)hipFree(c->mlp_list);
-    if (c->fb_list) (void)hipFree(c->fb_list);
     if (c->long_list) (void)hipFree(c->long_list);
     if (c->feat) (void)hipFree(c->feat);
     if (c->y) (void)hipFree(c->y);
     if (c->sdata) (void)hipFree(c->sdata);
-    c->mlp_list = c->fb_list = c->long_list = nullptr;
+    c->mlp_list = c->long_list = nullptr;
     c->feat = c->y = nullptr;
     c->sdata = nullptr;
     c->cap = 0;
     HIP_OK(hipMalloc(&c->mlp_list, n * sizeof(long long)));
-    HIP_OK(hipMalloc(&c->fb_list, n * sizeof(long long)));
+    if ((rc = ensure_fallback(c, n))) return rc;
     HIP_OK(hipMalloc(&c->long_list, n * sizeof(long long)));
     HIP_OK(hipMalloc(&c->feat, n * 8 * sizeof(float)));
     HIP_OK(hipMalloc(&c->y, n * 3 * sizeof(float)));
@@ -1264,11 +1303,7 @@ int torchgpu_thermo_cells(torchgpu_cooling* c, int64_t n, const double* in, doub
         if (total_substeps) *total_substeps = 0;
         return TORCHGPU_OK;
     }
-    int rc = zero_counters(c);
-    if (rc) return rc;
-    const long long* order = nullptr;
-    if ((rc = lpt_order(c, n, n, nullptr, nullptr, in, &order))) return rc;
-    rc = launch_fp64(c, n, n, nullptr, order, in, out, nullptr);
+    int rc = integrate_own(c, n, n, nullptr, nullptr, in, out, nullptr);
     if (rc) return rc;
     if (total_substeps) {
         unsigned long long tot = 0;
@@ -1305,9 +1340,7 @@ int torchgpu_thermo_cells_noalloc(torchgpu_cooling* c, int64_t n, const double* 
     unsigned long long* hist = reinterpret_cast<unsigned long long*>(base);
     long long* order = reinterpret_cast<long long*>(base + NOALLOC_HIST_BYTES);
     unsigned char* bucket = base + NOALLOC_HIST_BYTES + NOALLOC_ORDER_BYTES;
-    if ((rc = zero_counters(c))) return rc;
-    if ((rc = lpt_order_into(c, n, n, nullptr, nullptr, in, order, bucket, hist))) return rc;
-    if ((rc = launch_fp64(c, n, n, nullptr, order, in, out, nullptr))) return rc;
+    if ((rc = integrate(c, n, n, nullptr, nullptr, in, out, nullptr, order, bucket, hist))) return rc;
     if (total_substeps) {
         unsigned long long tot = 0;
         HIP_OK(hipMemcpyAsync(&tot, c->counters + 1, sizeof tot, hipMemcpyDeviceToHost, c->stream));
@@ -1353,6 +1386,25 @@ struct ApplyDst {
     const double* pre_rate;  // heating rate and pre-step RATE of each cell on this state, or NULL
 };
 
+// The FP64 step on the grid state: as the surrogate's, with every cell past
+// SHORT_STEPS subcycles integrated by the persistent kernel.
+static int fp64_grid_step(torchgpu_cooling* c, int64_t n, double* in, double* out, uint8_t* path, const tg::GridSrc& gs,
+                          const ApplyDst& apply) {
+    if (n == 0) return TORCHGPU_OK;
+    int rc = ensure_fallback(c, n);
+    if (rc || (rc = zero_counters(c))) return rc;
+    tg::SurrogateConsts sc{};
+    sc.nexact = tg::SHORT_STEPS;
+    long long nb = (n + 255) / 256;
+    if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
+    hipLaunchKernelGGL((tg::surrogate_prepass_kernel<true, tg::PRE_FALLBACK>), dim3((unsigned)nb), dim3(256), 0,
+                       c->stream, c->t, c->tables, sc, (long long)n, in, out, path, (long long*)nullptr,
+                       (float*)nullptr, (tg::SurrCell*)nullptr, (float*)nullptr, c->fb_list, c->counters, c->err, gs,
+                       apply.U, apply.qf, apply.st, (long long*)nullptr, apply.pre_rate);
+    HIP_OK(hipGetLastError());
+    return integrate_own(c, n, n, c->counters + 3, c->fb_list, in, out, path);
+}
+
 // The surrogate step on `in` (gs and apply NULL), or on the grid state (gs
 // and apply both given: the inputs are formed in the prepass, `in` receives
 // those of the queued cells, and the prepass applies the update of the cells
@@ -1373,12 +1425,12 @@ static int surrogate_step(torchgpu_cooling* c, int64_t n, double* in, double* ou
     long long nb = (n + 255) / 256;
     if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
     if (gs)
-        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<true, true>), dim3((unsigned)nb), dim3(256), 0, c->stream, c->t,
+        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<true, tg::PRE_DEFER>), dim3((unsigned)nb), dim3(256), 0, c->stream, c->t,
                            c->tables, sc, (long long)n, in, out, path, c->mlp_list, c->feat, c->sdata, (float*)nullptr,
                            c->fb_list, c->counters, c->err, *gs, apply->U, apply->qf, apply->st, c->long_list,
                            apply->pre_rate);
     else
-        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, true>), dim3((unsigned)nb), dim3(256), 0, c->stream,
+        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, tg::PRE_DEFER>), dim3((unsigned)nb), dim3(256), 0, c->stream,
                            c->t, c->tables, sc, (long long)n, in, out, path, c->mlp_list, c->feat, c->sdata,
                            (float*)nullptr, c->fb_list, c->counters, c->err, tg::GridSrc{}, (double*)nullptr,
                            (float*)nullptr, (tg::StepState*)nullptr, c->long_list, (const double*)nullptr);
@@ -1394,12 +1446,8 @@ static int surrogate_step(torchgpu_cooling* c, int64_t n, double* in, double* ou
     hipLaunchKernelGGL(tg::surrogate_finish_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, c->t, sc,
                        (long long)n, c->counters, c->mlp_list, c->sdata, c->y, out, path, c->fb_list, c->counters);
     HIP_OK(hipGetLastError());
-    // fallback queue through the FP64 integrator (work counter reset first)
-    hipLaunchKernelGGL(tg::zero_u64_kernel, dim3(1), dim3(64), 0, c->stream, c->counters, 1);
-    HIP_OK(hipGetLastError());
-    const long long* order = nullptr;
-    if ((rc = lpt_order(c, n, n, c->counters + 3, c->fb_list, in, &order))) return rc;
-    if ((rc = launch_fp64(c, n, n, c->counters + 3, order, in, out, path))) return rc;
+    // fallback queue through the FP64 integrator
+    if ((rc = integrate_own(c, n, n, c->counters + 3, c->fb_list, in, out, path))) return rc;
     if (counts) {
         unsigned long long h[4];
         HIP_OK(hipMemcpyAsync(h, c->counters, sizeof h, hipMemcpyDeviceToHost, c->stream));
@@ -1440,7 +1488,7 @@ int torchgpu_surrogate_training_data(torchgpu_cooling* c, int64_t n, const doubl
     };
     long long nb = (n + 255) / 256;
     if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
-    hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, false>), dim3((unsigned)nb), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, tg::PRE_ROUTE>), dim3((unsigned)nb), dim3(256), 0, c->stream,
                        c->t, c->tables, sc, (long long)n, const_cast<double*>(in), scratch, (unsigned char*)nullptr,
                        (long long*)list, feat, c->sdata, raw, c->fb_list, c->counters, c->err, tg::GridSrc{},
                        (double*)nullptr, (float*)nullptr, (tg::StepState*)nullptr, (long long*)nullptr,
@@ -1567,20 +1615,20 @@ static int grid_substep_dev(torchgpu_ctx* ctx, torchgpu_cooling* c, const double
                             const double* F, int64_t excluded, double dt, int surrogate, bool kept_rate = false) {
     tg::CtxView v = tg::ctx_view(ctx);
     const long long n = v.g->ncell;
-    // the surrogate step forms the inputs in its prepass unless the heating
-    // record needs the gathered array
-    const bool direct = surrogate && !(v.heat && c->t.subcycling);
+    // the inputs are formed in the prepass, which also applies the update
+    // (Thermodynamics::updateSourceTerms + advSolution(dt) + fixSolution) to
+    // the cells it finishes (the queued cells get it once the network and the
+    // integrator have run), unless the heating record needs the gathered array
+    const bool direct = !(v.heat && c->t.subcycling);
     int rc;
     if (direct) {
-        // the inputs formed in the prepass, which also applies the update
-        // (Thermodynamics::updateSourceTerms + advSolution(dt) +
-        // fixSolution) to the cells it finishes; the queued cells get it
-        // once the network and the fallback have run
         tg::GridSrc gs;
         if ((rc = grid_src(c, ctx, T_min, col_den, F, excluded, dt, gs))) return rc;
         float* qf = tg::ctx_qf_for_state(ctx);
         const ApplyDst ad{v.U, qf, v.st, kept_rate ? c->rcache : nullptr};
-        if ((rc = surrogate_step(c, n, c->in9, c->out5, c->gpath, nullptr, &gs, &ad))) return rc;
+        if (surrogate) rc = surrogate_step(c, n, c->in9, c->out5, c->gpath, nullptr, &gs, &ad);
+        else rc = fp64_grid_step(c, n, c->in9, c->out5, c->gpath, gs, ad);
+        if (rc) return rc;
         long long nb = (n + 255) / 256;
         if (nb > 65536) nb = 65536;
         hipLaunchKernelGGL(tg::queue_apply_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, gs, c->out5, c->gpath,
@@ -1855,8 +1903,9 @@ int torchgpu_run_full(torchgpu_ctx* ctx, torchgpu_cooling* c, torchgpu_radiation
         // a step that opens with the cooling sub-step (every other one: the
         // order turns each step) reuses the pre-step rates of the time step,
         // which sees the same state (not with radiation, whose pre-step
-        // comes in between)
-        const bool share = c && !r && surrogate && order_first(comps, ncomps, (launched + 1) % ncomps) == THERMO;
+        // comes in between, nor where the heating record has the inputs
+        // gathered)
+        const bool share = c && !r && !(v.heat && c->t.subcycling) && order_first(comps, ncomps, (launched + 1) % ncomps) == THERMO;
         if (c && (rc = grid_timestep_dev(ctx, c, T_min, col_den, F, excluded, v.st, share))) return rc;
         if (r && ((rc = tg::rad_pre_step_dev(r, 1)) || (rc = tg::rad_timestep_dev(r, 0.0, 1)))) return rc;
         HIP_OK(tg::launch_step_begin(v.st, 1, 0.0, v.stream, c ? c->dtbits : nullptr,
