@@ -77,6 +77,36 @@ def test_solver_limiter_variants_ragged_grid(gpu, orc, solver, limiter, order):
     np.testing.assert_array_equal(Ug, Uo)
 
 
+# sizes on both sides of the two FP64 layouts' rule (8 x 4 x 4 tiles below about
+# half a million cells, 16 x 16 columns marched along z above), none a
+# multiple of a tile, a column or a column's planes
+@pytest.mark.parametrize("nz,ny,nx", [(3, 5, 7), (21, 33, 18), (85, 91, 101), (4, 301, 323), (131, 70, 75)])
+@pytest.mark.parametrize("solver,limiter,order,bcs", [
+    ("RotatedHLLC", "albada", 1, ["periodic", "periodic", "reflecting", "outflow", "inflow", "reflecting"]),
+    ("RotatedHLLC", "minmod", 1, ["reflecting", "inflow", "periodic", "periodic", "periodic", "periodic"]),
+    ("HLLC", "albada", 0, ["free", "reflecting", "inflow", "free", "reflecting", "outflow"]),
+    ("HLL", "leer", 1, ["outflow", "free", "outflow", "periodic", "free", "inflow"])])
+def test_layouts_bitwise(gpu, orc, nz, ny, nx, solver, limiter, order, bcs):
+    if min(nz, ny, nx) < 4 and "reflecting" in bcs:
+        bcs = ["outflow" if b == "reflecting" else b for b in bcs]  # cells 1 and 2 of such an axis are read
+    rng = np.random.Generator(np.random.PCG64(nx))
+    z, y, x = np.meshgrid(*[np.arange(n) / n for n in (nz, ny, nx)], indexing="ij")
+    Q = np.empty((7, nz, ny, nx))
+    for v in range(7):
+        k = rng.integers(1, 4, 3)
+        Q[v] = np.sin(2 * np.pi * (k[0] * x + k[1] * y + k[2] * z) + v) + 0.1 * rng.standard_normal((nz, ny, nx))
+    Q[:2] = np.exp(0.5 * Q[:2])
+    Q[2:4] = 0.5 + 0.3 * Q[2:4]
+    Q[4:, : nz // 2, : ny // 3] = 0.25  # a region of uniform flow: the solver's pure paths
+    Q[5:, :, :, : nx // 4] = 0.0
+    kw = dict(tfloor=1e-12, pfloor=0.1 * 8.314462e7 * 1e-30 * 1e-12, solver=solver, limiter=limiter,
+              spatial_order=order, bc=bcs)
+    Ug, Uo, cg, co = _run_both(gpu, orc, Q, 3, gkw=dict(kw), okw=dict(kw))
+    assert Ug is not None
+    np.testing.assert_array_equal(Ug, Uo)
+    assert cg == co
+
+
 def test_explicit_step_and_timestep(gpu, orc):
     Q = setups.turbulent(16, 1.0, 2.0)
     kw = dict(tfloor=1e-12, pfloor=0.1 * 8.314462e7 * 1e-30 * 1e-12)

@@ -220,8 +220,6 @@ int torchgpu_create(const torchgpu_params* p, void* stream, torchgpu_ctx** out) 
     tg::HydroGeom& g = c->g;
     std::memset(&g, 0, sizeof g);
     g.nx = p->nx; g.ny = p->ny; g.nz = p->nz;
-    g.ntx = (p->nx + 7) / 8; g.nty = (p->ny + 7) / 8; g.ntz = (p->nz + 7) / 8;
-    g.ntiles = g.ntx * g.nty * g.ntz;
     for (int d = 0; d < 3; ++d) { g.bc_l[d] = p->bc_left[d]; g.bc_r[d] = p->bc_right[d]; }
     g.limiter = p->slope_limiter;
     g.spatial_order = p->spatial_order;

@@ -15,207 +15,504 @@
 //
 // Data layout: conserved state U is structure-of-arrays in HBM,
 // U[v * ncell + x + nx * (y + ny * z)], v in UID order, x fastest.
-// A workgroup owns an 8x8x8 tile of cells (576 threads = 9 waves).  Q of the
-// tile lives in LDS; for each sweep direction the 2-deep halo slabs on both
-// sides are staged in LDS, every one of the 9x8x8 faces of that direction is
-// solved once by one thread, the fluxes go to LDS, and each cell thread
-// accumulates its two faces in the reference's order.  Tiles are assigned
-// XCD-contiguously (consecutive workgroups round-robin over the 8 XCDs, so
-// workgroup b is given tile (b % 8) * (ntiles / 8) + b / 8) so that each
-// XCD's L2 sees neighbouring tiles' halos.
 //
-// This is the FP64 parity kernel: compiled with -ffp-contract=off it keeps
-// the reference's operand order and is bitwise equal to its x86-64 build.
-// The sweep fluxes of all three directions stay in LDS (140 KB) and are
-// accumulated once per cell after the sweeps, so the accumulators are not
-// live across the face solves.  The mixed-precision kernel is in
-// hydro_mixed.hip.
+// These are the FP64 parity kernels: compiled with -ffp-contract=off they
+// keep the reference's operand order and are bitwise equal to its x86-64
+// build.  Two layouts of one stage, chosen by the grid's size
+// (launch_hydro_stage):
+//
+//  hydro_march_kernel  a workgroup of 256 threads owns a 16 x 16 column of
+//      cells and marches it along z.  Each thread keeps the primitives of its
+//      column at planes k .. k+2, the limited z slope of plane k and the last
+//      z flux in registers; plane k with its 2-deep x and y halos, and each
+//      cell's x and y slope (limited once for both its faces), go through
+//      LDS.  Per cell 3.125 face solves (and 1/planes), 21 limited slopes and
+//      1.5 cell loads, where the 8^3 tiles this replaces took 3.375, 47 and
+//      2.5; 72 KB of LDS and 256 registers leave two workgroups per CU (eight
+//      waves on four SIMDs), where those tiles' 140 KB left one of nine waves.
+//  hydro_tile_kernel   an 8 x 4 x 4 tile per workgroup of 512 threads, all
+//      faces of the three directions solved at once, one per thread: a grid
+//      too small to fill the chip is bound by the length of one workgroup's
+//      serial chain, here one load, one solve and one update, where the
+//      tiles took three sweeps and a march takes a solve per plane.
+//
+// Workgroups are handed out XCD-contiguously (consecutive workgroups
+// round-robin over the 8 XCDs, so workgroup b is given tile (b % 8) *
+// (ntiles / 8) + b / 8) so that each XCD's L2 sees neighbouring halos.  The
+// mixed-precision kernel is in hydro_mixed.hip.
 
 #include "hydro_device.hpp"
 
 namespace tg {
 
-struct TileLDS {
-    double qc[7][TCELLS];
-    double qh[7][THALO];
-    double fl[3][7][TFACES];  // face fluxes of the three sweeps
-    double red[NTHREADS / 64];
+// Limited slope of cell b between its neighbours a and c (0 at first order).
+// ALB: van Albada, the default, without the other limiters' code.
+template <bool ALB>
+__device__ __forceinline__ void cell_slope(const HydroGeom& g, const double a[7], const double b[7], const double c[7],
+                                           double s[7]) {
+    if (g.spatial_order == 1) {
+#pragma unroll
+        for (int v = 0; v < 7; ++v) s[v] = limiter<double>(ALB ? (int)LIM_ALBADA : g.limiter, b[v] - a[v], c[v] - b[v]);
+    } else {
+#pragma unroll
+        for (int v = 0; v < 7; ++v) s[v] = 0.0;
+    }
+}
+
+// Flux along DIM through the face between cells b and c with limited slopes
+// sb and sc: QR of b and QL of c (Hydrodynamics::reconstruct) and the Riemann
+// solve.  yswap (DIM 0): a y face, solved as an x face with the x and y
+// velocity components exchanged (see hydro_math.hpp).  Returns true if the
+// HII flux is NaN.
+template <int SOLVER, int DIM>
+__device__ __forceinline__ bool slope_flux(const HydroGeom& g, const double b[7], const double sb[7], const double c[7],
+                                           const double sc[7], const GasConsts<double>& gc, double F[7],
+                                           bool yswap = false) {
+    double ql[7], qr[7];
+#pragma unroll
+    for (int v = 0; v < 7; ++v) {
+        ql[v] = b[v] + 0.5 * sb[v];
+        qr[v] = c[v] - 0.5 * sc[v];
+    }
+    if (DIM == 0 && yswap) {
+        const double lx = ql[VEL], rx = qr[VEL];
+        ql[VEL] = ql[VEL + 1];
+        qr[VEL] = qr[VEL + 1];
+        ql[VEL + 1] = lx;
+        qr[VEL + 1] = rx;
+    }
+    const double a_l2 = gc.g * ql[PRE] / ql[DEN];
+    const double a_r2 = gc.g * qr[PRE] / qr[DEN];
+    const bool bad = riemann<SOLVER, double, DIM>(F, ql, qr, a_l2, a_r2, gc, yswap);
+    if (DIM == 0 && yswap) {
+        const double fx = F[VEL];
+        F[VEL] = F[VEL + 1];
+        F[VEL + 1] = fx;
+    }
+    return bad;
+}
+
+// Fluid::advSolution + fixSolution of one cell from its base state u and
+// flux divergence (the gravity source is zero, GRAV = 0), in place; stage 2
+// returns the CFL term of the new state.
+template <int STAGE>
+__device__ __forceinline__ double update_cell(const HydroGeom& g, double u[7], const double udot[7], double dtf,
+                                              StepState* st) {
+#pragma unroll
+    for (int v = 0; v < 7; ++v) u[v] += dtf * udot[v];
+    if (fix_solution(g, u)) set_error(st, STAGE == 1 ? ERR_FIX_SOLUTION_1 : ERR_FIX_SOLUTION_2);
+    if (STAGE == 1) return 0.0;
+    double q[7];
+    QfromU(q, u, g.gm1);
+    fix_primitives(g, q, u[DEN]);
+    return cfl_inv_t(g, q);
+}
+
+// ---------------------------------------------------------------------------
+// Small grids: 8 x 4 x 4 tiles, every face of the tile at once
+// ---------------------------------------------------------------------------
+constexpr int QX = 8, QY = 4, QZ = 4, QCELLS = QX * QY * QZ;
+constexpr int QHX = 4 * QY * QZ, QHY = 4 * QX * QZ, QHZ = 4 * QX * QY;  // 2-deep halos at both ends
+constexpr int QNX = (QX + 1) * QY * QZ, QNY = QX * (QY + 1) * QZ, QNZ = QX * QY * (QZ + 1);
+constexpr int QTHREADS = 512;
+constexpr int QZ0 = 320;  // first thread of the z faces: whole waves per solver
+static_assert(QNX + QNY <= QZ0 && QZ0 % 64 == 0 && QZ0 + QNZ <= QTHREADS, "one face per thread");
+static_assert(QCELLS + QHX + QHY + QHZ <= QTHREADS, "one cell per thread");
+
+struct SmallLDS {
+    double q[7][QCELLS + QHX + QHY + QHZ];
+    double fx[7][QNX], fy[7][QNY], fz[7][QNZ];
+    double red[QTHREADS / 64];
 };
 
-// LDS address of the Q value at along-position pos (-2..9) of sweep DIM with
-// transverse coordinates (ta, tb).
-template <int DIM>
-__device__ __forceinline__ int center_index(int pos, int ta, int tb) {
-    if (DIM == 0) return pos + TILE * (ta + TILE * tb);
-    if (DIM == 1) return ta + TILE * (pos + TILE * tb);
-    return ta + TILE * (tb + TILE * pos);
+// LDS slot of tile position (x, y, z), of which one may lie in a 2-deep halo.
+__device__ __forceinline__ int qslot(int x, int y, int z) {
+    if ((unsigned)x >= (unsigned)QX) return QCELLS + (x < 0 ? x + 2 : x - QX + 2) * (QY * QZ) + y + QY * z;
+    if ((unsigned)y >= (unsigned)QY) return QCELLS + QHX + (y < 0 ? y + 2 : y - QY + 2) * (QX * QZ) + x + QX * z;
+    if ((unsigned)z >= (unsigned)QZ)
+        return QCELLS + QHX + QHY + (z < 0 ? z + 2 : z - QZ + 2) * (QX * QY) + x + QX * y;
+    return x + QX * (y + QY * z);
 }
 
-template <int DIM>
-__device__ __forceinline__ void q_at(const TileLDS& s, int pos, int ta, int tb, double q[7]) {
-    if (pos >= 0 && pos < TILE) {
-        const int i = center_index<DIM>(pos, ta, tb);
+// Face f of tile row (ox, oy, oz) + f along DIM: the four stencil cells, both
+// slopes and the solve.
+template <int SOLVER, bool ALB, int DIM>
+__device__ __forceinline__ bool small_face(const HydroGeom& g, const SmallLDS& s, int x, int y, int z, bool yface,
+                                           const GasConsts<double>& gc, double F[7]) {
+    const int dx = DIM == 0 && !yface, dy = DIM == 0 && yface, dz = DIM == 2;
+    double q[4][7], sb[7], sc[7];
 #pragma unroll
-        for (int v = 0; v < 7; ++v) q[v] = s.qc[v][i];
-    } else {
-        const int h = pos < 0 ? pos + 2 : pos - TILE + 2;
-        const int i = h * (TILE * TILE) + tb * TILE + ta;
+    for (int i = 0; i < 4; ++i) {
+        const int c = qslot(x + dx * (i - 2), y + dy * (i - 2), z + dz * (i - 2));
 #pragma unroll
-        for (int v = 0; v < 7; ++v) q[v] = s.qh[v][i];
+        for (int v = 0; v < 7; ++v) q[i][v] = s.q[v][c];
     }
+    cell_slope<ALB>(g, q[0], q[1], q[2], sb);
+    cell_slope<ALB>(g, q[1], q[2], q[3], sc);
+    return slope_flux<SOLVER, DIM>(g, q[1], sb, q[2], sc, gc, F, yface);
 }
 
-// Flux through face f (between along-positions f-1 and f) of pencil (ta, tb)
-// of sweep DIM: reconstruction from the tile's LDS Q and the Riemann solve.
-// Returns true if the HII flux is NaN.
-template <int SOLVER, int DIM>
-__device__ __forceinline__ bool face_flux(const HydroGeom& g, const TileLDS& s, int f, int ta, int tb,
-                                          const GasConsts<double>& gc, double F[7]) {
-    double ql[7], qr[7];
-    if (g.spatial_order == 1) {
-        double a[7], b[7], cc[7], dd[7];
-        q_at<DIM>(s, f - 2, ta, tb, a);
-        q_at<DIM>(s, f - 1, ta, tb, b);
-        q_at<DIM>(s, f, ta, tb, cc);
-        q_at<DIM>(s, f + 1, ta, tb, dd);
-#pragma unroll
-        for (int v = 0; v < 7; ++v) {
-            double dl = limiter<double>(g.limiter, b[v] - a[v], cc[v] - b[v]);
-            ql[v] = b[v] + 0.5 * dl;   // QR of cell f-1
-            double dr = limiter<double>(g.limiter, cc[v] - b[v], dd[v] - cc[v]);
-            qr[v] = cc[v] - 0.5 * dr;  // QL of cell f
-        }
-    } else {
-        q_at<DIM>(s, f - 1, ta, tb, ql);
-        q_at<DIM>(s, f, ta, tb, qr);
-    }
-    double a_l2 = gc.g * ql[PRE] / ql[DEN];
-    double a_r2 = gc.g * qr[PRE] / qr[DEN];
-    return riemann<SOLVER, double, DIM>(F, ql, qr, a_l2, a_r2, gc);
-}
-
-template <int SOLVER, int STAGE, int DIM>
-__device__ __forceinline__ void sweep(const HydroGeom& g, TileLDS& s, const double* __restrict__ Usrc,
-                                      const int o[3], StepState* st, const GasConsts<double>& gc) {
-    const int tid = threadIdx.x;
-    const int N[3] = {g.nx, g.ny, g.nz};
-    constexpr int DA = DIM == 0 ? 1 : 0;       // transverse dim "a"
-    constexpr int DB = DIM == 2 ? 1 : 2;       // transverse dim "b"
-
-    // 1. halo slabs of this direction (the previous sweep's face phase, the
-    //    last reader of qh, ended at a barrier)
-    if (tid < THALO) {
-        const int h = tid >> 6, ta = tid & 7, tb = (tid >> 3) & 7;
-        const int pos = h < 2 ? h - 2 : TILE + h - 2;
-        int c[3];
-        c[DIM] = o[DIM] + pos;
-        c[DA] = o[DA] + ta;
-        c[DB] = o[DB] + tb;
-        double q[7];
-        load_q<STAGE, false>(g, Usrc, c[0], c[1], c[2], q, st, false);
-#pragma unroll
-        for (int v = 0; v < 7; ++v) s.qh[v][tid] = q[v];
-    }
-    __syncthreads();
-
-    // 2. one face per thread: face f sits between along-positions f-1 and f
-    {
-        const int f = tid % (TILE + 1), rest = tid / (TILE + 1);
-        const int ta = rest & 7, tb = rest >> 3;
-        const bool valid = (o[DIM] + f <= N[DIM]) && (o[DA] + ta < N[DA]) && (o[DB] + tb < N[DB]);
-        double F[7];
-        bool bad = false;
-        if (valid) bad = face_flux<SOLVER, DIM>(g, s, f, ta, tb, gc, F);
-        else {
-#pragma unroll
-            for (int v = 0; v < 7; ++v) F[v] = 0.0;
-        }
-        if (bad) set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
-#pragma unroll
-        for (int v = 0; v < 7; ++v) s.fl[DIM][v][tid] = F[v];
-    }
-    __syncthreads();
-}
-
-// Flux divergence of one cell in the reference order, per dimension
-// += (A/V) F_L, -= (A/V) F_R (Hydro.cpp:117-137).  The accumulators are only
-// live here, not across the face solves.
-__device__ __forceinline__ void flux_divergence(const HydroGeom& g, const TileLDS& s, int tid, double udot[7]) {
-    const int lc[3] = {tid & 7, (tid >> 3) & 7, tid >> 6};
-#pragma unroll
-    for (int v = 0; v < 7; ++v) udot[v] = 0.0;
-#pragma unroll
-    for (int dim = 0; dim < 3; ++dim) {
-        const int a = lc[dim];
-        const int ta = lc[dim == 0 ? 1 : 0], tb = lc[dim == 2 ? 1 : 2];
-        const int fL = (tb * TILE + ta) * (TILE + 1) + a;
-#pragma unroll
-        for (int v = 0; v < 7; ++v) {
-            double u = udot[v];
-            u += g.kflux * s.fl[dim][v][fL];
-            u -= g.kflux * s.fl[dim][v][fL + 1];
-            udot[v] = u;
-        }
-    }
-}
-
-// dtf_host >= 0 overrides the stage's dt (st->dt / 2.0 for the predictor,
-// st->dt for the corrector) with a host-given, already scaled dt.
-template <int SOLVER, int STAGE>
-__global__ __launch_bounds__(NTHREADS) void hydro_stage_kernel(HydroGeom g, const double* __restrict__ Usrc,
-                                                              const double* Ubase, double* Udst, StepState* st,
-                                                              double dtf_host) {
-    __shared__ TileLDS s;
+template <int SOLVER, bool ALB, int STAGE>
+__global__ __launch_bounds__(QTHREADS) void hydro_tile_kernel(HydroGeom g, int ntx, int nty, int ntz,
+                                                              const double* __restrict__ Usrc, const double* Ubase,
+                                                              double* Udst, StepState* st, double dtf_host) {
+    __shared__ SmallLDS s;
     if (st->halted) return;  // a halted sub-step's pass-through is launch_halted_copy's
-    const int tile = tile_of_block(blockIdx.x, g.ntiles);
-    const int tx = tile % g.ntx, ty = (tile / g.ntx) % g.nty, tz = tile / (g.ntx * g.nty);
-    const int o[3] = {tx * TILE, ty * TILE, tz * TILE};
+    const int tile = tile_of_block(blockIdx.x, ntx * nty * ntz);
+    const int ox = (tile % ntx) * QX, oy = (tile / ntx % nty) * QY, oz = tile / (ntx * nty) * QZ;
     const int tid = threadIdx.x;
     const GasConsts<double> gc = {g.g, g.gm1, g.g2};
-
-    // tile cells: Q into LDS (ghost mapping for positions outside the grid)
-    const int lx = tid & 7, ly = (tid >> 3) & 7, lz = tid >> 6;
-    const int gx = o[0] + lx, gy = o[1] + ly, gz = o[2] + lz;
-    const bool active = tid < TCELLS && gx < g.nx && gy < g.ny && gz < g.nz;
-    if (tid < TCELLS) {
-        double q[7];
-        load_q<STAGE, false>(g, Usrc, gx, gy, gz, q, st, active);
-#pragma unroll
-        for (int v = 0; v < 7; ++v) s.qc[v][tid] = q[v];
-    }
-    sweep<SOLVER, STAGE, 0>(g, s, Usrc, o, st, gc);
-    sweep<SOLVER, STAGE, 1>(g, s, Usrc, o, st, gc);
-    sweep<SOLVER, STAGE, 2>(g, s, Usrc, o, st, gc);
-
-    double inv_t = 0.0;
-    if (active) {
-        double udot[7];
-        flux_divergence(g, s, tid, udot);
-        // gravity source with GRAV = 0 (Hydro.cpp:134-137)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const double grav = 0.0;
-            udot[VEL + i] += grav;
-            udot[PRE] += s.qc[VEL + i][tid] * grav;
+    const int lx = tid % QX, ly = tid / QX % QY, lz = tid / (QX * QY);
+    const bool active = tid < QCELLS && ox + lx < g.nx && oy + ly < g.ny && oz + lz < g.nz;
+    if (tid < QCELLS + QHX + QHY + QHZ) {
+        int x = lx, y = ly, z = lz;
+        if (tid >= QCELLS + QHX + QHY) {
+            const int h = tid - (QCELLS + QHX + QHY), l = h / (QX * QY);
+            x = h % QX, y = h / QX % QY, z = l < 2 ? l - 2 : QZ + l - 2;
+        } else if (tid >= QCELLS + QHX) {
+            const int h = tid - (QCELLS + QHX), l = h / (QX * QZ);
+            x = h % QX, z = h / QX % QZ, y = l < 2 ? l - 2 : QY + l - 2;
+        } else if (tid >= QCELLS) {
+            const int h = tid - QCELLS, l = h / (QY * QZ);
+            y = h % QY, z = h / QY % QZ, x = l < 2 ? l - 2 : QX + l - 2;
         }
-        const long long c = (long long)gx + (long long)g.nx * ((long long)gy + (long long)g.ny * gz);
-        const double dtf = stage_dtf(dtf_host, st, STAGE);
-        double u[7];
+        double q[7];
+        load_q<STAGE, false>(g, Usrc, ox + x, oy + y, oz + z, q, st, active);
+#pragma unroll
+        for (int v = 0; v < 7; ++v) s.q[v][tid] = q[v];
+    }
+    double u[7];  // the cell's base state, on its way while the faces are solved
+    const long long c = (long long)(ox + lx) + (long long)g.nx * ((long long)(oy + ly) + (long long)g.ny * (oz + lz));
+    if (active) {
 #pragma unroll
         for (int v = 0; v < 7; ++v) u[v] = Ubase[v * g.ncell + c];
+    }
+    __syncthreads();
+    bool bad = false;
+    double F[7] = {0, 0, 0, 0, 0, 0, 0};
+    if (tid < QZ0) {
+        const bool yface = tid >= QNX;
+        const int j = yface ? tid - QNX : tid;
+        const int x = yface ? j % QX : j % (QX + 1), y = yface ? j / (QX * QZ) : j / (QX + 1) % QY;
+        const int z = yface ? j / QX % QZ : j / ((QX + 1) * QY);
+        if (tid < QNX + QNY) {
+            if (ox + x < g.nx + !yface && oy + y < g.ny + yface && oz + z < g.nz)
+                bad = small_face<SOLVER, ALB, 0>(g, s, x, y, z, yface, gc, F);
+            double* dst = yface ? &s.fy[0][j] : &s.fx[0][j];
+            const int n = yface ? QNY : QNX;
 #pragma unroll
-        for (int v = 0; v < 7; ++v) u[v] += dtf * udot[v];
-        if (fix_solution(g, u)) set_error(st, STAGE == 1 ? ERR_FIX_SOLUTION_1 : ERR_FIX_SOLUTION_2);
+            for (int v = 0; v < 7; ++v) dst[v * n] = F[v];
+        }
+    } else if (tid < QZ0 + QNZ) {
+        const int j = tid - QZ0, x = j % QX, y = j / QX % QY, z = j / (QX * QY);
+        if (ox + x < g.nx && oy + y < g.ny && oz + z <= g.nz)
+            bad = small_face<SOLVER, ALB, 2>(g, s, x, y, z, false, gc, F);
+#pragma unroll
+        for (int v = 0; v < 7; ++v) s.fz[v][j] = F[v];
+    }
+    if (bad) set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+    __syncthreads();
+    double inv_t = 0.0;
+    if (active) {
+        // += (A/V) F_L, -= (A/V) F_R per dimension (Hydro.cpp:117-137)
+        double udot[7];
+        const int jx = lx + (QX + 1) * (ly + QY * lz), jy = lx + QX * (lz + QZ * ly), jz = lx + QX * (ly + QY * lz);
+#pragma unroll
+        for (int v = 0; v < 7; ++v) {
+            double d = 0.0;
+            d += g.kflux * s.fx[v][jx];
+            d -= g.kflux * s.fx[v][jx + 1];
+            d += g.kflux * s.fy[v][jy];
+            d -= g.kflux * s.fy[v][jy + QX * QZ];
+            d += g.kflux * s.fz[v][jz];
+            d -= g.kflux * s.fz[v][jz + QX * QY];
+            udot[v] = d;
+        }
+        inv_t = update_cell<STAGE>(g, u, udot, stage_dtf(dtf_host, st, STAGE), st);
 #pragma unroll
         for (int v = 0; v < 7; ++v) Udst[v * g.ncell + c] = u[v];
-        if (STAGE == 2) {
-            double q[7];
-            QfromU(q, u, g.gm1);
-            fix_primitives(g, q, u[DEN]);
-            inv_t = cfl_inv_t(g, q);
-        }
     }
-    if (STAGE == 2) block_max_to(inv_t, &st->maxinv, s.red);
+    if (STAGE == 2) block_max_to<QTHREADS>(inv_t, &st->maxinv, s.red);
+}
+
+// ---------------------------------------------------------------------------
+// The z march
+// ---------------------------------------------------------------------------
+constexpr int DT = 16;                      // columns are DT x DT cells
+constexpr int DTHREADS = DT * DT;
+constexpr int DPW = DT + 4;                 // plane row with its halos
+constexpr int DHALO = 8 * DT;               // x and y halo cells per plane
+constexpr int DNF = (DT + 1) * DT;          // x (and y) faces per plane
+constexpr int DNS = (DT + 2) * DT;          // cells with an x (and y) slope per plane
+constexpr int DN3 = 2 * DNF - 2 * DTHREADS; // faces past two per thread
+
+struct ColumnLDS {
+    double p[7][DPW * DPW];   // plane k: cell (x, y) at (y + 2) DPW + x + 2
+    // the limited slopes of plane k, then (after a barrier) its face fluxes
+    union {
+        struct {
+            double x[7][DNS];  // x slope of cell (x, y): y (DT + 2) + x + 1
+            double y[7][DNS];  // y slope of cell (x, y): (y + 1) DT + x
+        } s;
+        struct {
+            double x[7][DNF];  // x faces of plane k: y (DT + 1) + f
+            double y[7][DNF];  // y faces of plane k: f DT + x
+        } f;
+    } sf;
+    // fluxes that wait for the slopes' LDS: a thread's first face and the
+    // faces past two per thread
+    double park0[7][DTHREADS];
+    double park2[7][DN3];
+    double red[DTHREADS / 64];
+};
+
+__device__ __forceinline__ int dslot(int x, int y) { return (y + 2) * DPW + x + 2; }
+
+// Element at byte offset `off` (within one plane) of variable v at plane
+// base U + plane: scalar base plus 32-bit offset.
+template <typename T>
+__device__ __forceinline__ T* plane_at(T* U, long long ncell, int v, long long plane, unsigned int off) {
+    return (T*)((char*)(U + (v * ncell + plane)) + off);
+}
+
+// Halo cell h (0 .. DHALO - 1) of a plane: x halos first, then y halos.
+__device__ __forceinline__ void dhalo_pos(int h, int& x, int& y) {
+    const int l = (h & (4 * DT - 1)) / DT, r = h & (DT - 1), e = l < 2 ? l - 2 : DT + l - 2;
+    x = h < 4 * DT ? e : r;
+    y = h < 4 * DT ? r : e;
+}
+
+// x and y slopes of plane k: each thread its own cell's, 4 DT threads those of
+// the 1-deep halo cells, which the column's boundary faces read.
+template <bool ALB>
+__device__ __forceinline__ void dmarch_slopes(const HydroGeom& g, ColumnLDS& s, int tid, int ht, int tx, int ty,
+                                              const double w[7]) {
+    double a[7], c[7], sl[7];
+    const int o = dslot(tx, ty);
+#pragma unroll
+    for (int v = 0; v < 7; ++v) {
+        a[v] = s.p[v][o - 1];
+        c[v] = s.p[v][o + 1];
+    }
+    cell_slope<ALB>(g, a, w, c, sl);
+#pragma unroll
+    for (int v = 0; v < 7; ++v) s.sf.s.x[v][ty * (DT + 2) + tx + 1] = sl[v];
+#pragma unroll
+    for (int v = 0; v < 7; ++v) {
+        a[v] = s.p[v][o - DPW];
+        c[v] = s.p[v][o + DPW];
+    }
+    cell_slope<ALB>(g, a, w, c, sl);
+#pragma unroll
+    for (int v = 0; v < 7; ++v) s.sf.s.y[v][(ty + 1) * DT + tx] = sl[v];
+    if (ht < 4 * DT) {
+        const bool yh = ht >= 2 * DT;
+        const int side = (ht / DT) & 1, r = ht & (DT - 1);
+        const int hx = yh ? r : (side ? DT : -1), hy = yh ? (side ? DT : -1) : r;
+        const int ho = dslot(hx, hy), st = yh ? DPW : 1;
+        double b[7];
+#pragma unroll
+        for (int v = 0; v < 7; ++v) {
+            a[v] = s.p[v][ho - st];
+            b[v] = s.p[v][ho];
+            c[v] = s.p[v][ho + st];
+        }
+        cell_slope<ALB>(g, a, b, c, sl);
+        double* dst = yh ? &s.sf.s.y[0][(hy + 1) * DT + hx] : &s.sf.s.x[0][hy * (DT + 2) + hx + 1];
+#pragma unroll
+        for (int v = 0; v < 7; ++v) dst[v * DNS] = sl[v];
+    }
+}
+
+// One x face (item < DNF: row y = item / (DT + 1), face f) or y face (face f
+// = j / DT of column x) of plane k: flux in F (zero outside the grid).
+template <int SOLVER, int STAGE>
+__device__ __forceinline__ void dmarch_face(const HydroGeom& g, const ColumnLDS& s, int item, int ox, int oy,
+                                            StepState* st, const GasConsts<double>& gc, double F[7]) {
+    const bool yface = item >= DNF;
+    int qb, qs, sb, ss;
+    bool valid;
+    if (!yface) {
+        const int y = item / (DT + 1), f = item - y * (DT + 1);
+        valid = (ox + f <= g.nx) && (oy + y < g.ny);
+        qb = dslot(f - 1, y);
+        qs = 1;
+        sb = y * (DT + 2) + f;
+        ss = 1;
+    } else {
+        const int j = item - DNF, f = j / DT, x = j - f * DT;
+        valid = (oy + f <= g.ny) && (ox + x < g.nx);
+        qb = dslot(x, f - 1);
+        qs = DPW;
+        sb = DNS * 7 + f * DT + x;  // into the y slopes, which follow the x slopes
+        ss = DT;
+    }
+#pragma unroll
+    for (int v = 0; v < 7; ++v) F[v] = 0.0;
+    if (valid) {
+        double b[7], c[7], sbv[7], scv[7];
+        const double* sl = &s.sf.s.x[0][0];
+#pragma unroll
+        for (int v = 0; v < 7; ++v) {
+            b[v] = s.p[v][qb];
+            c[v] = s.p[v][qb + qs];
+            sbv[v] = sl[v * DNS + sb];
+            scv[v] = sl[v * DNS + sb + ss];
+        }
+        if (slope_flux<SOLVER, 0>(g, b, sbv, c, scv, gc, F, yface))
+            set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+    }
+}
+
+__device__ __forceinline__ void dstore_flux(ColumnLDS& s, int item, const double F[7]) {
+    double* dst = item >= DNF ? &s.sf.f.y[0][item - DNF] : &s.sf.f.x[0][item];
+#pragma unroll
+    for (int v = 0; v < 7; ++v) dst[v * DNF] = F[v];
+}
+
+template <int SOLVER, bool ALB, int STAGE>
+__global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) void hydro_march_kernel(
+    HydroGeom g, int ntx, int nty, int ntz, int mz, const double* __restrict__ Usrc, const double* Ubase, double* Udst,
+    StepState* st, double dtf_host) {
+    __shared__ ColumnLDS s;
+    if (st->halted) return;  // a halted sub-step's pass-through is launch_halted_copy's
+    const int tile = tile_of_block(blockIdx.x, ntx * nty * ntz);
+    const int ox = (tile % ntx) * DT, oy = (tile / ntx % nty) * DT, z0 = tile / (ntx * nty) * mz;
+    const int z1 = min(z0 + mz, g.nz);
+    const int tid = threadIdx.x, tx = tid % DT, ty = tid / DT;
+    const int gx = ox + tx, gy = oy + ty;
+    const bool col = gx < g.nx && gy < g.ny;
+    const GasConsts<double> gc = {g.g, g.gm1, g.g2};
+    const double dtf = stage_dtf(dtf_host, st, STAGE);
+    const long long pl = (long long)g.nx * g.ny;
+    // the own column's source in a plane and, past the x or y end of the grid
+    // (a ghost column that the last faces read), its velocity rule
+    const CellSrc own = cell_source(g, gx, gy, z0);
+    const unsigned int off = 8u * (unsigned int)(own.idx - pl * z0);
+    // Q of the own column's plane z (ghost planes by the z boundary
+    // condition; own cells are checked once, by the workgroup that owns them)
+    const auto load_u = [&](int z, double u[7]) {
+        const int zs = ghost_map(z, g.nz, g.bc_l[2], g.bc_r[2]).src;
+#pragma unroll
+        for (int v = 0; v < 7; ++v) u[v] = *plane_at(Usrc, g.ncell, v, pl * zs, off);
+    };
+    const auto to_q = [&](int z, const double u[7], double q[7]) {
+        const bool zg = (unsigned)z >= (unsigned)g.nz;
+        const int zmode = ghost_map(z, g.nz, g.bc_l[2], g.bc_r[2]).mode;
+        q_of_cell<STAGE, false>(g, u, own.mdim ? own.mode : zmode, own.mdim ? own.mdim : (zg ? 3 : 0), q, st,
+                                col && z >= z0 && z < z1);
+    };
+
+    double sk[7], w1[7], w2[7], w3[7], fz[7];
+    {
+        double a[7], w0[7], s0[7], u[7];
+        load_u(z0 - 2, u);
+        to_q(z0 - 2, u, a);
+        load_u(z0 - 1, u);
+        to_q(z0 - 1, u, w0);
+        load_u(z0, u);
+        to_q(z0, u, w1);
+        load_u(z0 + 1, u);
+        to_q(z0 + 1, u, w2);
+        cell_slope<ALB>(g, a, w0, w1, s0);
+        cell_slope<ALB>(g, w0, w1, w2, sk);
+        if (col && slope_flux<SOLVER, 2>(g, w0, s0, w1, sk, gc, fz))  // face z0 - 1/2
+            set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+        load_u(z0 + 2, u);
+        to_q(z0 + 2, u, w3);
+    }
+    double inv_t = 0.0;
+    for (int k = z0; k < z1; ++k) {
+        // The extra work of a plane (halo cells, halo slopes, third faces)
+        // goes to another wave each plane.
+        const int turn = (tid + 64 * (k & 3)) & (DTHREADS - 1);
+        double un[7];
+        if (k + 1 < z1) load_u(k + 3, un);  // used at the plane's end
+#pragma unroll
+        for (int v = 0; v < 7; ++v) s.p[v][dslot(tx, ty)] = w1[v];
+        if (turn < DHALO) {
+            int hx, hy;
+            dhalo_pos(turn, hx, hy);
+            double hq[7];
+            load_q<STAGE, false>(g, Usrc, ox + hx, oy + hy, k, hq, st, false);
+            const int hs = dslot(hx, hy);
+#pragma unroll
+            for (int v = 0; v < 7; ++v) s.p[v][hs] = hq[v];
+        }
+        __syncthreads();
+        // x and y slopes, then the faces; each flux waits (in LDS or, the
+        // last one solved, in registers) until every face has read the
+        // slopes, whose LDS the fluxes then take over
+        dmarch_slopes<ALB>(g, s, tid, turn, tx, ty, w1);
+        __syncthreads();
+        {
+            double F[7];
+#pragma unroll 1
+            for (int j = turn < DN3 ? -1 : 0; j < 2; ++j) {
+                dmarch_face<SOLVER, STAGE>(g, s, j < 0 ? 2 * DTHREADS + turn : tid + j * DTHREADS, ox, oy, st, gc, F);
+                if (j < 0) {
+#pragma unroll
+                    for (int v = 0; v < 7; ++v) s.park2[v][turn] = F[v];
+                } else if (j == 0) {
+#pragma unroll
+                    for (int v = 0; v < 7; ++v) s.park0[v][tid] = F[v];
+                }
+            }
+            __syncthreads();
+            dstore_flux(s, tid + DTHREADS, F);
+#pragma unroll
+            for (int v = 0; v < 7; ++v) F[v] = s.park0[v][tid];
+            dstore_flux(s, tid, F);
+            if (turn < DN3) {
+#pragma unroll
+                for (int v = 0; v < 7; ++v) F[v] = s.park2[v][turn];
+                dstore_flux(s, turn + 2 * DTHREADS, F);
+            }
+        }
+        // z face k + 1/2 from registers
+        double fzn[7] = {0, 0, 0, 0, 0, 0, 0}, u[7];
+        {
+            double sn[7];
+            cell_slope<ALB>(g, w1, w2, w3, sn);
+            if (col && slope_flux<SOLVER, 2>(g, w1, sk, w2, sn, gc, fzn))
+                set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+#pragma unroll
+            for (int v = 0; v < 7; ++v) sk[v] = sn[v];
+        }
+        if (col) {
+#pragma unroll
+            for (int v = 0; v < 7; ++v) u[v] = *plane_at(Ubase, g.ncell, v, pl * k, off);
+        }
+        __syncthreads();
+        if (col) {
+            // += (A/V) F_L, -= (A/V) F_R per dimension (Hydro.cpp:117-137)
+            double udot[7];
+            const int fxl = ty * (DT + 1) + tx, fyl = ty * DT + tx;
+#pragma unroll
+            for (int v = 0; v < 7; ++v) {
+                double d = 0.0;
+                d += g.kflux * s.sf.f.x[v][fxl];
+                d -= g.kflux * s.sf.f.x[v][fxl + 1];
+                d += g.kflux * s.sf.f.y[v][fyl];
+                d -= g.kflux * s.sf.f.y[v][fyl + DT];
+                d += g.kflux * fz[v];
+                d -= g.kflux * fzn[v];
+                udot[v] = d;
+            }
+            const double t = update_cell<STAGE>(g, u, udot, dtf, st);
+            if (t > inv_t) inv_t = t;
+#pragma unroll
+            for (int v = 0; v < 7; ++v) *plane_at(Udst, g.ncell, v, pl * k, off) = u[v];
+        }
+#pragma unroll
+        for (int v = 0; v < 7; ++v) {
+            fz[v] = fzn[v];
+            w1[v] = w2[v];
+            w2[v] = w3[v];
+        }
+        if (k + 1 < z1) to_q(k + 3, un, w3);
+    }
+    if (STAGE == 2) block_max_to<DTHREADS>(inv_t, &st->maxinv, s.red);
 }
 
 // Standalone CFL reduction over U (Hydrodynamics::calculateTimeStep on
@@ -496,23 +793,81 @@ hipError_t launch_fix_solution(const HydroGeom& g, double* U, const double* rate
     return hipGetLastError();
 }
 
-template <int SOLVER>
+// Which layout, and how many planes per march workgroup: the smallest of
+// estimates from times measured on this part (one stage, rotated solver, van
+// Albada).  A march workgroup takes about 17 us per plane alone on a CU and
+// 26 us beside a second one, with 1.2 planes' worth of work before its first;
+// up to 512 run at once, and of more the last leave half a workgroup's time
+// unfilled.  The tiles take 12 us and 0.29 ns per cell.  Measured us per step
+// (two stages), tiles / march / the single 8^3-tile kernel before: 16^3 26 /
+// 169 (pieces of 4 planes) / 97; 64^3 159 / 169 / 200; 80^3 307 / 240 / 383;
+// 128^3 1,193 / 864 / 1,487; 205x173x190 4,194 / 2,943 / 5,093; 256^3 9,870 /
+// 6,609 / 12,251 (1,369 -> 2,539 Mcell-updates/s).
+struct StagePlan {
+    bool march;
+    int mz;
+};
+
+static StagePlan stage_plan(const HydroGeom& g) {
+    const long long cols = (long long)((g.nx + DT - 1) / DT) * ((g.ny + DT - 1) / DT);
+    StagePlan p{false, g.nz};
+    double best = 12.0 + 0.29e-3 * (double)g.ncell;
+    // the march's 32-bit offsets cover planes of fewer than 2^29 cells
+    if ((long long)g.nx * g.ny >= (1LL << 29)) return p;
+    // pieces of 2 .. 32 planes (longer ones lose the halo's reuse in L2)
+    for (int pieces = (g.nz + 31) / 32; pieces <= 4 * ((g.nz + 31) / 32) + 12; ++pieces) {
+        const int mz = (g.nz + pieces - 1) / pieces;
+        if (mz < 2 && g.nz > 1) break;
+        const long long blocks = cols * ((g.nz + mz - 1) / mz);
+        const double rounds = blocks <= 256 ? 17.0 / 26.0 : blocks <= 512 ? 1.0 : 0.5 + (double)blocks / 512.0;
+        const double t = 26.0 * rounds * (mz + 1.2);
+        if (t < best) {
+            best = t;
+            p = StagePlan{true, mz};
+        }
+    }
+    return p;
+}
+
+template <int SOLVER, bool ALB>
 static hipError_t launch_stage_t(const HydroGeom& g, int stage, const double* Usrc, const double* Ubase, double* Udst,
                                  StepState* st, double dtf, hipStream_t stream) {
-    dim3 grid(g.ntiles), block(NTHREADS);
+    const StagePlan plan = stage_plan(g);
+    if (plan.march) {
+        const int mtx = (g.nx + DT - 1) / DT, mty = (g.ny + DT - 1) / DT, mtz = (g.nz + plan.mz - 1) / plan.mz;
+        dim3 grid(mtx * mty * mtz), block(DTHREADS);
+        if (stage == 1)
+            hipLaunchKernelGGL((hydro_march_kernel<SOLVER, ALB, 1>), grid, block, 0, stream, g, mtx, mty, mtz, plan.mz,
+                               Usrc, Ubase, Udst, st, dtf);
+        else
+            hipLaunchKernelGGL((hydro_march_kernel<SOLVER, ALB, 2>), grid, block, 0, stream, g, mtx, mty, mtz, plan.mz,
+                               Usrc, Ubase, Udst, st, dtf);
+        return hipGetLastError();
+    }
+    const int ntx = (g.nx + QX - 1) / QX, nty = (g.ny + QY - 1) / QY, ntz = (g.nz + QZ - 1) / QZ;
+    dim3 grid(ntx * nty * ntz), block(QTHREADS);
     if (stage == 1)
-        hipLaunchKernelGGL((hydro_stage_kernel<SOLVER, 1>), grid, block, 0, stream, g, Usrc, Ubase, Udst, st, dtf);
+        hipLaunchKernelGGL((hydro_tile_kernel<SOLVER, ALB, 1>), grid, block, 0, stream, g, ntx, nty, ntz, Usrc, Ubase,
+                           Udst, st, dtf);
     else
-        hipLaunchKernelGGL((hydro_stage_kernel<SOLVER, 2>), grid, block, 0, stream, g, Usrc, Ubase, Udst, st, dtf);
+        hipLaunchKernelGGL((hydro_tile_kernel<SOLVER, ALB, 2>), grid, block, 0, stream, g, ntx, nty, ntz, Usrc, Ubase,
+                           Udst, st, dtf);
     return hipGetLastError();
+}
+
+template <int SOLVER>
+static hipError_t launch_stage_l(const HydroGeom& g, int stage, const double* Usrc, const double* Ubase, double* Udst,
+                                 StepState* st, double dtf, hipStream_t stream) {
+    if (g.limiter == LIM_ALBADA) return launch_stage_t<SOLVER, true>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
+    return launch_stage_t<SOLVER, false>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
 }
 
 hipError_t launch_hydro_stage(const HydroGeom& g, int solver, int stage, const double* Usrc, const double* Ubase,
                               double* Udst, StepState* st, hipStream_t stream, double dtf) {
     switch (solver) {
-    case SOLVER_HLL:  return launch_stage_t<SOLVER_HLL>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
-    case SOLVER_HLLC: return launch_stage_t<SOLVER_HLLC>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
-    default:          return launch_stage_t<SOLVER_ROTATED>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
+    case SOLVER_HLL:  return launch_stage_l<SOLVER_HLL>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
+    case SOLVER_HLLC: return launch_stage_l<SOLVER_HLLC>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
+    default:          return launch_stage_l<SOLVER_ROTATED>(g, stage, Usrc, Ubase, Udst, st, dtf, stream);
     }
 }
 

@@ -9,12 +9,6 @@
 
 namespace tg {
 
-constexpr int TILE = 8;
-constexpr int TCELLS = TILE * TILE * TILE;        // 512
-constexpr int TFACES = (TILE + 1) * TILE * TILE;  // 576
-constexpr int THALO = 4 * TILE * TILE;            // 256 (2 layers x 2 sides)
-constexpr int NTHREADS = TFACES;
-
 __device__ __forceinline__ int tile_of_block(int b, int ntiles) {
     const int q = ntiles >> 3, r = ntiles & 7;
     const int x = b & 7, i = b >> 3;
@@ -191,7 +185,8 @@ __device__ __forceinline__ void set_error(StepState* st, unsigned int bit) {
 }
 
 // Block-wide max of non-negative doubles (NaN entries ignored) -> one
-// atomicMax on the bit pattern.  All NTHREADS threads must call it.
+// atomicMax on the bit pattern.  All NT threads must call it.
+template <int NT>
 __device__ __forceinline__ void block_max_to(double v, unsigned long long* dst, double* red) {
     if (!(v >= 0.0)) v = 0.0;
 #pragma unroll
@@ -201,7 +196,7 @@ __device__ __forceinline__ void block_max_to(double v, unsigned long long* dst, 
     __syncthreads();
     if (threadIdx.x == 0) {
         double m = red[0];
-        for (int w = 1; w < NTHREADS / 64; ++w) m = fmax(m, red[w]);
+        for (int w = 1; w < NT / 64; ++w) m = fmax(m, red[w]);
         atomicMax(dst, (unsigned long long)__double_as_longlong(m));
     }
 }

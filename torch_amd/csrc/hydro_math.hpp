@@ -14,7 +14,10 @@
 //                          dot x0+(x1+x2), mat*vec (l0r0+l1r1)+l2r2,
 //                          normalize x*(1/|x|).
 // The face normal DIM is a template parameter so that every component index
-// is resolved at compile time (no dynamically indexed register arrays).
+// is resolved at compile time (no dynamically indexed register arrays).  y
+// faces go through the x-face code with the x and y velocity components
+// exchanged: every sum of the solvers is over two terms, or adds x and y
+// first, where the exchange commutes, except the norms of rotated_hllc.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -184,140 +187,143 @@ __device__ __forceinline__ bool hll(R F[7], const R* Ql, const R* Qr, R a_l2, R 
     return F[HII] != F[HII];
 }
 
+// Rotation that maps a unit vector n onto the face axis d (getRotationFromA2B,
+// Riemann.cpp: M = (I + [v]x) + (k [v]x) [v]x with v = n x d,
+// k = (1 - n.d) / |v|^2), and back.  With d a coordinate axis v has two
+// components and [v]x four, so M holds n's transverse components, k times
+// them and 1 minus their products; the products left out are exact zeros and
+// ones, so every entry is the full form's bit for bit (up to the sign of a
+// zero).  The map back (d onto n) has the same k and products and the
+// opposite transverse signs.  Four 3 x 3 matrix evaluations with two divides
+// and two square roots more per face went with this.
 template <typename R>
-__device__ __forceinline__ void cross3(const R a[3], const R b[3], R r[3]) {
-    r[0] = a[1] * b[2] - a[2] * b[1];
-    r[1] = a[2] * b[0] - a[0] * b[2];
-    r[2] = a[0] * b[1] - a[1] * b[0];
-}
-template <typename R>
-__device__ __forceinline__ R dot3(const R a[3], const R b[3]) {
-    return a[0] * b[0] + (a[1] * b[1] + a[2] * b[2]);
-}
-template <typename R>
-__device__ __forceinline__ R norm3(const R a[3]) { return sqrt(dot3(a, a)); }
+struct AxisRotation {
+    R a, b;                    // transverse components of n
+    R nn, aa, bb, ab, ba;      // M_NN, M_AA, M_BB, M_AB, M_BA
+};
 
-// getRotationFromA2B: R = (I + [v]x) + (k [v]x) [v]x with v = A x B,
-// k = (1 - A.B) / |v|^2.
+// n: normal component and transverse ones; s: |(a, b)|
 template <typename R>
-__device__ __forceinline__ void rot_a2b(const R A[3], const R B[3], R M[3][3]) {
-    R v[3];
-    cross3(A, B, v);
-    R s = norm3(v);
-    R cc = dot3(A, B);
-    const R vx[3][3] = {{R(0), -v[2], v[1]}, {v[2], R(0), -v[0]}, {-v[1], v[0], R(0)}};
-    R k = (R(1.0) - cc) / (s * s);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            R p = (k * vx[i][0]) * vx[0][j];
-            p += (k * vx[i][1]) * vx[1][j];
-            p += (k * vx[i][2]) * vx[2][j];
-            M[i][j] = ((i == j ? R(1.0) : R(0.0)) + vx[i][j]) + p;
-        }
+__device__ __forceinline__ AxisRotation<R> axis_rotation(R n, R a, R b, R s) {
+    AxisRotation<R> m;
+    const R k = (R(1.0) - n) / (s * s);
+    const R ka = k * a, kb = k * b;
+    const R x = ka * a, y = kb * b;
+    m.a = a;
+    m.b = b;
+    m.nn = R(1.0) - (x + y);
+    m.aa = R(1.0) - x;
+    m.bb = R(1.0) - y;
+    m.ab = -(ka * b);
+    m.ba = -(kb * a);
+    return m;
 }
 
-template <typename R>
-__device__ __forceinline__ void rotate(const R M[3][3], R* v) {
-    const R a = v[VEL + 0], b = v[VEL + 1], cz = v[VEL + 2];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        R r = M[i][0] * a;
-        r += M[i][1] * b;
-        r += M[i][2] * cz;
-        v[VEL + i] = r;
-    }
-}
-
-// RotatedHartenLaxLeerSolver::solve (Nishikawa & Kitamura 2008).
-template <typename R, int DIM>
-__device__ __forceinline__ bool rotated_hllc(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c) {
-    bool pureHLLC = false, pureHLL = false;
-    const R d[3] = {DIM == 0 ? R(1) : R(0), DIM == 1 ? R(1) : R(0), DIM == 2 ? R(1) : R(0)};
-    R n1[3] = {Qr[VEL + 0] - Ql[VEL + 0], Qr[VEL + 1] - Ql[VEL + 1], Qr[VEL + 2] - Ql[VEL + 2]};
-    R n2[3] = {R(0), R(0), R(0)};
-    R t[3];
-    if (n1[DIM] < R(0)) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) n1[i] = R(-1.0) * n1[i];
-    }
-    if (norm3(n1) < R(1.0e-6)) {
-        pureHLLC = true;
+// v <- M v (BACK: the map back); each row is summed in component order, as
+// Eigen's product does.
+template <typename R, int DIM, bool BACK>
+__device__ __forceinline__ void rotate(const AxisRotation<R>& m, R* v) {
+    constexpr int A = VEL + (DIM == 0 ? 1 : 0), B = VEL + (DIM == 2 ? 1 : 2), N = VEL + DIM;
+    const R a = BACK ? -m.a : m.a, b = BACK ? -m.b : m.b;
+    const R n = v[N], va = v[A], vb = v[B];
+    if (DIM == 2) {
+        v[N] = (a * va + b * vb) + m.nn * n;
+        v[A] = (m.aa * va + m.ab * vb) - a * n;
+        v[B] = (m.ba * va + m.bb * vb) - b * n;
     } else {
-        const R inv = R(1.0) / norm3(n1);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) n1[i] *= inv;
-        cross3(n1, d, t);
-        if (norm3(t) == R(0)) {
-            pureHLL = true;
-        } else {
-            cross3(t, n1, n2);
-            if (norm3(n2) == R(0)) {
-                pureHLL = true;
-            } else {
-                if (n2[DIM] < R(0)) {
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) n2[i] = R(-1.0) * n2[i];
-                }
-                const R inv2 = R(1.0) / norm3(n2);
-#pragma unroll
-                for (int i = 0; i < 3; ++i) n2[i] *= inv2;
-                cross3(n2, d, t);
-                if (norm3(t) == R(0)) pureHLLC = true;
-            }
-        }
+        v[N] = (m.nn * n + a * va) + b * vb;
+        v[A] = (m.aa * va - a * n) + m.ab * vb;
+        v[B] = (m.ba * va - b * n) + m.bb * vb;
     }
+}
+
+// RotatedHartenLaxLeerSolver::solve (Nishikawa & Kitamura 2008).  yface (DIM
+// 0 only): a y face whose x and y velocity components the caller has
+// exchanged; sums of three squares are then taken in the original order (all
+// other sums are over two terms, or commute in x and y).
+template <typename R, int DIM>
+__device__ __forceinline__ bool rotated_hllc(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c,
+                                             bool yface) {
+    static_assert(DIM == 0 || DIM == 2, "y faces are solved as x faces");
+    constexpr int A = DIM == 0 ? 1 : 0, B = DIM == 2 ? 1 : 2;
+    const auto norm = [yface](const R v[3]) {
+        const R x = v[0] * v[0], y = v[1] * v[1], z = v[2] * v[2];
+        if (DIM == 2) return sqrt(x + (y + z));
+        return sqrt((yface ? y : x) + ((yface ? x : y) + z));
+    };
+    R n1[3] = {Qr[VEL + 0] - Ql[VEL + 0], Qr[VEL + 1] - Ql[VEL + 1], Qr[VEL + 2] - Ql[VEL + 2]};
+    const bool neg = n1[DIM] < R(0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) n1[i] = neg ? -n1[i] : n1[i];
+    const R l1 = norm(n1);
+    bool pureHLLC = l1 < R(1.0e-6);
+    // n1 along the velocity jump; n2 = (n1 x d) x n1 perpendicular to it in
+    // the plane of n1 and the axis d
+    const R inv = R(1.0) / l1;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) n1[i] *= inv;
+    const R s1sq = n1[A] * n1[A] + n1[B] * n1[B], s1 = sqrt(s1sq);
+    R n2[3];
+    n2[DIM] = s1sq;
+    n2[A] = -(n1[A] * n1[DIM]);
+    n2[B] = -(n1[B] * n1[DIM]);
+    const R l2 = norm(n2);
+    const bool pureHLL = !pureHLLC && (s1 == R(0) || l2 == R(0));
+    const R inv2 = R(1.0) / l2;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) n2[i] *= inv2;
+    const R s2sq = n2[A] * n2[A] + n2[B] * n2[B], s2 = sqrt(s2sq);
+    pureHLLC = pureHLLC || (!pureHLL && s2 == R(0));
     // One HLL and one HLLC solve per face for every lane: on the hybrid path
     // they take the rotated states, on the pure paths the unrotated ones (the
     // reference's single solve; the other result is discarded), so a wave
     // with mixed paths runs the solvers once instead of once per path.
     const bool hybrid = !pureHLLC && !pureHLL;
-    R F1[7], F2[7], QlR[7], QrR[7], Qa[7], Qb[7], M[3][3];
+    const AxisRotation<R> m1 = axis_rotation<R>(n1[DIM], n1[A], n1[B], s1);
+    R F1[7], F2[7], QlR[7], QrR[7], Qa[7], Qb[7];
 #pragma unroll
     for (int i = 0; i < 7; ++i) { QlR[i] = Ql[i]; QrR[i] = Qr[i]; }
-    rot_a2b(n1, d, M);
-    rotate(M, QlR);
-    rotate(M, QrR);
+    rotate<R, DIM, false>(m1, QlR);
+    rotate<R, DIM, false>(m1, QrR);
 #pragma unroll
     for (int i = 0; i < 7; ++i) { Qa[i] = hybrid ? QlR[i] : Ql[i]; Qb[i] = hybrid ? QrR[i] : Qr[i]; }
     const bool bad1 = hll<R, DIM>(F1, Qa, Qb, a_l2, a_r2, c);
-    rot_a2b(d, n1, M);
-    rotate(M, QlR);
-    rotate(M, QrR);
+    rotate<R, DIM, true>(m1, QlR);
+    rotate<R, DIM, true>(m1, QrR);
     // A = w1 * (M F1) on the hybrid path (the first term of the reference's
     // w1 F1 + w2 F2), F1 itself on the pure-HLL path
-    const R w1 = fabs(dot3(d, n1));
+    const R w1 = fabs(n1[DIM]);
     {
         R Fr[7];
 #pragma unroll
         for (int i = 0; i < 7; ++i) Fr[i] = F1[i];
-        rotate(M, Fr);
+        rotate<R, DIM, true>(m1, Fr);
 #pragma unroll
         for (int i = 0; i < 7; ++i) F1[i] = hybrid ? w1 * Fr[i] : F1[i];
     }
-    rot_a2b(n2, d, M);
-    rotate(M, QlR);
-    rotate(M, QrR);
+    const AxisRotation<R> m2 = axis_rotation<R>(n2[DIM], n2[A], n2[B], s2);
+    rotate<R, DIM, false>(m2, QlR);
+    rotate<R, DIM, false>(m2, QrR);
 #pragma unroll
     for (int i = 0; i < 7; ++i) { Qa[i] = hybrid ? QlR[i] : Ql[i]; Qb[i] = hybrid ? QrR[i] : Qr[i]; }
     const bool bad2 = hllc<R, DIM>(F2, Qa, Qb, a_l2, a_r2, c);
-    rot_a2b(d, n2, M);
-    const R w2 = fabs(dot3(d, n2));
+    const R w2 = fabs(n2[DIM]);
     R Fr[7];
 #pragma unroll
     for (int i = 0; i < 7; ++i) Fr[i] = F2[i];
-    rotate(M, Fr);
+    rotate<R, DIM, true>(m2, Fr);
 #pragma unroll
     for (int i = 0; i < 7; ++i) F[i] = hybrid ? F1[i] + w2 * Fr[i] : (pureHLL ? F1[i] : F2[i]);
     return hybrid ? (bad1 || bad2) : (pureHLL ? bad1 : bad2);
 }
 
+// Face flux along DIM (0 or 2; yface: see rotated_hllc).
 template <int SOLVER, typename R, int DIM>
-__device__ __forceinline__ bool riemann(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c) {
+__device__ __forceinline__ bool riemann(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c,
+                                        bool yface) {
     if constexpr (SOLVER == SOLVER_HLL) return hll<R, DIM>(F, Ql, Qr, a_l2, a_r2, c);
     else if constexpr (SOLVER == SOLVER_HLLC) return hllc<R, DIM>(F, Ql, Qr, a_l2, a_r2, c);
-    else return rotated_hllc<R, DIM>(F, Ql, Qr, a_l2, a_r2, c);
+    else return rotated_hllc<R, DIM>(F, Ql, Qr, a_l2, a_r2, c, yface);
 }
 
 // ---------------------------------------------------------------------------

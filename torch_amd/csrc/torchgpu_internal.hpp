@@ -11,8 +11,6 @@ namespace tg {
 // Grid + hydro parameters, passed by value to every hydro kernel.
 struct HydroGeom {
     int nx, ny, nz;
-    int ntx, nty, ntz;      // 8^3 tiles per dimension
-    int ntiles;
     int bc_l[3], bc_r[3];
     int limiter;
     int spatial_order;
