@@ -78,7 +78,7 @@ def test_solver_limiter_variants_ragged_grid(gpu, orc, solver, limiter, order):
 
 
 # sizes on both sides of the two FP64 layouts' rule (8 x 4 x 4 tiles below about
-# half a million cells, 16 x 16 columns marched along z above), none a
+# a quarter of a million cells, 16 x 16 columns marched along z above), none a
 # multiple of a tile, a column or a column's planes
 @pytest.mark.parametrize("nz,ny,nx", [(3, 5, 7), (21, 33, 18), (85, 91, 101), (4, 301, 323), (131, 70, 75)])
 @pytest.mark.parametrize("solver,limiter,order,bcs", [
@@ -102,6 +102,38 @@ def test_layouts_bitwise(gpu, orc, nz, ny, nx, solver, limiter, order, bcs):
     kw = dict(tfloor=1e-12, pfloor=0.1 * 8.314462e7 * 1e-30 * 1e-12, solver=solver, limiter=limiter,
               spatial_order=order, bc=bcs)
     Ug, Uo, cg, co = _run_both(gpu, orc, Q, 3, gkw=dict(kw), okw=dict(kw))
+    assert Ug is not None
+    np.testing.assert_array_equal(Ug, Uo)
+    assert cg == co
+
+
+# states partly outside the range of the quick divisions: velocities and
+# fractions down to 1e-110 (below 2^-300, or with differences and products
+# that are) from a middle plane on, in one corner, or everywhere in steps of
+# 1e-12 (the march stops at them), thin gas, a cell wider than 2^64; a tile grid and two
+# march grids with several pieces along z
+@pytest.mark.parametrize("nz,ny,nx", [(9, 13, 18), (70, 85, 91), (131, 70, 75)])
+@pytest.mark.parametrize("state", ["tails", "corner", "quiet", "thin", "wide"])
+@pytest.mark.parametrize("solver", ["RotatedHLLC", "HLL"])
+def test_quick_division_range_bitwise(gpu, orc, nz, ny, nx, state, solver):
+    rng = np.random.Generator(np.random.PCG64(nz))
+    Q = 0.5 + 0.3 * rng.random((7, nz, ny, nx))
+    Q[4:] -= 0.65
+    kw = dict(tfloor=1e-12, pfloor=1e-60, dfloor=1e-60, solver=solver, limiter="albada")
+    gkw = dict(kw)
+    if state == "tails":
+        Q[2:, nz // 3 + 1:] *= 10.0 ** rng.uniform(-110.0, 0.0, Q[2:, nz // 3 + 1:].shape)
+    elif state == "corner":
+        Q[4:, -2:, -2:, -1:] = 1e-100
+        Q[3, 0, 0, 0] = 1e-300
+    elif state == "quiet":  # the solver's pure paths, and its choice between them
+        Q[4:] *= 10.0 ** (-12.0 * rng.integers(0, 9, (1, nz, 1, 1)))
+        Q[0], Q[1] = 1.0, 1.0
+    elif state == "thin":
+        Q[:2, nz // 2:, ny // 2:, :5] *= 1e-33
+    else:
+        gkw["side_length"] = 1e22
+    Ug, Uo, cg, co = _run_both(gpu, orc, Q, 3, gkw=gkw, okw=dict(kw))
     assert Ug is not None
     np.testing.assert_array_equal(Ug, Uo)
     assert cg == co

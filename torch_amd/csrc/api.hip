@@ -8,6 +8,7 @@
 #include <utility>
 
 #include "../../include/torchgpu.h"
+#include "hydro_device.hpp"
 #include "torchgpu_internal.hpp"
 
 struct torchgpu_ctx {
@@ -248,6 +249,7 @@ int torchgpu_create(const torchgpu_params* p, void* stream, torchgpu_ctx** out) 
     g.igm1f = 1.0f / g.gm1f;
     g.igm1 = 1.0 / g.gm1;
     g.idx = 1.0 / g.dx;
+    g.fast = tg::constants_in_range(g) ? 1 : 0;
 
     c->stream = (hipStream_t)stream;  // NULL: the null (default) stream
     const size_t bytes = state_bytes(c);
@@ -258,6 +260,11 @@ int torchgpu_create(const torchgpu_params* p, void* stream, torchgpu_ctx** out) 
     }
     if (p->precision == TORCHGPU_MIXED &&
         (hipMalloc(&c->qf[0], bytes / 2) != hipSuccess || hipMalloc(&c->qf[1], bytes / 2) != hipSuccess)) {
+        torchgpu_destroy(c);
+        return TORCHGPU_ERR_HIP;
+    }
+    if (p->precision == TORCHGPU_FP64 &&
+        hipMalloc(&g.resume, sizeof(int) * (size_t)(tg::march_blocks(g) + 1)) != hipSuccess) {
         torchgpu_destroy(c);
         return TORCHGPU_ERR_HIP;
     }
@@ -280,6 +287,7 @@ void torchgpu_destroy(torchgpu_ctx* c) {
     if (c->qf[0]) (void)hipFree(c->qf[0]);
     if (c->qf[1]) (void)hipFree(c->qf[1]);
     if (c->heat) (void)hipFree(c->heat);
+    if (c->g.resume) (void)hipFree(c->g.resume);
     delete c;
 }
 

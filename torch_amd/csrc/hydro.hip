@@ -41,18 +41,24 @@
 // (ntiles / 8) + b / 8) so that each XCD's L2 sees neighbouring halos.  The
 // mixed-precision kernel is in hydro_mixed.hip.
 
+#include <type_traits>
+
 #include "hydro_device.hpp"
 
 namespace tg {
 
 // Limited slope of cell b between its neighbours a and c (0 at first order).
 // ALB: van Albada, the default, without the other limiters' code.
-template <bool ALB>
+// FAST: the three cells keep the divisions in range (Recip, hydro_math.hpp).
+template <bool ALB, bool FAST>
 __device__ __forceinline__ void cell_slope(const HydroGeom& g, const double a[7], const double b[7], const double c[7],
                                            double s[7]) {
     if (g.spatial_order == 1) {
 #pragma unroll
-        for (int v = 0; v < 7; ++v) s[v] = limiter<double>(ALB ? (int)LIM_ALBADA : g.limiter, b[v] - a[v], c[v] - b[v]);
+        for (int v = 0; v < 7; ++v) {
+            if constexpr (ALB) s[v] = albada<FAST>(b[v] - a[v], c[v] - b[v]);
+            else s[v] = limiter<double>(g.limiter, b[v] - a[v], c[v] - b[v]);
+        }
     } else {
 #pragma unroll
         for (int v = 0; v < 7; ++v) s[v] = 0.0;
@@ -63,8 +69,8 @@ __device__ __forceinline__ void cell_slope(const HydroGeom& g, const double a[7]
 // sb and sc: QR of b and QL of c (Hydrodynamics::reconstruct) and the Riemann
 // solve.  yswap (DIM 0): a y face, solved as an x face with the x and y
 // velocity components exchanged (see hydro_math.hpp).  Returns true if the
-// HII flux is NaN.
-template <int SOLVER, int DIM>
+// HII flux is NaN or, FAST, the flux not to be trusted.
+template <int SOLVER, int DIM, bool FAST>
 __device__ __forceinline__ bool slope_flux(const HydroGeom& g, const double b[7], const double sb[7], const double c[7],
                                            const double sc[7], const GasConsts<double>& gc, double F[7],
                                            bool yswap = false) {
@@ -81,9 +87,9 @@ __device__ __forceinline__ bool slope_flux(const HydroGeom& g, const double b[7]
         ql[VEL + 1] = lx;
         qr[VEL + 1] = rx;
     }
-    const double a_l2 = gc.g * ql[PRE] / ql[DEN];
-    const double a_r2 = gc.g * qr[PRE] / qr[DEN];
-    const bool bad = riemann<SOLVER, double, DIM>(F, ql, qr, a_l2, a_r2, gc, yswap);
+    const double a_l2 = div_r<FAST>(gc.g * ql[PRE], ql[DEN]);
+    const double a_r2 = div_r<FAST>(gc.g * qr[PRE], qr[DEN]);
+    const bool bad = riemann<SOLVER, FAST, DIM>(F, ql, qr, a_l2, a_r2, gc, yswap);
     if (DIM == 0 && yswap) {
         const double fx = F[VEL];
         F[VEL] = F[VEL + 1];
@@ -93,19 +99,23 @@ __device__ __forceinline__ bool slope_flux(const HydroGeom& g, const double b[7]
 }
 
 // Fluid::advSolution + fixSolution of one cell from its base state u and
-// flux divergence (the gravity source is zero, GRAV = 0), in place; stage 2
-// returns the CFL term of the new state.
-template <int STAGE>
-__device__ __forceinline__ double update_cell(const HydroGeom& g, double u[7], const double udot[7], double dtf,
-                                              StepState* st) {
+// flux divergence (the gravity source is zero, GRAV = 0), in place; inv_t: the
+// CFL term of the new state (stage 2).  Returns false (FAST) where the result
+// is not to be trusted.
+template <int STAGE, bool FAST>
+__device__ __forceinline__ bool update_cell(const HydroGeom& g, double u[7], const double udot[7], double dtf,
+                                            StepState* st, double& inv_t) {
 #pragma unroll
     for (int v = 0; v < 7; ++v) u[v] += dtf * udot[v];
-    if (fix_solution(g, u)) set_error(st, STAGE == 1 ? ERR_FIX_SOLUTION_1 : ERR_FIX_SOLUTION_2);
-    if (STAGE == 1) return 0.0;
-    double q[7];
-    QfromU(q, u, g.gm1);
-    fix_primitives(g, q, u[DEN]);
-    return cfl_inv_t(g, q);
+    const bool ok = !FAST || (conserved_in_range(u) & (dtf * g.kflux < 0x1p200));
+    if (fix_solution<FAST>(g, u) && ok) set_error(st, STAGE == 1 ? ERR_FIX_SOLUTION_1 : ERR_FIX_SOLUTION_2);
+    if (STAGE == 2) {
+        double q[7];
+        QfromU<FAST>(q, u, g.gm1);
+        fix_primitives<FAST>(g, q, u[DEN]);
+        inv_t = cfl_inv_t<FAST>(g, q);
+    }
+    return ok;
 }
 
 // ---------------------------------------------------------------------------
@@ -123,6 +133,7 @@ struct SmallLDS {
     double q[7][QCELLS + QHX + QHY + QHZ];
     double fx[7][QNX], fy[7][QNY], fz[7][QNZ];
     double red[QTHREADS / 64];
+    int slow;  // a cell, face or result is out of the quick divisions' range
 };
 
 // LDS slot of tile position (x, y, z), of which one may lie in a 2-deep halo.
@@ -136,7 +147,7 @@ __device__ __forceinline__ int qslot(int x, int y, int z) {
 
 // Face f of tile row (ox, oy, oz) + f along DIM: the four stencil cells, both
 // slopes and the solve.
-template <int SOLVER, bool ALB, int DIM>
+template <int SOLVER, bool ALB, int DIM, bool FAST>
 __device__ __forceinline__ bool small_face(const HydroGeom& g, const SmallLDS& s, int x, int y, int z, bool yface,
                                            const GasConsts<double>& gc, double F[7]) {
     const int dx = DIM == 0 && !yface, dy = DIM == 0 && yface, dz = DIM == 2;
@@ -147,9 +158,9 @@ __device__ __forceinline__ bool small_face(const HydroGeom& g, const SmallLDS& s
 #pragma unroll
         for (int v = 0; v < 7; ++v) q[i][v] = s.q[v][c];
     }
-    cell_slope<ALB>(g, q[0], q[1], q[2], sb);
-    cell_slope<ALB>(g, q[1], q[2], q[3], sc);
-    return slope_flux<SOLVER, DIM>(g, q[1], sb, q[2], sc, gc, F, yface);
+    cell_slope<ALB, FAST>(g, q[0], q[1], q[2], sb);
+    cell_slope<ALB, FAST>(g, q[1], q[2], q[3], sc);
+    return slope_flux<SOLVER, DIM, FAST>(g, q[1], sb, q[2], sc, gc, F, yface);
 }
 
 template <int SOLVER, bool ALB, int STAGE>
@@ -164,6 +175,8 @@ __global__ __launch_bounds__(QTHREADS) void hydro_tile_kernel(HydroGeom g, int n
     const GasConsts<double> gc = {g.g, g.gm1, g.g2};
     const int lx = tid % QX, ly = tid / QX % QY, lz = tid / (QX * QY);
     const bool active = tid < QCELLS && ox + lx < g.nx && oy + ly < g.ny && oz + lz < g.nz;
+    if (tid == 0) s.slow = 0;
+    __syncthreads();
     if (tid < QCELLS + QHX + QHY + QHZ) {
         int x = lx, y = ly, z = lz;
         if (tid >= QCELLS + QHX + QHY) {
@@ -177,58 +190,73 @@ __global__ __launch_bounds__(QTHREADS) void hydro_tile_kernel(HydroGeom g, int n
             y = h % QY, z = h / QY % QZ, x = l < 2 ? l - 2 : QX + l - 2;
         }
         double q[7];
-        load_q<STAGE, false>(g, Usrc, ox + x, oy + y, oz + z, q, st, active);
+        if (!load_q<STAGE, Q_BOTH>(g, Usrc, ox + x, oy + y, oz + z, q, st, active)) s.slow = 1;
 #pragma unroll
         for (int v = 0; v < 7; ++v) s.q[v][tid] = q[v];
     }
-    double u[7];  // the cell's base state, on its way while the faces are solved
+    double ub[7];  // the cell's base state, on its way while the faces are solved
     const long long c = (long long)(ox + lx) + (long long)g.nx * ((long long)(oy + ly) + (long long)g.ny * (oz + lz));
     if (active) {
 #pragma unroll
-        for (int v = 0; v < 7; ++v) u[v] = Ubase[v * g.ncell + c];
+        for (int v = 0; v < 7; ++v) ub[v] = Ubase[v * g.ncell + c];
     }
     __syncthreads();
-    bool bad = false;
-    double F[7] = {0, 0, 0, 0, 0, 0, 0};
-    if (tid < QZ0) {
-        const bool yface = tid >= QNX;
-        const int j = yface ? tid - QNX : tid;
-        const int x = yface ? j % QX : j % (QX + 1), y = yface ? j / (QX * QZ) : j / (QX + 1) % QY;
-        const int z = yface ? j / QX % QZ : j / ((QX + 1) * QY);
-        if (tid < QNX + QNY) {
-            if (ox + x < g.nx + !yface && oy + y < g.ny + yface && oz + z < g.nz)
-                bad = small_face<SOLVER, ALB, 0>(g, s, x, y, z, yface, gc, F);
-            double* dst = yface ? &s.fy[0][j] : &s.fx[0][j];
-            const int n = yface ? QNY : QNX;
+    const double dtf = stage_dtf(dtf_host, st, STAGE);
+    double inv_t = 0.0, u[7];
+    const auto solve = [&](auto fast_c) {
+        constexpr bool FAST = decltype(fast_c)::value;
+        bool bad = false;
+        double F[7] = {0, 0, 0, 0, 0, 0, 0};
+        if (tid < QZ0) {
+            const bool yface = tid >= QNX;
+            const int j = yface ? tid - QNX : tid;
+            const int x = yface ? j % QX : j % (QX + 1), y = yface ? j / (QX * QZ) : j / (QX + 1) % QY;
+            const int z = yface ? j / QX % QZ : j / ((QX + 1) * QY);
+            if (tid < QNX + QNY) {
+                if (ox + x < g.nx + !yface && oy + y < g.ny + yface && oz + z < g.nz)
+                    bad = small_face<SOLVER, ALB, 0, FAST>(g, s, x, y, z, yface, gc, F);
+                double* dst = yface ? &s.fy[0][j] : &s.fx[0][j];
+                const int n = yface ? QNY : QNX;
 #pragma unroll
-            for (int v = 0; v < 7; ++v) dst[v * n] = F[v];
+                for (int v = 0; v < 7; ++v) dst[v * n] = F[v];
+            }
+        } else if (tid < QZ0 + QNZ) {
+            const int j = tid - QZ0, x = j % QX, y = j / QX % QY, z = j / (QX * QY);
+            if (ox + x < g.nx && oy + y < g.ny && oz + z <= g.nz)
+                bad = small_face<SOLVER, ALB, 2, FAST>(g, s, x, y, z, false, gc, F);
+#pragma unroll
+            for (int v = 0; v < 7; ++v) s.fz[v][j] = F[v];
         }
-    } else if (tid < QZ0 + QNZ) {
-        const int j = tid - QZ0, x = j % QX, y = j / QX % QY, z = j / (QX * QY);
-        if (ox + x < g.nx && oy + y < g.ny && oz + z <= g.nz)
-            bad = small_face<SOLVER, ALB, 2>(g, s, x, y, z, false, gc, F);
+        if (bad && !FAST) set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+        __syncthreads();
+        bool ok = true;
+        if (active) {
+            // += (A/V) F_L, -= (A/V) F_R per dimension (Hydro.cpp:117-137)
+            double udot[7];
+            const int jx = lx + (QX + 1) * (ly + QY * lz), jy = lx + QX * (lz + QZ * ly), jz = lx + QX * (ly + QY * lz);
 #pragma unroll
-        for (int v = 0; v < 7; ++v) s.fz[v][j] = F[v];
+            for (int v = 0; v < 7; ++v) {
+                double d = 0.0;
+                d += g.kflux * s.fx[v][jx];
+                d -= g.kflux * s.fx[v][jx + 1];
+                d += g.kflux * s.fy[v][jy];
+                d -= g.kflux * s.fy[v][jy + QX * QZ];
+                d += g.kflux * s.fz[v][jz];
+                d -= g.kflux * s.fz[v][jz + QX * QY];
+                udot[v] = d;
+                u[v] = ub[v];
+            }
+            ok = update_cell<STAGE, FAST>(g, u, udot, dtf, st, inv_t);
+        }
+        return ok && !bad;
+    };
+    if (s.slow == 0) {
+        const bool ok = solve(std::true_type{});
+        if (!ok) s.slow = 1;
+        __syncthreads();
     }
-    if (bad) set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
-    __syncthreads();
-    double inv_t = 0.0;
+    if (s.slow != 0) solve(std::false_type{});
     if (active) {
-        // += (A/V) F_L, -= (A/V) F_R per dimension (Hydro.cpp:117-137)
-        double udot[7];
-        const int jx = lx + (QX + 1) * (ly + QY * lz), jy = lx + QX * (lz + QZ * ly), jz = lx + QX * (ly + QY * lz);
-#pragma unroll
-        for (int v = 0; v < 7; ++v) {
-            double d = 0.0;
-            d += g.kflux * s.fx[v][jx];
-            d -= g.kflux * s.fx[v][jx + 1];
-            d += g.kflux * s.fy[v][jy];
-            d -= g.kflux * s.fy[v][jy + QX * QZ];
-            d += g.kflux * s.fz[v][jz];
-            d -= g.kflux * s.fz[v][jz + QX * QY];
-            udot[v] = d;
-        }
-        inv_t = update_cell<STAGE>(g, u, udot, stage_dtf(dtf_host, st, STAGE), st);
 #pragma unroll
         for (int v = 0; v < 7; ++v) Udst[v * g.ncell + c] = u[v];
     }
@@ -264,6 +292,7 @@ struct ColumnLDS {
     double park0[7][DTHREADS];
     double park2[7][DN3];
     double red[DTHREADS / 64];
+    int stop[2];  // plane k & 1: a cell or face is out of the quick divisions' range
 };
 
 __device__ __forceinline__ int dslot(int x, int y) { return (y + 2) * DPW + x + 2; }
@@ -284,7 +313,7 @@ __device__ __forceinline__ void dhalo_pos(int h, int& x, int& y) {
 
 // x and y slopes of plane k: each thread its own cell's, 4 DT threads those of
 // the 1-deep halo cells, which the column's boundary faces read.
-template <bool ALB>
+template <bool ALB, bool FAST>
 __device__ __forceinline__ void dmarch_slopes(const HydroGeom& g, ColumnLDS& s, int tid, int ht, int tx, int ty,
                                               const double w[7]) {
     double a[7], c[7], sl[7];
@@ -294,7 +323,7 @@ __device__ __forceinline__ void dmarch_slopes(const HydroGeom& g, ColumnLDS& s, 
         a[v] = s.p[v][o - 1];
         c[v] = s.p[v][o + 1];
     }
-    cell_slope<ALB>(g, a, w, c, sl);
+    cell_slope<ALB, FAST>(g, a, w, c, sl);
 #pragma unroll
     for (int v = 0; v < 7; ++v) s.sf.s.x[v][ty * (DT + 2) + tx + 1] = sl[v];
 #pragma unroll
@@ -302,7 +331,7 @@ __device__ __forceinline__ void dmarch_slopes(const HydroGeom& g, ColumnLDS& s, 
         a[v] = s.p[v][o - DPW];
         c[v] = s.p[v][o + DPW];
     }
-    cell_slope<ALB>(g, a, w, c, sl);
+    cell_slope<ALB, FAST>(g, a, w, c, sl);
 #pragma unroll
     for (int v = 0; v < 7; ++v) s.sf.s.y[v][(ty + 1) * DT + tx] = sl[v];
     if (ht < 4 * DT) {
@@ -317,7 +346,7 @@ __device__ __forceinline__ void dmarch_slopes(const HydroGeom& g, ColumnLDS& s, 
             b[v] = s.p[v][ho];
             c[v] = s.p[v][ho + st];
         }
-        cell_slope<ALB>(g, a, b, c, sl);
+        cell_slope<ALB, FAST>(g, a, b, c, sl);
         double* dst = yh ? &s.sf.s.y[0][(hy + 1) * DT + hx] : &s.sf.s.x[0][hy * (DT + 2) + hx + 1];
 #pragma unroll
         for (int v = 0; v < 7; ++v) dst[v * DNS] = sl[v];
@@ -325,10 +354,11 @@ __device__ __forceinline__ void dmarch_slopes(const HydroGeom& g, ColumnLDS& s, 
 }
 
 // One x face (item < DNF: row y = item / (DT + 1), face f) or y face (face f
-// = j / DT of column x) of plane k: flux in F (zero outside the grid).
-template <int SOLVER, int STAGE>
-__device__ __forceinline__ void dmarch_face(const HydroGeom& g, const ColumnLDS& s, int item, int ox, int oy,
-                                            StepState* st, const GasConsts<double>& gc, double F[7]) {
+// = j / DT of column x) of plane k: flux in F (zero outside the grid).  Returns
+// as slope_flux does.
+template <int SOLVER, bool FAST>
+__device__ __forceinline__ bool dmarch_face(const HydroGeom& g, const ColumnLDS& s, int item, int ox, int oy,
+                                            const GasConsts<double>& gc, double F[7]) {
     const bool yface = item >= DNF;
     int qb, qs, sb, ss;
     bool valid;
@@ -359,9 +389,9 @@ __device__ __forceinline__ void dmarch_face(const HydroGeom& g, const ColumnLDS&
             sbv[v] = sl[v * DNS + sb];
             scv[v] = sl[v * DNS + sb + ss];
         }
-        if (slope_flux<SOLVER, 0>(g, b, sbv, c, scv, gc, F, yface))
-            set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+        return slope_flux<SOLVER, 0, FAST>(g, b, sbv, c, scv, gc, F, yface);
     }
+    return false;
 }
 
 __device__ __forceinline__ void dstore_flux(ColumnLDS& s, int item, const double F[7]) {
@@ -370,15 +400,27 @@ __device__ __forceinline__ void dstore_flux(ColumnLDS& s, int item, const double
     for (int v = 0; v < 7; ++v) dst[v * DNF] = F[v];
 }
 
-template <int SOLVER, bool ALB, int STAGE>
+// FAST: the quick divisions and square roots (Recip, hydro_math.hpp) alone.  A
+// workgroup that meets a cell or face out of their range ends before that
+// plane's update, having noted the plane in `resume`, and the instance with the full ones, launched
+// next, goes on from there (resume null: from the start), leaving at once
+// where nothing is left (4 us).  Us per step: 256^3 6,609 with full divisions
+// only, 5,715 so; 205x173x190 2,943 and 2,527; 128^3 864 and 750.  Both in one
+// kernel, chosen per plane, held 105 spilled registers and were slower than
+// full divisions alone (256^3 7,170).  What bounds the march is the latency of
+// its instruction stream: two waves per SIMD issue about half of the time.
+template <int SOLVER, bool ALB, int STAGE, bool FAST>
 __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) void hydro_march_kernel(
     HydroGeom g, int ntx, int nty, int ntz, int mz, const double* __restrict__ Usrc, const double* Ubase, double* Udst,
-    StepState* st, double dtf_host) {
+    StepState* st, double dtf_host, int* __restrict__ resume) {
     __shared__ ColumnLDS s;
     if (st->halted) return;  // a halted sub-step's pass-through is launch_halted_copy's
     const int tile = tile_of_block(blockIdx.x, ntx * nty * ntz);
-    const int ox = (tile % ntx) * DT, oy = (tile / ntx % nty) * DT, z0 = tile / (ntx * nty) * mz;
+    const int ox = (tile % ntx) * DT, oy = (tile / ntx % nty) * DT;
+    int z0 = tile / (ntx * nty) * mz;
     const int z1 = min(z0 + mz, g.nz);
+    if (!FAST && resume) z0 = resume[blockIdx.x];
+    if (z0 >= z1) return;
     const int tid = threadIdx.x, tx = tid % DT, ty = tid / DT;
     const int gx = ox + tx, gy = oy + ty;
     const bool col = gx < g.nx && gy < g.ny;
@@ -399,28 +441,37 @@ __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
     const auto to_q = [&](int z, const double u[7], double q[7]) {
         const bool zg = (unsigned)z >= (unsigned)g.nz;
         const int zmode = ghost_map(z, g.nz, g.bc_l[2], g.bc_r[2]).mode;
-        q_of_cell<STAGE, false>(g, u, own.mdim ? own.mode : zmode, own.mdim ? own.mdim : (zg ? 3 : 0), q, st,
-                                col && z >= z0 && z < z1);
+        return q_of_cell<STAGE, FAST ? Q_FAST : Q_FULL>(g, u, own.mdim ? own.mode : zmode,
+                                                        own.mdim ? own.mdim : (zg ? 3 : 0), q, st,
+                                                        col && z >= z0 && z < z1);
     };
+    unsigned int ok;  // FAST, bit j: plane k + 2 - j of the own column is in range
 
     double sk[7], w1[7], w2[7], w3[7], fz[7];
     {
         double a[7], w0[7], s0[7], u[7];
         load_u(z0 - 2, u);
-        to_q(z0 - 2, u, a);
+        ok = to_q(z0 - 2, u, a);
         load_u(z0 - 1, u);
-        to_q(z0 - 1, u, w0);
+        ok = 2 * ok + to_q(z0 - 1, u, w0);
         load_u(z0, u);
-        to_q(z0, u, w1);
+        ok = 2 * ok + to_q(z0, u, w1);
         load_u(z0 + 1, u);
-        to_q(z0 + 1, u, w2);
-        cell_slope<ALB>(g, a, w0, w1, s0);
-        cell_slope<ALB>(g, w0, w1, w2, sk);
-        if (col && slope_flux<SOLVER, 2>(g, w0, s0, w1, sk, gc, fz))  // face z0 - 1/2
-            set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+        ok = 2 * ok + to_q(z0 + 1, u, w2);
+        cell_slope<ALB, FAST>(g, a, w0, w1, s0);
+        cell_slope<ALB, FAST>(g, w0, w1, w2, sk);
+        bool bad = false;
+        if (col) bad = slope_flux<SOLVER, 2, FAST>(g, w0, s0, w1, sk, gc, fz);  // face z0 - 1/2
+        if (FAST) ok = bad ? 0 : ok;
+        else if (bad) set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
         load_u(z0 + 2, u);
-        to_q(z0 + 2, u, w3);
+        ok = 2 * ok + to_q(z0 + 2, u, w3);
     }
+    if (FAST) {
+        if (tid < 2) s.stop[tid] = 0;
+        __syncthreads();
+    }
+    int done = z1;
     double inv_t = 0.0;
     for (int k = z0; k < z1; ++k) {
         // The extra work of a plane (halo cells, halo slopes, third faces)
@@ -430,11 +481,17 @@ __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
         if (k + 1 < z1) load_u(k + 3, un);  // used at the plane's end
 #pragma unroll
         for (int v = 0; v < 7; ++v) s.p[v][dslot(tx, ty)] = w1[v];
+        if (FAST) {
+            // planes k - 1 .. k + 2 of the own column, and k - 2 behind its first face
+            const unsigned int need = k == z0 ? 31u : 15u;
+            if ((ok & need) != need) s.stop[k & 1] = 1;
+        }
         if (turn < DHALO) {
             int hx, hy;
             dhalo_pos(turn, hx, hy);
             double hq[7];
-            load_q<STAGE, false>(g, Usrc, ox + hx, oy + hy, k, hq, st, false);
+            const bool in = load_q<STAGE, FAST ? Q_FAST : Q_FULL>(g, Usrc, ox + hx, oy + hy, k, hq, st, false);
+            if (FAST && !in) s.stop[k & 1] = 1;
             const int hs = dslot(hx, hy);
 #pragma unroll
             for (int v = 0; v < 7; ++v) s.p[v][hs] = hq[v];
@@ -443,13 +500,17 @@ __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
         // x and y slopes, then the faces; each flux waits (in LDS or, the
         // last one solved, in registers) until every face has read the
         // slopes, whose LDS the fluxes then take over
-        dmarch_slopes<ALB>(g, s, tid, turn, tx, ty, w1);
+        dmarch_slopes<ALB, FAST>(g, s, tid, turn, tx, ty, w1);
         __syncthreads();
         {
             double F[7];
 #pragma unroll 1
             for (int j = turn < DN3 ? -1 : 0; j < 2; ++j) {
-                dmarch_face<SOLVER, STAGE>(g, s, j < 0 ? 2 * DTHREADS + turn : tid + j * DTHREADS, ox, oy, st, gc, F);
+                const int item = j < 0 ? 2 * DTHREADS + turn : tid + j * DTHREADS;
+                if (dmarch_face<SOLVER, FAST>(g, s, item, ox, oy, gc, F)) {
+                    if (FAST) s.stop[k & 1] = 1;
+                    else set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+                }
                 if (j < 0) {
 #pragma unroll
                     for (int v = 0; v < 7; ++v) s.park2[v][turn] = F[v];
@@ -473,9 +534,11 @@ __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
         double fzn[7] = {0, 0, 0, 0, 0, 0, 0}, u[7];
         {
             double sn[7];
-            cell_slope<ALB>(g, w1, w2, w3, sn);
-            if (col && slope_flux<SOLVER, 2>(g, w1, sk, w2, sn, gc, fzn))
-                set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+            cell_slope<ALB, FAST>(g, w1, w2, w3, sn);
+            if (col && slope_flux<SOLVER, 2, FAST>(g, w1, sk, w2, sn, gc, fzn)) {
+                if (FAST) s.stop[k & 1] = 1;
+                else set_error(st, STAGE == 1 ? ERR_RIEMANN_NAN_1 : ERR_RIEMANN_NAN_2);
+            }
 #pragma unroll
             for (int v = 0; v < 7; ++v) sk[v] = sn[v];
         }
@@ -484,6 +547,7 @@ __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
             for (int v = 0; v < 7; ++v) u[v] = *plane_at(Ubase, g.ncell, v, pl * k, off);
         }
         __syncthreads();
+        double t = 0.0;
         if (col) {
             // += (A/V) F_L, -= (A/V) F_R per dimension (Hydro.cpp:117-137)
             double udot[7];
@@ -499,8 +563,17 @@ __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
                 d -= g.kflux * fzn[v];
                 udot[v] = d;
             }
-            const double t = update_cell<STAGE>(g, u, udot, dtf, st);
-            if (t > inv_t) inv_t = t;
+            if (!update_cell<STAGE, FAST>(g, u, udot, dtf, st, t)) s.stop[k & 1] = 1;
+        }
+        if (FAST) {
+            __syncthreads();
+            if (s.stop[k & 1]) {  // nothing of this plane has left the workgroup
+                done = k;
+                break;
+            }
+        }
+        if (col) {
+            if (STAGE == 2 && t > inv_t) inv_t = t;
 #pragma unroll
             for (int v = 0; v < 7; ++v) *plane_at(Udst, g.ncell, v, pl * k, off) = u[v];
         }
@@ -510,8 +583,9 @@ __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
             w1[v] = w2[v];
             w2[v] = w3[v];
         }
-        if (k + 1 < z1) to_q(k + 3, un, w3);
+        if (k + 1 < z1) ok = 2 * ok + to_q(k + 3, un, w3);
     }
+    if (FAST && tid == 0) resume[blockIdx.x] = done;
     if (STAGE == 2) block_max_to<DTHREADS>(inv_t, &st->maxinv, s.red);
 }
 
@@ -795,14 +869,15 @@ hipError_t launch_fix_solution(const HydroGeom& g, double* U, const double* rate
 
 // Which layout, and how many planes per march workgroup: the smallest of
 // estimates from times measured on this part (one stage, rotated solver, van
-// Albada).  A march workgroup takes about 17 us per plane alone on a CU and
-// 26 us beside a second one, with 1.2 planes' worth of work before its first;
-// up to 512 run at once, and of more the last leave half a workgroup's time
-// unfilled.  The tiles take 12 us and 0.29 ns per cell.  Measured us per step
-// (two stages), tiles / march / the single 8^3-tile kernel before: 16^3 26 /
-// 169 (pieces of 4 planes) / 97; 64^3 159 / 169 / 200; 80^3 307 / 240 / 383;
-// 128^3 1,193 / 864 / 1,487; 205x173x190 4,194 / 2,943 / 5,093; 256^3 9,870 /
-// 6,609 / 12,251 (1,369 -> 2,539 Mcell-updates/s).
+// Albada).  A march workgroup takes about 13.5 us per plane alone on a CU and
+// 20.5 us beside a second one, with 1.2 planes' worth of work before its
+// first; up to 512 run at once, and of more the last leave half a workgroup's
+// time unfilled; the second launch takes 4 us.  The tiles take 12 us and 0.29
+// ns per cell.  Measured us per step (two stages), tiles / march / the single
+// 8^3-tile kernel before: 16^3 25 / 169 (pieces of 4 planes) / 97; 48^3 86 /
+// 118; 64^3 162 / 154 / 200; 72^3 236 / 209; 80^3 312 / 215 / 383; 128^3 1,203
+// / 750 / 1,487; 205x173x190 4,227 / 2,527 / 5,093; 256^3 10,044 / 5,715 /
+// 12,251 (1,369 -> 2,936 Mcell-updates/s).
 struct StagePlan {
     bool march;
     int mz;
@@ -819,14 +894,19 @@ static StagePlan stage_plan(const HydroGeom& g) {
         const int mz = (g.nz + pieces - 1) / pieces;
         if (mz < 2 && g.nz > 1) break;
         const long long blocks = cols * ((g.nz + mz - 1) / mz);
-        const double rounds = blocks <= 256 ? 17.0 / 26.0 : blocks <= 512 ? 1.0 : 0.5 + (double)blocks / 512.0;
-        const double t = 26.0 * rounds * (mz + 1.2);
+        const double rounds = blocks <= 256 ? 13.5 / 20.5 : blocks <= 512 ? 1.0 : 0.5 + (double)blocks / 512.0;
+        const double t = 4.0 + 20.5 * rounds * (mz + 1.2);
         if (t < best) {
             best = t;
             p = StagePlan{true, mz};
         }
     }
     return p;
+}
+
+long long march_blocks(const HydroGeom& g) {
+    const StagePlan p = stage_plan(g);
+    return p.march ? (long long)((g.nx + DT - 1) / DT) * ((g.ny + DT - 1) / DT) * ((g.nz + p.mz - 1) / p.mz) : 0;
 }
 
 template <int SOLVER, bool ALB>
@@ -836,12 +916,16 @@ static hipError_t launch_stage_t(const HydroGeom& g, int stage, const double* Us
     if (plan.march) {
         const int mtx = (g.nx + DT - 1) / DT, mty = (g.ny + DT - 1) / DT, mtz = (g.nz + plan.mz - 1) / plan.mz;
         dim3 grid(mtx * mty * mtz), block(DTHREADS);
-        if (stage == 1)
-            hipLaunchKernelGGL((hydro_march_kernel<SOLVER, ALB, 1>), grid, block, 0, stream, g, mtx, mty, mtz, plan.mz,
-                               Usrc, Ubase, Udst, st, dtf);
-        else
-            hipLaunchKernelGGL((hydro_march_kernel<SOLVER, ALB, 2>), grid, block, 0, stream, g, mtx, mty, mtz, plan.mz,
-                               Usrc, Ubase, Udst, st, dtf);
+        const auto launch = [&](auto fast, int* resume) {
+            if (stage == 1)
+                hipLaunchKernelGGL((hydro_march_kernel<SOLVER, ALB, 1, decltype(fast)::value>), grid, block, 0, stream,
+                                   g, mtx, mty, mtz, plan.mz, Usrc, Ubase, Udst, st, dtf, resume);
+            else
+                hipLaunchKernelGGL((hydro_march_kernel<SOLVER, ALB, 2, decltype(fast)::value>), grid, block, 0, stream,
+                                   g, mtx, mty, mtz, plan.mz, Usrc, Ubase, Udst, st, dtf, resume);
+        };
+        if (g.fast) launch(std::true_type{}, g.resume);
+        launch(std::false_type{}, g.fast ? g.resume : nullptr);
         return hipGetLastError();
     }
     const int ntx = (g.nx + QX - 1) / QX, nty = (g.ny + QY - 1) / QY, ntz = (g.nz + QZ - 1) / QZ;

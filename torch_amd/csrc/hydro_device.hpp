@@ -17,38 +17,41 @@ __device__ __forceinline__ int tile_of_block(int b, int ntiles) {
 
 // fixPrimitives for one cell (Fluid.cpp:138-150).  u_den is U[DEN] of the
 // same cell, used by the reference's temperature floor.
+template <bool FAST = false>
 __device__ __forceinline__ void fix_primitives(const HydroGeom& g, double q[7], double u_den) {
     q[HII] = smax(smin(q[HII], 1.0), 0.0);
     q[ADV] = smax(smin(q[ADV], 1.0), 0.0);
     q[DEN] = smax(q[DEN], g.dfloor);
     q[PRE] = smax(q[PRE], g.pfloor);
     double mu_inv = g.X * (q[HII] + 1.0) + g.mu_c;
-    double temperature = q[PRE] / (mu_inv * g.Rgas * q[DEN]);
+    double temperature = div_r<FAST>(q[PRE], mu_inv * g.Rgas * q[DEN]);
     if (temperature < g.tfloor) q[PRE] = mu_inv * g.Rgas * u_den * g.tfloor;
 }
 
 // fixSolution for one cell (Fluid.cpp:89-136).  Returns true if the
 // reference would throw.
+template <bool FAST = false>
 __device__ __forceinline__ bool fix_solution(const HydroGeom& g, double u[7]) {
     bool bad = !isfinite(u[DEN]) || !isfinite(u[PRE]);
-    double hii = smax(smin(u[HII] / u[DEN], 1.0), 0.0);
-    double adv = smax(smin(u[ADV] / u[DEN], 1.0), 0.0);
+    const Recip<FAST> over(u[DEN]);
+    double hii = smax(smin(over(u[HII]), 1.0), 0.0);
+    double adv = smax(smin(over(u[ADV]), 1.0), 0.0);
     double den = smax(u[DEN], g.dfloor);
     double v[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) v[d] = u[VEL + d] / u[DEN];
+    for (int d = 0; d < 3; ++d) v[d] = over(u[VEL + d]);
     double ke = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) ke += v[d] * v[d];
     ke *= 0.5 * u[DEN];
     double pre = (u[PRE] - ke) * g.gm1;
-    ke *= den / u[DEN];
+    ke *= over(den);
     if (pre < g.pfloor) pre = g.pfloor;
     double mu_inv = g.X * (hii + 1.0) + g.mu_c;
-    double temperature = pre / (mu_inv * g.Rgas * den);
+    double temperature = div_r<FAST>(pre, mu_inv * g.Rgas * den);
     if (temperature < g.tfloor) pre = mu_inv * g.Rgas * den * g.tfloor;
     u[DEN] = den;
-    u[PRE] = pre / g.gm1 + ke;
+    u[PRE] = div_r<FAST>(pre, g.gm1) + ke;
     u[HII] = hii * den;
     u[ADV] = adv * den;
 #pragma unroll
@@ -59,12 +62,46 @@ __device__ __forceinline__ bool fix_solution(const HydroGeom& g, double u[7]) {
     return bad;
 }
 
+// Whether an updated cell's conserved state (before fix_solution) may keep
+// fluxes found by the quick divisions, and whether those of fix_solution,
+// QfromU, fix_primitives and cfl_inv_t on it are in range (Recip,
+// hydro_math.hpp), given constants_in_range.
+__device__ __forceinline__ bool conserved_in_range(const double u[7]) {
+    bool ok = exponent_in<-100, 100>(u[DEN]) & exponent_in<-200, 200>(u[PRE]);
+#pragma unroll
+    for (int v = HII; v < 7; ++v)
+        ok &= (u[v] == 0.0) | (v < VEL ? exponent_in<-400, 200>(u[v]) : exponent_in<-200, 200>(u[v]));
+    return ok;
+}
+
+__host__ __device__ __forceinline__ bool constants_in_range(const HydroGeom& g) {
+    const double lo = 0x1p-64, hi = 0x1p64;  // code units put a gas constant near 1e16, a cell near 1e9
+    return g.Rgas > lo && g.Rgas < hi && g.gm1 > lo && g.gm1 < hi && g.dx > lo && g.dx < hi && g.X >= 0.0 &&
+           g.X <= 1.0 && (g.X > lo || g.mu_c > lo) && g.dfloor < hi &&
+           (g.pfloor == 0.0 || g.pfloor > 0x1p-600) && g.pfloor < 0x1p200;
+}
+
+// Whether a cell's primitives q, found from the conserved u, keep every
+// division and square root of a face solve in range (Recip, hydro_math.hpp).
+// FIXED: fractions below 0 were clamped to 0.
+template <bool FIXED>
+__device__ __forceinline__ bool primitives_in_range(const double q[7], const double u[7]) {
+    bool ok = exponent_in<-100, 100>(q[DEN]) & exponent_in<-100, 100>(q[PRE]) & exponent_in<-100, 100>(u[DEN]);
+#pragma unroll
+    for (int v = HII; v < 7; ++v)
+        ok &= (u[v] == 0.0) | (FIXED && v < VEL && u[v] < 0.0) |
+              (v < VEL ? exponent_in<-400, 100>(q[v]) : exponent_in<-128, 100>(q[v]));
+    return ok;
+}
+
 // CFL term of one cell, Hydro.cpp:80-85 (inv_t == 0 -> 1/dt_max).
+template <bool FAST = false>
 __device__ __forceinline__ double cfl_inv_t(const HydroGeom& g, const double q[7]) {
     double inv_t = 0;
-    double ss = sqrt(g.g * q[PRE] / q[DEN]);
+    double ss = sqrt_z<FAST>(div_r<FAST>(g.g * q[PRE], q[DEN]));
+    const Recip<FAST> over_dx(g.dx);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) inv_t += (fabs(q[VEL + d]) + ss) / g.dx;
+    for (int d = 0; d < 3; ++d) inv_t += over_dx(fabs(q[VEL + d]) + ss);
     if (inv_t == 0) inv_t = 1.0 / g.dt_max;
     return inv_t;
 }
@@ -284,14 +321,26 @@ __device__ __forceinline__ CellSrc cell_source(const HydroGeom& g, int x, int y,
 
 // Q of a stencil cell from its conserved values u: QfromU, in stage 1
 // fixPrimitives and the "hydro before" check, then the ghost velocity rule.
-template <int STAGE, bool MIXED>
-__device__ __forceinline__ void q_of_cell(const HydroGeom& g, const double u[7], int mode, int mdim, double q[7],
+// Returns whether the result keeps a face solve in range (Q_FULL: false).
+// Q_FAST: by the quick divisions alone, right only where it returns true;
+// Q_BOTH: a wave with a lane out of range, if only in a dividend (a quotient
+// that should not be zero), takes the full ones.
+enum QDivisions { Q_FULL, Q_FAST, Q_BOTH };
+template <int STAGE, QDivisions DIV>
+__device__ __forceinline__ bool q_of_cell(const HydroGeom& g, const double u[7], int mode, int mdim, double q[7],
                                           StepState* st, bool check) {
-    if constexpr (MIXED) q_from_u_mixed(q, u, g.gm1);
-    else QfromU(q, u, g.gm1);
+    bool ok = false;
+    if (DIV != Q_FULL) {
+        QfromU<true>(q, u, g.gm1);
+        if (STAGE == 1) fix_primitives<true>(g, q, u[DEN]);
+        ok = g.fast && primitives_in_range<STAGE == 1>(q, u);
+    }
+    if (DIV == Q_FULL || (DIV == Q_BOTH && !__all(ok))) {
+        QfromU(q, u, g.gm1);
+        if (STAGE == 1) fix_primitives(g, q, u[DEN]);
+        ok = ok && primitives_in_range<STAGE == 1>(q, u);
+    }
     if (STAGE == 1) {
-        if constexpr (MIXED) fix_primitives_mixed(g, q, u[DEN]);
-        else fix_primitives(g, q, u[DEN]);
         if (check) {
             // Torch::checkValues("hydro before"), Torch.cpp:420-443
             bool bad = (q[DEN] == 0.0) || (q[PRE] == 0.0);
@@ -301,16 +350,17 @@ __device__ __forceinline__ void q_of_cell(const HydroGeom& g, const double u[7],
         }
     }
     if (mdim) apply_ghost_mode(q, mode, mdim - 1);
+    return ok;
 }
 
-template <int STAGE, bool MIXED>
-__device__ __forceinline__ void load_q(const HydroGeom& g, const double* __restrict__ U, int x, int y, int z,
+template <int STAGE, QDivisions DIV>
+__device__ __forceinline__ bool load_q(const HydroGeom& g, const double* __restrict__ U, int x, int y, int z,
                                        double q[7], StepState* st, bool check) {
     const CellSrc src = cell_source(g, x, y, z);
     double u[7];
 #pragma unroll
     for (int v = 0; v < 7; ++v) u[v] = U[v * g.ncell + src.idx];
-    q_of_cell<STAGE, MIXED>(g, u, src.mode, src.mdim, q, st, check);
+    return q_of_cell<STAGE, DIV>(g, u, src.mode, src.mdim, q, st, check);
 }
 
 // Element (v, c) of a [7][ncell] state array.  A32: the variable's base

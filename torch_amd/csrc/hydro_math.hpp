@@ -37,6 +37,76 @@ struct GasConsts {
     R g, gm1, g2;
 };
 
+// FP64 division and square root by the compiler's own sequences (correctly
+// rounded: reciprocal or reciprocal square root, Newton steps, residual),
+// with (FAST) the parts left out that only out-of-range operands need: the
+// scaling of extreme exponents and the fix-up of zeros, infinities and NaN.
+// In range the remaining operations are the same, so the bits are.  One
+// reciprocal then serves every division by the same quantity (8 in QfromU, 7
+// in the HLL flux): 3 instructions each instead of 11.
+//
+// Zero divisors and overflows of the quick forms give NaN.  In range means:
+// dividends are zero or above 2^-961, divisors and quotients normal, the
+// argument of a square root above 2^-766 (sqrt_z: or zero).  For a face solve
+// the cells of its stencil (primitives_in_range, hydro_device.hpp) imply it:
+// densities and pressures within 2^+-100 and velocities 0 or 2^-128 .. 2^100
+// leave nonzero velocity jumps above 2^-234 and nonzero components of n1 (and
+// norms) above 2^-335, with three exceptions, which the caller sees:
+//  - S_c's dividend, tested in hllc;
+//  - the HLL numerators (and the sums in u_tilde, which d absorbs): one below
+//    2^-961 makes a flux and an update below 2^-700 inexact, which vanishes
+//    in any conserved quantity but one that comes out so small itself, or
+//    that is not finite (a zero divisor): conserved_in_range on the updated
+//    cell is false;
+//  - a NaN in the HII flux, returned as such.
+// The caller then solves again with the full forms.
+template <bool FAST>
+struct Recip {
+    double d, r;
+    __device__ __forceinline__ explicit Recip(double x) : d(x) {
+        if (FAST) {
+            r = __builtin_amdgcn_rcp(x);
+            r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+            r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+        }
+    }
+    // n / d
+    __device__ __forceinline__ double operator()(double n) const {
+        if (!FAST) return n / d;
+        const double q = n * r;
+        return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+    }
+};
+
+template <bool FAST>
+__device__ __forceinline__ double div_r(double n, double d) { return Recip<FAST>(d)(n); }
+
+template <bool FAST>
+__device__ __forceinline__ double sqrt_r(double x) {
+    if (!FAST) return sqrt(x);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+template <bool FAST>
+__device__ __forceinline__ double sqrt_z(double x) {
+    if (!FAST) return sqrt(x);
+    const double s = sqrt_r<true>(x);
+    return x == 0.0 ? x : s;
+}
+
+// |x| within 2^lo .. 2^hi, by its exponent (false for infinities and NaN)
+template <int LO, int HI>
+__device__ __forceinline__ bool exponent_in(double x) {
+    const unsigned int h = (unsigned int)__double2hiint(x) & 0x7fffffffu;
+    return h - ((unsigned int)(1023 + LO) << 20) <= ((unsigned int)(HI - LO) << 20);
+}
+
 template <typename R>
 __device__ __forceinline__ R smin(R a, R b) { return (b < a) ? b : a; }  // std::min
 template <typename R>
@@ -72,6 +142,13 @@ __device__ __forceinline__ R limiter(int lim, R a, R b) {
     }
 }
 
+// van Albada (FAST: a and b in range where the product passes the test)
+template <bool FAST>
+__device__ __forceinline__ double albada(double a, double b) {
+    const double s = div_r<FAST>(a * b * (a + b), a * a + b * b);
+    return a * b <= 1.0e-30 ? 0.0 : s;
+}
+
 template <typename R>
 __device__ __forceinline__ void UfromQ(R u[7], const R q[7], const GasConsts<R>& c) {
     R ke = R(0);
@@ -87,17 +164,19 @@ __device__ __forceinline__ void UfromQ(R u[7], const R q[7], const GasConsts<R>&
 }
 
 // FP64 primitive recovery (kept in FP64 in both precision modes).
+template <bool FAST = false>
 __device__ __forceinline__ void QfromU(double q[7], const double u[7], double gm1) {
+    const Recip<FAST> over(u[DEN]);
     q[DEN] = u[DEN];
     double ke = 0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        q[VEL + d] = u[VEL + d] / u[DEN];
-        ke += 0.5 * u[VEL + d] * u[VEL + d] / u[DEN];
+        q[VEL + d] = over(u[VEL + d]);
+        ke += over(0.5 * u[VEL + d] * u[VEL + d]);
     }
     q[PRE] = (u[PRE] - ke) * gm1;
-    q[HII] = u[HII] / u[DEN];
-    q[ADV] = u[ADV] / u[DEN];
+    q[HII] = over(u[HII]);
+    q[ADV] = over(u[ADV]);
 }
 
 template <typename R, int DIM>
@@ -116,15 +195,33 @@ __device__ __forceinline__ void FfromQ(R f[7], const R q[7], const GasConsts<R>&
     f[ADV] = q[DEN] * q[VEL + DIM] * q[ADV];
 }
 
-template <typename R, int DIM>
-__device__ __forceinline__ void wave_speeds(R a_l2, R a_r2, const R* Ql, const R* Qr, R& S_l, R& S_r) {
-    R sqrtrho_l = sqrt(Ql[DEN]);
-    R sqrtrho_r = sqrt(Qr[DEN]);
-    R u_tilde = (sqrtrho_l * Ql[VEL + DIM] + sqrtrho_r * Qr[VEL + DIM]) / (sqrtrho_l + sqrtrho_r);
-    R nu2 = R(0.5) * sqrtrho_r * sqrtrho_l / ((sqrtrho_l + sqrtrho_r) * (sqrtrho_l + sqrtrho_r));
-    R dsqrd = (sqrtrho_l * a_l2 + sqrtrho_r * a_r2) / (sqrtrho_l + sqrtrho_r);
+// UfromQ with the division by gamma - 1 through its reciprocal
+template <bool FAST>
+__device__ __forceinline__ void UfromQ(double u[7], const double q[7], const Recip<FAST>& gm1) {
+    double ke = 0.0;
+    u[DEN] = q[DEN];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        u[VEL + d] = q[VEL + d] * q[DEN];
+        ke += 0.5 * q[DEN] * q[VEL + d] * q[VEL + d];
+    }
+    u[PRE] = gm1(q[PRE]) + ke;
+    u[HII] = q[HII] * q[DEN];
+    u[ADV] = q[ADV] * q[DEN];
+}
+
+template <bool FAST, int DIM>
+__device__ __forceinline__ void wave_speeds(double a_l2, double a_r2, const double* Ql, const double* Qr, double& S_l,
+                                            double& S_r) {
+    const double sqrtrho_l = sqrt_r<FAST>(Ql[DEN]);
+    const double sqrtrho_r = sqrt_r<FAST>(Qr[DEN]);
+    const double sum = sqrtrho_l + sqrtrho_r;
+    const Recip<FAST> over(sum);
+    const double u_tilde = over(sqrtrho_l * Ql[VEL + DIM] + sqrtrho_r * Qr[VEL + DIM]);
+    const double nu2 = div_r<FAST>(0.5 * sqrtrho_r * sqrtrho_l, sum * sum);
+    double dsqrd = over(sqrtrho_l * a_l2 + sqrtrho_r * a_r2);
     dsqrd += nu2 * (Qr[VEL + DIM] - Ql[VEL + DIM]) * (Qr[VEL + DIM] - Ql[VEL + DIM]);
-    R d = sqrt(dsqrd);
+    const double d = sqrt_r<FAST>(dsqrd);
     S_l = u_tilde - d;
     S_r = u_tilde + d;
 }
@@ -134,55 +231,60 @@ __device__ __forceinline__ void wave_speeds(R a_l2, R a_r2, const R* Ql, const R
 // selected first and F(Q_side) is the reference's supersonic flux and the
 // Fk of its subsonic star-state flux alike, so every lane runs one FfromQ;
 // the values are those of the reference's branches.
-template <typename R, int DIM>
-__device__ __forceinline__ bool hllc(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c) {
-    R S_l, S_r;
-    wave_speeds<R, DIM>(a_l2, a_r2, Ql, Qr, S_l, S_r);
-    R S_c = Qr[PRE] - Ql[PRE];
+template <bool FAST, int DIM>
+__device__ __forceinline__ bool hllc(double F[7], const double* Ql, const double* Qr, double a_l2, double a_r2,
+                                     const GasConsts<double>& c, const Recip<FAST>& gm1) {
+    double S_l, S_r;
+    wave_speeds<FAST, DIM>(a_l2, a_r2, Ql, Qr, S_l, S_r);
+    double S_c = Qr[PRE] - Ql[PRE];
     S_c += Ql[DEN] * Ql[VEL + DIM] * (S_l - Ql[VEL + DIM]);
     S_c -= Qr[DEN] * Qr[VEL + DIM] * (S_r - Qr[VEL + DIM]);
-    S_c /= (Ql[DEN] * (S_l - Ql[VEL + DIM]) - Qr[DEN] * (S_r - Qr[VEL + DIM]));
-    const bool sup_l = S_l >= R(0);
-    const bool sup_r = !sup_l && S_r <= R(0);
-    const bool left = sup_l || (!sup_r && S_c >= R(0));
-    R Q[7];
+    const bool tiny = FAST && (S_c != 0.0) & (fabs(S_c) < 0x1p-900);
+    S_c = div_r<FAST>(S_c, Ql[DEN] * (S_l - Ql[VEL + DIM]) - Qr[DEN] * (S_r - Qr[VEL + DIM]));
+    const bool sup_l = S_l >= 0.0;
+    const bool sup_r = !sup_l && S_r <= 0.0;
+    const bool left = sup_l || (!sup_r && S_c >= 0.0);
+    double Q[7];
 #pragma unroll
     for (int i = 0; i < 7; ++i) Q[i] = left ? Ql[i] : Qr[i];
-    const R S = left ? S_l : S_r;
-    R U[7], Fk[7], Uc[7];
-    UfromQ<R>(U, Q, c);
-    FfromQ<R, DIM>(Fk, Q, c);
-    R A = Q[DEN] * (S - Q[VEL + DIM]) / (S - S_c);
+    const double S = left ? S_l : S_r;
+    double U[7], Fk[7], Uc[7];
+    UfromQ<FAST>(U, Q, gm1);
+    FfromQ<double, DIM>(Fk, Q, c);
+    const double A = div_r<FAST>(Q[DEN] * (S - Q[VEL + DIM]), S - S_c);
     Uc[DEN] = A;
 #pragma unroll
     for (int id = 0; id < 3; ++id) Uc[VEL + id] = A * Q[VEL + id];
     Uc[VEL + DIM] = A * S_c;
-    Uc[PRE] = A * ((U[PRE] / Q[DEN]) + (S_c - Q[VEL + DIM]) * (S_c + Q[PRE] / (Q[DEN] * (S - Q[VEL + DIM]))));
+    Uc[PRE] = A * (div_r<FAST>(U[PRE], Q[DEN]) +
+                   (S_c - Q[VEL + DIM]) * (S_c + div_r<FAST>(Q[PRE], Q[DEN] * (S - Q[VEL + DIM]))));
     Uc[HII] = A * Q[HII];
     Uc[ADV] = A * Q[ADV];
     const bool sub = !sup_l && !sup_r;
 #pragma unroll
     for (int i = 0; i < 7; ++i) F[i] = sub ? Fk[i] + S * (Uc[i] - U[i]) : Fk[i];
-    return F[HII] != F[HII];
+    return (F[HII] != F[HII]) | (sub & tiny);
 }
 
 // HartenLaxLeerSolver::solve, branch-free (both one-sided fluxes are needed
 // by the subsonic case; the three candidates are selected per lane).
-template <typename R, int DIM>
-__device__ __forceinline__ bool hll(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c) {
-    R S_l, S_r;
-    wave_speeds<R, DIM>(a_l2, a_r2, Ql, Qr, S_l, S_r);
-    R U_l[7], U_r[7], F_l[7], F_r[7];
-    UfromQ<R>(U_l, Ql, c);
-    UfromQ<R>(U_r, Qr, c);
-    FfromQ<R, DIM>(F_l, Ql, c);
-    FfromQ<R, DIM>(F_r, Qr, c);
-    const bool right = S_r <= R(0);
-    const bool left = !right && S_l >= R(0);
+template <bool FAST, int DIM>
+__device__ __forceinline__ bool hll(double F[7], const double* Ql, const double* Qr, double a_l2, double a_r2,
+                                    const GasConsts<double>& c, const Recip<FAST>& gm1) {
+    double S_l, S_r;
+    wave_speeds<FAST, DIM>(a_l2, a_r2, Ql, Qr, S_l, S_r);
+    double U_l[7], U_r[7], F_l[7], F_r[7];
+    UfromQ<FAST>(U_l, Ql, gm1);
+    UfromQ<FAST>(U_r, Qr, gm1);
+    FfromQ<double, DIM>(F_l, Ql, c);
+    FfromQ<double, DIM>(F_r, Qr, c);
+    const bool right = S_r <= 0.0;
+    const bool left = !right && S_l >= 0.0;
+    const Recip<FAST> over(S_r - S_l);
 #pragma unroll
     for (int i = 0; i < 7; ++i) {
-        const R hl = (S_r * F_l[i] - S_l * F_r[i] + S_l * S_r * (U_r[i] - U_l[i])) / (S_r - S_l);
-        F[i] = right ? F_r[i] : (left ? F_l[i] : hl);
+        const double h = over(S_r * F_l[i] - S_l * F_r[i] + S_l * S_r * (U_r[i] - U_l[i]));
+        F[i] = right ? F_r[i] : (left ? F_l[i] : h);
     }
     return F[HII] != F[HII];
 }
@@ -196,24 +298,23 @@ __device__ __forceinline__ bool hll(R F[7], const R* Ql, const R* Qr, R a_l2, R 
 // zero).  The map back (d onto n) has the same k and products and the
 // opposite transverse signs.  Four 3 x 3 matrix evaluations with two divides
 // and two square roots more per face went with this.
-template <typename R>
 struct AxisRotation {
-    R a, b;                    // transverse components of n
-    R nn, aa, bb, ab, ba;      // M_NN, M_AA, M_BB, M_AB, M_BA
+    double a, b;                    // transverse components of n
+    double nn, aa, bb, ab, ba;      // M_NN, M_AA, M_BB, M_AB, M_BA
 };
 
 // n: normal component and transverse ones; s: |(a, b)|
-template <typename R>
-__device__ __forceinline__ AxisRotation<R> axis_rotation(R n, R a, R b, R s) {
-    AxisRotation<R> m;
-    const R k = (R(1.0) - n) / (s * s);
-    const R ka = k * a, kb = k * b;
-    const R x = ka * a, y = kb * b;
+template <bool FAST>
+__device__ __forceinline__ AxisRotation axis_rotation(double n, double a, double b, double s) {
+    AxisRotation m;
+    const double k = div_r<FAST>(1.0 - n, s * s);
+    const double ka = k * a, kb = k * b;
+    const double x = ka * a, y = kb * b;
     m.a = a;
     m.b = b;
-    m.nn = R(1.0) - (x + y);
-    m.aa = R(1.0) - x;
-    m.bb = R(1.0) - y;
+    m.nn = 1.0 - (x + y);
+    m.aa = 1.0 - x;
+    m.bb = 1.0 - y;
     m.ab = -(ka * b);
     m.ba = -(kb * a);
     return m;
@@ -221,11 +322,11 @@ __device__ __forceinline__ AxisRotation<R> axis_rotation(R n, R a, R b, R s) {
 
 // v <- M v (BACK: the map back); each row is summed in component order, as
 // Eigen's product does.
-template <typename R, int DIM, bool BACK>
-__device__ __forceinline__ void rotate(const AxisRotation<R>& m, R* v) {
+template <int DIM, bool BACK>
+__device__ __forceinline__ void rotate(const AxisRotation& m, double* v) {
     constexpr int A = VEL + (DIM == 0 ? 1 : 0), B = VEL + (DIM == 2 ? 1 : 2), N = VEL + DIM;
-    const R a = BACK ? -m.a : m.a, b = BACK ? -m.b : m.b;
-    const R n = v[N], va = v[A], vb = v[B];
+    const double a = BACK ? -m.a : m.a, b = BACK ? -m.b : m.b;
+    const double n = v[N], va = v[A], vb = v[B];
     if (DIM == 2) {
         v[N] = (a * va + b * vb) + m.nn * n;
         v[A] = (m.aa * va + m.ab * vb) - a * n;
@@ -241,89 +342,91 @@ __device__ __forceinline__ void rotate(const AxisRotation<R>& m, R* v) {
 // 0 only): a y face whose x and y velocity components the caller has
 // exchanged; sums of three squares are then taken in the original order (all
 // other sums are over two terms, or commute in x and y).
-template <typename R, int DIM>
-__device__ __forceinline__ bool rotated_hllc(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c,
-                                             bool yface) {
+template <bool FAST, int DIM>
+__device__ __forceinline__ bool rotated_hllc(double F[7], const double* Ql, const double* Qr, double a_l2, double a_r2,
+                                             const GasConsts<double>& c, const Recip<FAST>& gm1, bool yface) {
     static_assert(DIM == 0 || DIM == 2, "y faces are solved as x faces");
     constexpr int A = DIM == 0 ? 1 : 0, B = DIM == 2 ? 1 : 2;
-    const auto norm = [yface](const R v[3]) {
-        const R x = v[0] * v[0], y = v[1] * v[1], z = v[2] * v[2];
-        if (DIM == 2) return sqrt(x + (y + z));
-        return sqrt((yface ? y : x) + ((yface ? x : y) + z));
+    const auto norm = [yface](const double v[3]) {
+        const double x = v[0] * v[0], y = v[1] * v[1], z = v[2] * v[2];
+        if (DIM == 2) return sqrt_z<FAST>(x + (y + z));
+        return sqrt_z<FAST>((yface ? y : x) + ((yface ? x : y) + z));
     };
-    R n1[3] = {Qr[VEL + 0] - Ql[VEL + 0], Qr[VEL + 1] - Ql[VEL + 1], Qr[VEL + 2] - Ql[VEL + 2]};
-    const bool neg = n1[DIM] < R(0);
+    double n1[3] = {Qr[VEL + 0] - Ql[VEL + 0], Qr[VEL + 1] - Ql[VEL + 1], Qr[VEL + 2] - Ql[VEL + 2]};
+    const bool neg = n1[DIM] < 0.0;
 #pragma unroll
     for (int i = 0; i < 3; ++i) n1[i] = neg ? -n1[i] : n1[i];
-    const R l1 = norm(n1);
-    bool pureHLLC = l1 < R(1.0e-6);
+    const double l1 = norm(n1);
+    bool pureHLLC = l1 < 1.0e-6;
     // n1 along the velocity jump; n2 = (n1 x d) x n1 perpendicular to it in
     // the plane of n1 and the axis d
-    const R inv = R(1.0) / l1;
+    const double inv = div_r<FAST>(1.0, l1);
 #pragma unroll
     for (int i = 0; i < 3; ++i) n1[i] *= inv;
-    const R s1sq = n1[A] * n1[A] + n1[B] * n1[B], s1 = sqrt(s1sq);
-    R n2[3];
+    const double s1sq = n1[A] * n1[A] + n1[B] * n1[B], s1 = sqrt_z<FAST>(s1sq);
+    double n2[3];
     n2[DIM] = s1sq;
     n2[A] = -(n1[A] * n1[DIM]);
     n2[B] = -(n1[B] * n1[DIM]);
-    const R l2 = norm(n2);
-    const bool pureHLL = !pureHLLC && (s1 == R(0) || l2 == R(0));
-    const R inv2 = R(1.0) / l2;
+    const double l2 = norm(n2);
+    const bool pureHLL = !pureHLLC && (s1 == 0.0 || l2 == 0.0);
+    const double inv2 = div_r<FAST>(1.0, l2);
 #pragma unroll
     for (int i = 0; i < 3; ++i) n2[i] *= inv2;
-    const R s2sq = n2[A] * n2[A] + n2[B] * n2[B], s2 = sqrt(s2sq);
-    pureHLLC = pureHLLC || (!pureHLL && s2 == R(0));
+    const double s2sq = n2[A] * n2[A] + n2[B] * n2[B], s2 = sqrt_z<FAST>(s2sq);
+    pureHLLC = pureHLLC || (!pureHLL && s2 == 0.0);
     // One HLL and one HLLC solve per face for every lane: on the hybrid path
     // they take the rotated states, on the pure paths the unrotated ones (the
     // reference's single solve; the other result is discarded), so a wave
     // with mixed paths runs the solvers once instead of once per path.
     const bool hybrid = !pureHLLC && !pureHLL;
-    const AxisRotation<R> m1 = axis_rotation<R>(n1[DIM], n1[A], n1[B], s1);
-    R F1[7], F2[7], QlR[7], QrR[7], Qa[7], Qb[7];
+    const AxisRotation m1 = axis_rotation<FAST>(n1[DIM], n1[A], n1[B], s1);
+    double F1[7], F2[7], QlR[7], QrR[7], Qa[7], Qb[7];
 #pragma unroll
     for (int i = 0; i < 7; ++i) { QlR[i] = Ql[i]; QrR[i] = Qr[i]; }
-    rotate<R, DIM, false>(m1, QlR);
-    rotate<R, DIM, false>(m1, QrR);
+    rotate<DIM, false>(m1, QlR);
+    rotate<DIM, false>(m1, QrR);
 #pragma unroll
     for (int i = 0; i < 7; ++i) { Qa[i] = hybrid ? QlR[i] : Ql[i]; Qb[i] = hybrid ? QrR[i] : Qr[i]; }
-    const bool bad1 = hll<R, DIM>(F1, Qa, Qb, a_l2, a_r2, c);
-    rotate<R, DIM, true>(m1, QlR);
-    rotate<R, DIM, true>(m1, QrR);
+    const bool bad1 = hll<FAST, DIM>(F1, Qa, Qb, a_l2, a_r2, c, gm1);
+    rotate<DIM, true>(m1, QlR);
+    rotate<DIM, true>(m1, QrR);
     // A = w1 * (M F1) on the hybrid path (the first term of the reference's
     // w1 F1 + w2 F2), F1 itself on the pure-HLL path
-    const R w1 = fabs(n1[DIM]);
+    const double w1 = fabs(n1[DIM]);
     {
-        R Fr[7];
+        double Fr[7];
 #pragma unroll
         for (int i = 0; i < 7; ++i) Fr[i] = F1[i];
-        rotate<R, DIM, true>(m1, Fr);
+        rotate<DIM, true>(m1, Fr);
 #pragma unroll
         for (int i = 0; i < 7; ++i) F1[i] = hybrid ? w1 * Fr[i] : F1[i];
     }
-    const AxisRotation<R> m2 = axis_rotation<R>(n2[DIM], n2[A], n2[B], s2);
-    rotate<R, DIM, false>(m2, QlR);
-    rotate<R, DIM, false>(m2, QrR);
+    const AxisRotation m2 = axis_rotation<FAST>(n2[DIM], n2[A], n2[B], s2);
+    rotate<DIM, false>(m2, QlR);
+    rotate<DIM, false>(m2, QrR);
 #pragma unroll
     for (int i = 0; i < 7; ++i) { Qa[i] = hybrid ? QlR[i] : Ql[i]; Qb[i] = hybrid ? QrR[i] : Qr[i]; }
-    const bool bad2 = hllc<R, DIM>(F2, Qa, Qb, a_l2, a_r2, c);
-    const R w2 = fabs(n2[DIM]);
-    R Fr[7];
+    const bool bad2 = hllc<FAST, DIM>(F2, Qa, Qb, a_l2, a_r2, c, gm1);
+    const double w2 = fabs(n2[DIM]);
+    double Fr[7];
 #pragma unroll
     for (int i = 0; i < 7; ++i) Fr[i] = F2[i];
-    rotate<R, DIM, true>(m2, Fr);
+    rotate<DIM, true>(m2, Fr);
 #pragma unroll
     for (int i = 0; i < 7; ++i) F[i] = hybrid ? F1[i] + w2 * Fr[i] : (pureHLL ? F1[i] : F2[i]);
     return hybrid ? (bad1 || bad2) : (pureHLL ? bad1 : bad2);
 }
 
-// Face flux along DIM (0 or 2; yface: see rotated_hllc).
-template <int SOLVER, typename R, int DIM>
-__device__ __forceinline__ bool riemann(R F[7], const R* Ql, const R* Qr, R a_l2, R a_r2, const GasConsts<R>& c,
-                                        bool yface) {
-    if constexpr (SOLVER == SOLVER_HLL) return hll<R, DIM>(F, Ql, Qr, a_l2, a_r2, c);
-    else if constexpr (SOLVER == SOLVER_HLLC) return hllc<R, DIM>(F, Ql, Qr, a_l2, a_r2, c);
-    else return rotated_hllc<R, DIM>(F, Ql, Qr, a_l2, a_r2, c, yface);
+// Face flux along DIM (0 or 2; yface: see rotated_hllc).  Returns true if the
+// HII flux is NaN or, FAST, the flux not to be trusted.
+template <int SOLVER, bool FAST, int DIM>
+__device__ __forceinline__ bool riemann(double F[7], const double* Ql, const double* Qr, double a_l2, double a_r2,
+                                        const GasConsts<double>& c, bool yface) {
+    const Recip<FAST> gm1(c.gm1);
+    if constexpr (SOLVER == SOLVER_HLL) return hll<FAST, DIM>(F, Ql, Qr, a_l2, a_r2, c, gm1);
+    else if constexpr (SOLVER == SOLVER_HLLC) return hllc<FAST, DIM>(F, Ql, Qr, a_l2, a_r2, c, gm1);
+    else return rotated_hllc<FAST, DIM>(F, Ql, Qr, a_l2, a_r2, c, gm1, yface);
 }
 
 // ---------------------------------------------------------------------------

@@ -14,6 +14,8 @@ struct HydroGeom {
     int bc_l[3], bc_r[3];
     int limiter;
     int spatial_order;
+    int fast;               // FP64 kernels: the constants allow quick divisions (constants_in_range)
+    int* resume;            // FP64 march: per workgroup, the plane it stopped at [march_blocks]
     int addr64;             // mixed kernel: 64-bit addressing even where 32-bit offsets fit
     long long ncell;        // nx*ny*nz, SoA stride
     double dx;
@@ -181,6 +183,8 @@ int& ctx_counter_step(torchgpu_ctx* c);
 // leaves its HII fraction in Fluid::Q).
 void ctx_set_print_mode(torchgpu_ctx* c, int mode);
 double* ctx_print_buffer(torchgpu_ctx* c);
+// workgroups of the FP64 march on this grid (0: it takes the tiles)
+long long march_blocks(const HydroGeom& g);
 hipError_t launch_cfl(const HydroGeom& g, const double* U, StepState* st, hipStream_t stream);
 // p[0 .. n) = 0 with a kernel (no memset node if a caller captures a graph).
 hipError_t launch_zero(double* p, long long n, hipStream_t stream);
