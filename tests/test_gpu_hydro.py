@@ -239,6 +239,59 @@ def test_mixed_kernel_variants_ragged_grid(gpu, orc, solver, limiter, order):
     assert n == 6 and abs(tg - t) / t < 1e-5
 
 
+# pieces of 2 and more planes with a shorter last one, a single plane, and a
+# box whose pieces are longest; fields smooth along each axis, so no cell is
+# left to chance
+@pytest.mark.parametrize("nz,ny,nx", [(21, 20, 18), (1, 30, 17), (3, 5, 40), (67, 90, 150), (33, 129, 200)])
+@pytest.mark.parametrize("solver", ["RotatedHLLC", "HLLC", "HLL"])
+def test_mixed_pieces_along_z(gpu, orc, nz, ny, nx, solver):
+    """Against the FP64 oracle after 4 steps: FP32 rounding of the fluxes (6
+    faces, 2^-24 each) into 8 stages gives below 1e-5 in relative L1."""
+    z, y, x = np.meshgrid(*[np.arange(n) / n for n in (nz, ny, nx)], indexing="ij")
+    Q = np.empty((7, nz, ny, nx))
+    for v in range(7):
+        Q[v] = np.sin(2 * np.pi * (x + (v % 3) * y + (v % 2 + 1) * z) + v)
+    Q[:2] = np.exp(0.5 * Q[:2])
+    Q[2:4] = 0.5 + 0.3 * Q[2:4]
+    kw = dict(tfloor=1e-12, pfloor=0.1 * 8.314462e7 * 1e-30 * 1e-12, solver=solver, bc=["periodic"] * 6)
+    g = _grid(gpu, Q.shape[1:], precision=gpu.MIXED, **kw)
+    g.set_primitive(Q)
+    p = _oparams(orc, Q.shape[1:], dx=1.0 / nx, **kw)
+    Uo, _, _ = orc.run_hydro(p, _u0(orc, p, Q), 4)
+    g.run(4)
+    g.synchronize()
+    Ug = g.get_conserved()
+    for v in (0, 1, 4, 5, 6):
+        rel = np.abs(Ug[v] - Uo[v]).sum() / np.abs(Uo[v]).sum()
+        assert rel < 1e-5, (v, rel)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_mixed_faces_of_equal_states_moving_apart(gpu, orc, axis):
+    """A velocity jump along the face normal alone takes the hybrid solver's
+    HLL path; with equal states and jump^2 = 8 c^2 the HLLC solve that has no
+    weight there divides zero by zero, which must not reach the flux."""
+    n = 20
+    Q = np.empty((7, n, n, n))
+    Q[0], Q[1], Q[2], Q[3] = 1.0, 1.0, 0.5, 0.25
+    Q[4:] = 0.0
+    c = np.sqrt(5.0 / 3.0)
+    half = np.arange(n) >= n // 2
+    shape = [1, 1, 1]
+    shape[2 - axis] = n
+    for k, scale in enumerate((1.0, 1.0 - 2.0 ** -22, 1.0 + 2.0 ** -22, 1.0 + 2.0 ** -23)):
+        Q[4 + axis] = np.sqrt(2.0) * c * scale * np.where(half, 1.0, -1.0).reshape(shape)
+        kw = dict(gamma=5.0 / 3.0, tfloor=1e-12, pfloor=0.1 * 8.314462e7 * 1e-30 * 1e-12)
+        g = _grid(gpu, Q.shape[1:], precision=gpu.MIXED, **kw)
+        g.set_primitive(Q)
+        p = _oparams(orc, Q.shape[1:], dx=1.0 / n, **kw)
+        Uo, _, _ = orc.run_hydro(p, _u0(orc, p, Q), 1)
+        g.run(1)
+        g.synchronize()
+        np.testing.assert_allclose(g.get_conserved()[0], Uo[0], rtol=1e-5)
+        g.close()
+
+
 def test_mixed_kernel_interior_and_ring_columns(gpu, orc):
     """A 64 x 48 x 40 grid, large enough that the mixed kernel has columns
     whose x and y halos lie inside the grid (their loads skip the ghost

@@ -6,9 +6,10 @@
 // floors and the CFL reduction in FP64.
 //
 // Layout for throughput: a workgroup of 256 threads (4 waves) owns a 16 x 16
-// column of cells and marches it along z through MZ planes.  Each thread
-// keeps the float primitives of its own column at planes k .. k+2 and the
-// limited z slope of plane k in registers, so the z faces need neither LDS
+// column of cells and marches it along z through its planes (march_planes).
+// Each thread keeps the float primitives of its own column at planes k .. k+2
+// and the limited z slope of plane k in registers, so the z faces need neither
+// LDS
 // nor a reloaded z halo, and each z slope serves both z faces of its cell;
 // plane k with its 2-deep x and y halos (256 + 128 cells, float [7][384],
 // one plane per variable) goes through LDS.  Each thread limits the x and y
@@ -18,15 +19,16 @@
 // (consecutive lanes read consecutive x), are solved from the primitives
 // and slopes of their two cells, and their fluxes replace the slopes in LDS
 // once every face has read them.  The thread keeps the z flux of face
-// k+1/2 in registers for the update and as face k-1/2 of the next plane.  Per cell that is 3.125 face
-// solves (plus 1/MZ for the first z face of a column) and 1.5 cell loads, where
+// k+1/2 in registers for the update and as face k-1/2 of the next plane.  Per
+// cell that is 3.125 face solves (plus one for the first z face of a piece) and 1.5 cell loads, where
 // 8^3 tiles with 2-deep halos in all three directions needed 3.375 and 2.5.
 // After the faces each thread updates its cell of plane k in FP64 (fluxes
 // accumulated in the reference's order x, y, z; += F_L, -= F_R), applies
 // fixSolution, writes U, the float primitives of the output for the next
 // stage and (corrector) its CFL term.  34 KB LDS, 128 VGPRs: four waves per
 // SIMD, four workgroups per CU (neither the registers nor the LDS allow a
-// fifth).
+// fifth).  Bound by vector instructions: 1,300 per cell and stage, issued on
+// four cycles of five (256^3, 0.8 ms per stage).
 //
 // FP32 range: the float state is the FP64 state scaled by powers of two,
 // density by 2^kr and pressure by 2^kp with the grid's largest density and
@@ -114,10 +116,7 @@ __device__ __forceinline__ void apply_ghost_mode_f(float q[7], int mode, int dim
 __device__ __forceinline__ unsigned int max_bits_f(float v) { return v > 0.f ? __float_as_uint(v) : 0u; }
 
 
-#ifndef TG_MTX
-#define TG_MTX 16
-#endif
-constexpr int MTX = TG_MTX;               // x extent of a column
+constexpr int MTX = 16;                   // x extent of a column
 constexpr int MTY = 256 / MTX;            // y extent
 constexpr int MCELLS = MTX * MTY;         // 256 cells per plane
 constexpr int PW = MTX + 4, PH = MTY + 4; // plane with its 2-deep halos (corners unused)
@@ -561,17 +560,36 @@ __global__ __launch_bounds__(MTHREADS) __attribute__((amdgpu_waves_per_eu(4))) v
     }
 }
 
-// z planes per workgroup: 16 and 32 measured the same at 512^3, 16 ran 2 %
-// faster at 256^3 (twice the workgroups).
-#ifndef TG_MZ
-#define TG_MZ 16
-#endif
-constexpr int MZ = TG_MZ;
+// Planes per workgroup: the count whose pieces take the least time by an
+// estimate from measurements on this part (rotated solver, van Albada).  With
+// b workgroups per CU resident (at most 4) a plane takes 5 + 1.7 b us, and a
+// workgroup's start 1.6 planes' worth; of more workgroups the last leave
+// about 0.3 of a round unfilled.  Pieces of 2 .. 32 planes.  Us per step (two
+// stages) with 16 planes always, and so: 16^3 217 / 44; 64^3 225 / 71;
+// 96^3 234 / 128; 128^3 284 / 235; 150x97x118 308 / 249; 205x173x190 853 / 851;
+// 256^3 1,690 / 1,684.
+static int march_planes(const HydroGeom& g) {
+    const long long cols = (long long)((g.nx + MTX - 1) / MTX) * ((g.ny + MTY - 1) / MTY);
+    int best_mz = g.nz < 16 ? g.nz : 16;
+    double best = 1.0e300;
+    for (int pieces = (g.nz + 31) / 32; pieces <= 8 * ((g.nz + 31) / 32) + 8; ++pieces) {
+        const int mz = (g.nz + pieces - 1) / pieces;
+        if (mz < 2 && g.nz > 1) break;
+        const double b = (double)(cols * ((g.nz + mz - 1) / mz)) / 256.0;
+        const double t = (mz + 1.6) * (b <= 4.0 ? 5.0 + 1.7 * (b < 1.0 ? 1.0 : b) : 11.8 * (0.3 + 0.25 * b));
+        if (t < best) {
+            best = t;
+            best_mz = mz;
+        }
+    }
+    return best_mz;
+}
 
 template <int SOLVER, bool ALB>
 static hipError_t launch_mixed_t(const HydroGeom& g, int stage, const float* qin, const double* Ubase, double* Udst,
                                  float* qout, int qout_fix, StepState* st, double dtf, int ustar, hipStream_t stream) {
-    const int mtx = (g.nx + MTX - 1) / MTX, mty = (g.ny + MTY - 1) / MTY, mtz = (g.nz + MZ - 1) / MZ;
+    const int mz = march_planes(g);
+    const int mtx = (g.nx + MTX - 1) / MTX, mty = (g.ny + MTY - 1) / MTY, mtz = (g.nz + mz - 1) / mz;
     dim3 grid(mtx * mty * mtz), block(MTHREADS);
     // 32-bit byte offsets within a variable while the FP64 arrays allow it
     // (ncell < 2^29, i.e. up to ~812^3 cells)
@@ -579,17 +597,17 @@ static hipError_t launch_mixed_t(const HydroGeom& g, int stage, const float* qin
     if (stage == 1) {
         if (a32)
             hipLaunchKernelGGL((hydro_stage_mixed_kernel<SOLVER, ALB, 1, true>), grid, block, 0, stream, g, mtx, mty,
-                               mtz, MZ, qin, Ubase, Udst, qout, qout_fix, st, dtf, ustar);
+                               mtz, mz, qin, Ubase, Udst, qout, qout_fix, st, dtf, ustar);
         else
             hipLaunchKernelGGL((hydro_stage_mixed_kernel<SOLVER, ALB, 1, false>), grid, block, 0, stream, g, mtx, mty,
-                               mtz, MZ, qin, Ubase, Udst, qout, qout_fix, st, dtf, ustar);
+                               mtz, mz, qin, Ubase, Udst, qout, qout_fix, st, dtf, ustar);
     } else {
         if (a32)
             hipLaunchKernelGGL((hydro_stage_mixed_kernel<SOLVER, ALB, 2, true>), grid, block, 0, stream, g, mtx, mty,
-                               mtz, MZ, qin, Ubase, Udst, qout, qout_fix, st, dtf, 1);
+                               mtz, mz, qin, Ubase, Udst, qout, qout_fix, st, dtf, 1);
         else
             hipLaunchKernelGGL((hydro_stage_mixed_kernel<SOLVER, ALB, 2, false>), grid, block, 0, stream, g, mtx, mty,
-                               mtz, MZ, qin, Ubase, Udst, qout, qout_fix, st, dtf, 1);
+                               mtz, mz, qin, Ubase, Udst, qout, qout_fix, st, dtf, 1);
     }
     return hipGetLastError();
 }
