@@ -98,6 +98,26 @@ def test_ray_trace_matches_oracle(gpu, shape, star, wind_r):
         np.testing.assert_array_equal(dcolc, dcol_o.ravel(), err_msg=f"replay {rep}")
 
 
+# the sweep's tiles (12 x 12 from the star) and launches (4 shells): star in a
+# corner, one cell off the tiles' and the shells' edges, flat boxes, one row
+@pytest.mark.parametrize("shape,star", [((33, 33, 33), (0, 0, 0)), ((29, 26, 25), (12, 13, 11)),
+                                        ((1, 1, 40), (17, 0, 0)), ((3, 70, 66), (50, 8, 2)), ((9, 8, 7), (6, 0, 8)),
+                                        ((1, 1, 1), (0, 0, 0)), ((50, 2, 50), (25, 1, 24))])
+def test_ray_trace_tile_and_shell_edges(gpu, shape, star):
+    rng = np.random.default_rng(3)
+    c = orc.converter(*SCALES)
+    Q = np.zeros((7,) + shape)
+    Q[0] = 1e-22 * rng.uniform(0.1, 2.0, size=shape) * orc.to_code(c, 1.0, 1, -3, 0)
+    Q[1] = Q[0] * orc.to_code(c, 8.314462e7 * 300.0, 0, 2, -2)
+    Q[3] = 1.0
+    g, cool, dx = _setup(gpu, shape, Q, star, 0, orc.to_code(c, 4.9e48, 0, 0, -1))
+    in9, dcol = cool.grid_inputs(g)
+    geom = orc.star_geometry(shape, star, dx, cool.params.pi)
+    col_o, dcol_o = orc.thermo_ray_trace(shape, star, geom, cool.params.hydrogen_mass, in9[0].reshape(shape))
+    np.testing.assert_array_equal(in9[6], col_o.ravel())
+    np.testing.assert_array_equal(dcol, dcol_o.ravel())
+
+
 def test_star_outside_grid_rejected(gpu):
     g, cool, _ = _setup(gpu, (8, 8, 8), np.ones((7, 8, 8, 8)), (1, 1, 1), 0, 1.0)
     with pytest.raises(gpu.TorchGpuError) as e:

@@ -1012,8 +1012,6 @@ struct torchgpu_cooling {
     double* dcol = nullptr;
     double* col = nullptr;   // COL_DEN of the last ray trace
     long long dcol_cap = 0;
-    double* xface = nullptr;   // the ray trace's x-face buffers
-    long long xface_cap = 0;
     int device = 0;            // the HIP device current at create
 };
 
@@ -1286,7 +1284,7 @@ void torchgpu_cooling_destroy(torchgpu_cooling* c) {
                       (void*)c->feat, (void*)c->y, (void*)c->sdata, (void*)c->in9, (void*)c->out5, (void*)c->gpath, (void*)c->rcache,
                       (void*)c->dtbits,
                       (void*)c->lpt_order, (void*)c->lpt_bucket, (void*)c->lpt_hist, (void*)c->dcol,
-                      (void*)c->col, (void*)c->xface, (void*)c->tmin})
+                      (void*)c->col, (void*)c->tmin})
         if (ptr) (void)hipFree(ptr);
     delete c;
 }
@@ -1546,7 +1544,7 @@ static int grid_src(torchgpu_cooling* c, torchgpu_ctx* ctx, const double* T_min,
         // Thermodynamics::preTimeStepCalculations starts with rayTrace on
         // the fixed primitives (Thermodynamics.cpp:218-220): the density of
         // U with fixPrimitives' floor
-        HIP_OK(tg::launch_thermo_ray_trace(c->star, v.U, v.g->dfloor, c->col, c->dcol, c->xface, c->stream));
+        HIP_OK(tg::launch_thermo_ray_trace(c->star, v.U, v.g->dfloor, c->col, c->dcol, c->stream));
         col_den = c->col;
     }
     gs = tg::GridSrc{};
@@ -1707,7 +1705,7 @@ int torchgpu_fill_heating(torchgpu_ctx* ctx, torchgpu_cooling* c, const double* 
     if (rc) return rc;
     if (c->star.on && !col_den) {
         // fillHeatingArrays starts with rayTrace on Fluid::Q (Thermodynamics.cpp:420-421)
-        HIP_OK(tg::launch_thermo_ray_trace(c->star, Q, -HUGE_VAL, c->col, c->dcol, c->xface, c->stream));
+        HIP_OK(tg::launch_thermo_ray_trace(c->star, Q, -HUGE_VAL, c->col, c->dcol, c->stream));
         col_den = c->col;
     }
     long long nb = (n + 255) / 256;
@@ -1781,15 +1779,6 @@ int torchgpu_cooling_set_star(torchgpu_cooling* c, torchgpu_ctx* ctx, const torc
     s.photon_rate = star->photon_rate;
     s.pi = c->p.pi;
     s.hydrogen_mass = c->p.hydrogen_mass;
-    const long long nx = tg::xface_doubles(s);
-    if (nx > c->xface_cap) {
-        (void)hipStreamSynchronize(c->stream);
-        if (c->xface) (void)hipFree(c->xface);
-        c->xface = nullptr;
-        c->xface_cap = 0;
-        HIP_OK(hipMalloc(&c->xface, nx * sizeof(double)));
-        c->xface_cap = nx;
-    }
     c->star = s;
     return TORCHGPU_OK;
 }

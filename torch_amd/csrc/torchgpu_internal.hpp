@@ -201,13 +201,11 @@ hipError_t launch_step_end(StepState* st, hipStream_t stream);
 // Clock control for Torch::run's checkpoint printing: set the time (and the
 // checkpoint count Checkpointer::update gives for it), resume a paused run.
 hipError_t launch_set_time(StepState* st, double t, hipStream_t stream);
-// The column-density ray trace (Thermodynamics::rayTrace): one launch per
-// shell, den/col/dcol [n] device arrays (den floored at den_floor, as
+// The column-density ray trace (Thermodynamics::rayTrace): one launch per few
+// shells, den/col/dcol [n] device arrays (den floored at den_floor, as
 // fixPrimitives does; -HUGE_VAL: as given); the star's geometry per cell.
 hipError_t launch_thermo_ray_trace(const StarGeom& s, const double* den, double den_floor, double* col, double* dcol,
-                                   double* xface, hipStream_t stream);
-// doubles of the x-face buffers of launch_thermo_ray_trace
-long long xface_doubles(const StarGeom& s);
+                                   hipStream_t stream);
 // The cells of Chebyshev shell k around the star, and the largest k.
 void shell_faces(const StarGeom& s, int k, ShellFaces& f);
 int shell_max(const StarGeom& s);
