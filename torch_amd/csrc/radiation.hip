@@ -388,9 +388,11 @@ __global__ __launch_bounds__(256) void rad_dt_kernel(StarGeom s, RadConsts r, co
     }
 }
 
-// Face-contiguous copies of TAU, DTAU, TAU_A, DTAU_A for the x-fixed faces
-// of the last two shells (see raytrace.hip's coldens_shell_kernel): fields
-// [2 parities][2 sides][4][w * w], y fastest, frame centred on the star.
+// The x-fixed faces of a shell have no contiguous direction in the x-fastest
+// grid, so their cells also keep TAU, DTAU, TAU_A, DTAU_A in face-contiguous
+// copies of the last two shells: fields [2 parities][2 sides][4][w * w], y
+// fastest, frame centred on the star.  Every upstream neighbour of nonzero
+// weight of an x-face cell is on the same side's x-face of the shell before.
 struct RadXFaces {
     double* buf;
     int K, w;

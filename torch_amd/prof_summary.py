@@ -27,7 +27,8 @@ import json
 import re
 import sys
 
-KEEP = re.compile(r"hydro_stage|q_float|q_from_u|u_from_q|step_begin|step_end|cfl_kernel|scale_rotate|state_max")
+KEEP = re.compile(r"hydro_stage|hydro_march|hydro_tile|q_float|q_from_u|u_from_q|step_begin|step_end|cfl_kernel|scale_rotate|state_max")
+STAGE = re.compile(r"hydro_stage|hydro_march|hydro_tile")
 
 
 def short(name: str) -> str:
@@ -127,7 +128,8 @@ def main():
 
     lines = [f"# hydro stage kernels, {a.grid}^3 turbulent box: rocprofv3 summaries", ""]
     lines += [f"Workload: `{a.driver}` ({a.workload}, RotatedHLLC + van Albada, outflow); "
-              "FP64 parity kernel `hydro_stage_kernel<solver, stage>`, mixed-precision kernel "
+              "FP64 parity kernels `hydro_march_kernel<solver, albada, stage, fast>` (large grids; two launches per "
+              "stage) and `hydro_tile_kernel<solver, albada, stage>`, mixed-precision kernel "
               "`hydro_stage_mixed_kernel<solver, albada, stage, a32>` (solver 2 = RotatedHLLC; stage 1 predictor, "
               "2 corrector + CFL; a32: 32-bit byte offsets into the state, grids below 2^29 cells).", ""]
     if a.commands:
@@ -156,7 +158,7 @@ def main():
               "|---|---|---|---|---|---|---|"]
     out = {"grid": a.grid, "calibration": {"fetch_factor": ff, "write_factor": wf}, "kernels": {}}
     for k in sorted(fetch):
-        if "hydro_stage" not in k or k not in write:
+        if not STAGE.search(k) or k not in write:
             continue
         fk, wk = fetch[k]["FETCH_SIZE"], write[k]["WRITE_SIZE"]
         rb, wb = fk * 1024.0 * ff, wk * 1024.0 * wf
@@ -173,7 +175,7 @@ def main():
                   "VALU utilisation |", "|---|---|---|---|---|---|---|"]
         for k in sorted(sq):
             c = sq[k]
-            if "hydro_stage" not in k or "SQ_WAVES" not in c:
+            if not STAGE.search(k) or "SQ_WAVES" not in c:
                 continue
             cyc = c["GRBM_GUI_ACTIVE"] / a.xcds
             util = c["SQ_INSTS_VALU"] / (a.cus * cyc)
@@ -191,7 +193,7 @@ def main():
                   "|---|---|---|---|"]
         for k in sorted(ld):
             c = ld[k]
-            if "hydro_stage" not in k or "SQ_LDS_BANK_CONFLICT" not in c:
+            if not STAGE.search(k) or "SQ_LDS_BANK_CONFLICT" not in c:
                 continue
             cyc = a.cus * c["GRBM_GUI_ACTIVE"] / a.xcds
             act, bc = c["SQ_LDS_IDX_ACTIVE"], c["SQ_LDS_BANK_CONFLICT"]
