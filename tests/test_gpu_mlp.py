@@ -71,6 +71,62 @@ def test_mlp_kernels_at_tile_edges(gpu, B):
             assert err < 2.0 ** -8, (name, err)
 
 
+def test_mlp_training_silu_is_exact_to_rounding(gpu):
+    """Bias gradients of the last hidden layer with every other factor exact:
+    one cell, W1..W4 zero, so z = b4; W5 one for output 0 and zero for the
+    others, target 1, so the gradient into the layer is bf16(y - 1) = -1 (y is
+    -2.7e-4, less than half a bfloat16 step) and the result is -silu'(z).  With
+    u = 2^-24, half an ulp at most: exp 2 u, the sum 1 + e^-z and the division
+    u each, 1 - s and its product with z u each of what is 14/13 or less of the
+    next sum, that sum and the last product u each: 8.2 u."""
+    import torch
+
+    from torch_amd import surrogate as sg
+
+    z = np.linspace(-20.0, -14.0, 128).astype(np.float32)
+    W = np.zeros(sg.NW, np.float32)
+    W[-3 * 128:-2 * 128] = 1.0
+    b = np.zeros(sg.NB, np.float32)
+    b[3 * 128:4 * 128] = z
+    m = sg.MLP(max_batch=1)
+    m.set_params(W, b)
+    fd = torch.zeros((1, 8), dtype=torch.float32, device="cuda")
+    td = torch.tensor([[1.0, 0.0, 0.0]], dtype=torch.float32, device="cuda")
+    _, _, gb = m.loss_grad(fd, td)
+    ref = -omlp.dsilu(z.astype(np.float64))
+    err = np.abs(gb[3 * 128:4 * 128] / ref - 1.0).max()
+    assert err < 9 * 2.0 ** -24, err
+
+
+# The order of every sum of a training step is fixed, so its bits are: of
+# loss_grad and of three Adam steps (weight decay, error head on and off) on
+# one cell, ragged batches and more tiles than waves in flight.
+@pytest.mark.parametrize("B,digest", [(1, "06ec0ff1f4d23452"), (33, "60ac0bd48f919fd9"), (300, "882d32546a481b31"), (4096 + 31, "56fa934960cc5730"),
+                                      (32768 + 129, "4e8d027bee434fc8")])
+def test_mlp_training_bits(gpu, B, digest):
+    import hashlib
+
+    import torch
+
+    from torch_amd import surrogate as sg
+
+    rng = np.random.Generator(np.random.PCG64(B))
+    f = np.zeros((B, 8), np.float32)
+    f[:, :6] = rng.normal(0, 1, (B, 6))
+    t = rng.normal(0, 1, (B, 3)).astype(np.float32)
+    fd, td = torch.from_numpy(f).cuda(), torch.from_numpy(t).cuda()
+    W, b = sg.init_params(3)
+    m = sg.MLP(max_batch=B)
+    m.set_params(W, rng.normal(0, 0.1, b.shape).astype(np.float32))
+    _, gW, gb = m.loss_grad(fd, td, weights=(1, 0.5, 0.25), err_head=True)
+    for i in range(3):
+        m.train_step(fd, td, 1e-3, weights=(1, 1, 0.05), err_head=bool(i & 1), weight_decay=1e-4)
+    h = hashlib.sha256()
+    for a in (gW, gb, *m.get_params()):
+        h.update(a.tobytes())
+    assert h.hexdigest()[:16] == digest
+
+
 def test_mlp_fused_inference_matches_reference(gpu):
     m, p, f, t, fd, td = _setup(seed=3, B=1000)  # ragged: not a multiple of 32
     y = m.forward(fd).cpu().numpy()

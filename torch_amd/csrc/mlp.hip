@@ -9,29 +9,33 @@
 // features along MFMA rows, cells along columns), so that the FP32
 // accumulator of one layer, after SiLU and rounding, is directly the B
 // operand of the next and a wave carries its cells through every layer in
-// registers, forwards and backwards, with no exchange between waves.  The
-// k-order this implies inside each 32-wide K step (kperm) is built into the
-// weight fragments, which are kept packed in the order the lanes read them:
-// one conflict-free 16-byte LDS read (or one contiguous 1 KB L2 read per wave)
-// per fragment.  Row-major weights in LDS, whose 256-byte rows put the 16
-// lanes of a row group on the same banks, ran the 2^20-cell inference in
-// 258 us (408 TFLOP/s); the fragments, staged by 16-byte copies, run it in 157
-// us (669 TFLOP/s).
+// registers, forwards and backwards, with no exchange between waves.  Inside a
+// 32-wide K step that takes a permutation: of the columns (kslot) in the
+// inference fragments, of the rows (row_feature) in the training ones, whose
+// products so add their terms in the features' order.  The fragments are kept
+// packed in the order the lanes read them: one conflict-free 16-byte LDS read
+// (or one contiguous 1 KB L2 read per wave) per fragment.  Row-major weights
+// in LDS, whose 256-byte rows put the 16 lanes of a row group on the same
+// banks, ran the 2^20-cell inference in 258 us (408 TFLOP/s); the fragments,
+// staged by 16-byte copies, run it in 157 us (669 TFLOP/s).
 //
 // Training of a batch is three launches:
 //   mlp_train_kernel    forward, loss and data gradients, 16 cells per wave,
 //                       SiLU derivatives in registers; writes the activations
-//                       and their gradients in bfloat16, cells contiguous
+//                       and their gradients in bfloat16, cells contiguous, and
+//                       the bias-gradient terms of its cells
 //   mlp_wgrad_kernel    weight gradients dZ^T H as split-K products whose
 //                       operands are read as fragments straight from those
-//                       arrays (cells are the contraction index), no LDS
+//                       arrays (cells are the contraction index), no LDS; loss
+//                       and output-bias gradients of 256 cells
 //   reduce_adam_kernel  fixed-order sums of the partials, Adam, and the new
 //                       weights into their fragments
-// A batch of 65,536 took 2,750 us per step as one tiled GEMM launch per
+// A batch of 65,536 took 2,700 us per step as one tiled GEMM launch per
 // product with scalar operand loads, FP32 pre-activations in memory and a
-// serial sum of up to 1,024 bias partials per thread; it takes 161 us (87 in
-// the fused kernel, 33 in the weight gradients, 13 in the sums and Adam).  All
-// sums run in a fixed order: training is deterministic.
+// serial sum of up to 1,024 bias partials per thread; it takes 156 us, the same
+// bits: every sum runs in that form's order.  (With the hardware exponential
+// and reciprocal in the SiLU, and sums in whatever order suits the launches, it
+// took 126 us, activations up to 1e-6 off and weights 5e-4 after four steps.)
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -62,46 +66,57 @@ __device__ __forceinline__ unsigned int pack_bf16(float lo, float hi) {
 }
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
-// Logistic function from the hardware base-2 exponential and reciprocal
-// (about 1 ulp each): the activations that follow from it keep 8 significant
-// bits, and the gradients are summed from bfloat16 operands.
+// Logistic function of the inference kernel, from the hardware base-2
+// exponential and reciprocal.  The product below is rounded before the
+// exponential, so the relative error grows with |z|: 1e-7 near 0, 1e-6 at z =
+// -20.  The activations that follow from it keep 8 significant bits.
 __device__ __forceinline__ float sigmoid_f(float z) {
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
 }
 
-// k-permutation of one 32-wide K step: lane group q holds, after a layer's
-// 16x16 D tiles 2s and 2s+1, the features 32s + 4q + e (e < 4) and
+// k-permutation of one 32-wide K step (inference): lane group q holds, after a
+// layer's 16x16 D tiles 2s and 2s+1, the features 32s + 4q + e (e < 4) and
 // 32s + 16 + 4q + (e - 4) (e >= 4) as its 8 B-operand entries.  kslot is its
 // inverse: the place 8 q + e of position k.
 __device__ __forceinline__ int kslot(int k) { return k < 16 ? 8 * (k >> 2) + (k & 3) : 8 * ((k - 16) >> 2) + 4 + (k & 3); }
 
-// Place of element (row m, column k) of a fragment grid with `nks` K steps
-// per row tile, permuted columns.
-__device__ __forceinline__ int frag_at(int base, int nks, int m, int k) {
-    const int s = kslot(k & 31);
-    return (base + (m >> 4) * nks + (k >> 5)) * MLP_FRAG + ((s >> 3) * 16 + (m & 15)) * 8 + (s & 7);
+// Row permutation of a layer's 16-row tiles (training): row 4q + e of tile
+// 2s + h is feature 32s + 8q + 4h + e, which leaves the 8 features 32s + 8q ..
+// of the next K step with lane group q, in their order.
+__device__ __forceinline__ int row_feature(int t, int q) { return 32 * (t >> 1) + 8 * q + 4 * (t & 1); }  // e = 0
+__device__ __forceinline__ int feature_tile(int f) { return 2 * (f >> 5) + ((f >> 2) & 1); }
+__device__ __forceinline__ int feature_row(int f) { return 4 * ((f >> 3) & 3) + (f & 3); }
+
+// Place of row `row` of tile t and slot s (0 .. 31) of K step ks in a fragment
+// grid with `nks` K steps per tile.
+__device__ __forceinline__ int frag_at(int base, int nks, int t, int row, int ks, int s) {
+    return (base + t * nks + ks) * MLP_FRAG + ((s >> 3) * 16 + row) * 8 + (s & 7);
 }
 
-// Writes weight i of the master layout into its forward and backward
-// fragments (the padding stays as it was set at creation: zero).
+// Writes weight i of the master layout into its fragments (the padding stays
+// as it was set at creation: zero).
 __device__ __forceinline__ void pack_weight(int i, float w, bf16_t* __restrict__ packed) {
     const bf16_t v = to_bf16(w);
-    bf16_t* bwd = packed + MLP_NFF * MLP_FRAG;
-    if (i < MLP_H * MLP_IN) {  // W1: lane group 0 carries the 8 features, unpermuted
+    bf16_t* fwd = packed + MLP_NFF * MLP_FRAG;
+    bf16_t* bwd = fwd + MLP_NFF * MLP_FRAG;
+    if (i < MLP_H * MLP_IN) {  // W1: lane group 0 carries the 8 features
         const int o = i / MLP_IN, c = i % MLP_IN;
-        packed[(o >> 4) * MLP_FRAG + (o & 15) * 8 + c] = v;
+        packed[frag_at(0, 1, o >> 4, o & 15, 0, c)] = v;
+        fwd[frag_at(0, 1, feature_tile(o), feature_row(o), 0, c)] = v;
         return;
     }
     i -= MLP_H * MLP_IN;
     const int l = i / (MLP_H * MLP_H);
+    const int c = i % MLP_H, o = l < 3 ? (i / MLP_H) % MLP_H : (i - 3 * MLP_H * MLP_H) / MLP_H;
     if (l < 3) {
-        const int o = (i / MLP_H) % MLP_H, c = i % MLP_H;
-        packed[frag_at(8 + l * 32, 4, o, c)] = v;
-        bwd[frag_at(8 + l * 32, 4, c, o)] = v;
+        const int base = 8 + l * 32;
+        packed[frag_at(base, 4, o >> 4, o & 15, c >> 5, kslot(c & 31))] = v;
+        fwd[frag_at(base, 4, feature_tile(o), feature_row(o), c >> 5, c & 31)] = v;
+        bwd[frag_at(base, 4, feature_tile(c), feature_row(c), o >> 5, o & 31)] = v;
     } else {
-        const int o = (i - 3 * MLP_H * MLP_H) / MLP_H, c = i % MLP_H;
-        packed[frag_at(8 + 96, 4, o, c)] = v;
-        bwd[frag_at(0, 1, c, o)] = v;
+        packed[frag_at(8 + 96, 4, 0, o, c >> 5, kslot(c & 31))] = v;
+        fwd[frag_at(8 + 96, 4, 0, o, c >> 5, c & 31)] = v;
+        bwd[frag_at(0, 1, feature_tile(c), feature_row(c), 0, o)] = v;
     }
 }
 
@@ -141,8 +156,8 @@ __device__ __forceinline__ u32x4 load_features(const float* __restrict__ feat, l
 }
 
 struct NetLDS {
-    u32x4 w[MLP_NFF * 64];   // forward fragments, 108 KB
     float b[4 * MLP_H + 16]; // biases, the output layer's padded with zeros
+    u32x4 w[MLP_NFF * 64];   // forward fragments, 108 KB
 };
 
 __device__ __forceinline__ void stage_net(NetLDS& s, const bf16_t* __restrict__ packed, const float* __restrict__ bias,
@@ -237,93 +252,116 @@ __device__ __forceinline__ float dpp_f(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
 }
 
-// Sums of 16 values over the 16 lanes of a row: lane r returns the sum of
-// v[r].  Each step halves the values a lane carries: it keeps those of its
-// own side of a lane bit and adds its partner's, through DPP (row mirror,
-// half mirror, quad swaps).  15 steps and no branch; a rotation sum and a
-// guarded LDS add per value made 137 branches per 16 cells, which kept the
-// scheduler from overlapping the fragment loads.
-__device__ __forceinline__ float row_sums(float (&v)[16], int r) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = ((r & 8) ? v[i + 8] : v[i]) + dpp_f<0x140>((r & 8) ? v[i] : v[i + 8]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = ((r & 4) ? v[i + 4] : v[i]) + dpp_f<0x141>((r & 4) ? v[i] : v[i + 4]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) v[i] = ((r & 2) ? v[i + 2] : v[i]) + dpp_f<0x4E>((r & 2) ? v[i] : v[i + 2]);
-    return ((r & 1) ? v[1] : v[0]) + dpp_f<0xB1>((r & 1) ? v[0] : v[1]);
+// One value of a tile, in the sums below: lane j of each quad, to all four.
+template <int J>
+__device__ __forceinline__ float quad_f(float x) { return dpp_f<0x55 * J>(x); }
+
+// Bias-gradient terms of two features over a tile's 16 cells, in a fixed
+// order: lanes 0-7 of a row return a's sum, lanes 8-15 b's.  Lanes 0-7 of a
+// tile are eight consecutive cells and lanes 8-15 the eight 16 further on
+// (tile_cell); a quad adds its four cells and the four 16 further on one
+// after another, then the two quads are added.  14 steps for two features,
+// without a branch.
+__device__ __forceinline__ float tile_sums(float a, float b) {
+    const int ai = __float_as_int(a), bi = __float_as_int(b);
+    const float x = __int_as_float(__builtin_amdgcn_update_dpp(ai, bi, 0x128, 0xf, 0xc, false));  // cells 0-7 of either
+    const float y = __int_as_float(__builtin_amdgcn_update_dpp(bi, ai, 0x128, 0xf, 0x3, false));  // and 8-15
+    float s = quad_f<0>(x);
+    s += quad_f<1>(x);
+    s += quad_f<2>(x);
+    s += quad_f<3>(x);
+    s += quad_f<0>(y);
+    s += quad_f<1>(y);
+    s += quad_f<2>(y);
+    s += quad_f<3>(y);
+    return s + dpp_f<0x141>(s);
 }
 
-// Stores the two bfloat16 pairs (features f, f+1 and f+2, f+3 of the lane's
-// cell r) of a 16-cell tile as cells-contiguous rows dst[feature][32]: lanes
-// 2j and 2j+1 exchange, so that each writes two cells of one feature of each
-// pair (4-byte stores, 32 contiguous bytes per feature).
-__device__ __forceinline__ void store_rows(bf16_t* __restrict__ dst, int f, int r, unsigned int p0, unsigned int p1) {
-    const unsigned int sel = (r & 1) ? 0x03020706u : 0x05040100u;
+// The cell, within a block of 32, of lane r of the block's tile `half`.
+__device__ __forceinline__ int tile_cell(int half, int r) { return 8 * half + (r & 7) + 16 * (r >> 3); }
+
+// Stores the two bfloat16 pairs (features f .. f + 3 of one cell) of tile t as
+// cells-contiguous rows dst[feature][32]: lanes 2j and 2j+1 exchange, so that
+// each writes two cells of one feature of each pair.  at: the lane's place,
+// row_place(), in units of two cells.
+__device__ __forceinline__ unsigned int row_place(int q, int c) { return (unsigned int)((8 * q + (c & 1)) * 16 + (c >> 1)); }
+__device__ __forceinline__ void store_rows(bf16_t* __restrict__ dst, int t, unsigned int at, int lane, unsigned int p0,
+                                           unsigned int p1) {
+    const unsigned int sel = (lane & 1) ? 0x03020706u : 0x05040100u;
     const unsigned int n0 = __builtin_amdgcn_update_dpp(0, p0, 0xB1, 0xf, 0xf, true);
     const unsigned int n1 = __builtin_amdgcn_update_dpp(0, p1, 0xB1, 0xf, 0xf, true);
-    unsigned int* d = reinterpret_cast<unsigned int*>(dst);
-    const unsigned int o = (unsigned int)((f + (r & 1)) * 16 + (r >> 1));
-    d[o] = __builtin_amdgcn_perm(n0, p0, sel);
-    d[o + 32] = __builtin_amdgcn_perm(n1, p1, sel);  // two features on: 64 bf16
+    unsigned int* d = reinterpret_cast<unsigned int*>(dst) + row_feature(t, 0) * 16;
+    d[at] = __builtin_amdgcn_perm(n0, p0, sel);
+    d[at + 32] = __builtin_amdgcn_perm(n1, p1, sel);  // two features on: 64 bf16
 }
 
 constexpr int TRAIN_THREADS = 512, TRAIN_WAVES = TRAIN_THREADS / 64;
 
-struct TrainLDS {
-    NetLDS net;
-    float gb[TRAIN_WAVES][4 * MLP_H + 4];  // bias gradients of each wave's cells
-    float loss[TRAIN_WAVES];
-};
-
 // Data gradient through SiLU of one layer: dz = g ds, its sums over the
-// cells into gb (lane (q, r) keeps those of the features 64 i + 16 (r / 4) +
-// 4 q + r % 4), bfloat16 rows for the weight gradients, and the next B
-// operand.
+// tile's cells into sums[128], bfloat16 rows for the weight gradients, and the
+// next B operand.
 template <int NKS>
 __device__ __forceinline__ void train_backward(const u32x4* __restrict__ w, const u32x4 (&g)[NKS][1],
                                                const float (&ds)[32], u32x4 (&out)[4][1], bf16_t* __restrict__ rows,
-                                               float (&gb)[2], int lane) {
+                                               float* __restrict__ sums, unsigned int at, int lane) {
     const int q = lane >> 4, r = lane & 15;
+    float keep[2] = {0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        float d[16];
+    for (int s = 0; s < 4; ++s) {
+        float d[2][4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int t = 4 * i + j;
+        for (int h = 0; h < 2; ++h) {
+            const int t = 2 * s + h;
             f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
             row_tile<NKS, 1>(w, t, lane, g, acc);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) d[4 * j + e] = acc[0][e] * ds[t * 4 + e];
-            const unsigned int p0 = pack_bf16(d[4 * j], d[4 * j + 1]), p1 = pack_bf16(d[4 * j + 2], d[4 * j + 3]);
-            out[t >> 1][0][(t & 1) * 2] = p0;
-            out[t >> 1][0][(t & 1) * 2 + 1] = p1;
-            store_rows(rows, t * 16 + 4 * q, r, p0, p1);
+            for (int e = 0; e < 4; ++e) d[h][e] = acc[0][e] * ds[t * 4 + e];
+            const unsigned int p0 = pack_bf16(d[h][0], d[h][1]), p1 = pack_bf16(d[h][2], d[h][3]);
+            out[s][0][2 * h] = p0;
+            out[s][0][2 * h + 1] = p1;
+            store_rows(rows, t, at, lane, p0, p1);
         }
-        gb[i] += row_sums(d, r);
+        // lane r keeps the sums of tile 2s + r / 8, s = 2 i + (r / 4) % 2,
+        // element r % 4 in keep[i]
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = tile_sums(d[0][e], d[1][e]);
+            keep[s >> 1] = (r & 7) == (s & 1) * 4 + e ? v : keep[s >> 1];
+        }
     }
+    const int f = 32 * ((r >> 2) & 1) + 8 * q + 4 * (r >> 3) + (r & 3);
+    sums[f] = keep[0];
+    sums[64 + f] = keep[1];
 }
 
 // Forward layer keeping ds = silu'(z) in registers (FP32) and writing the
-// activations' rows.
+// activations' rows.  SiLU and its derivative from expf and exact divisions:
+// the hardware exponential and reciprocal of the inference kernel are up to
+// 1e-6 off at z = -20, and the gradients see it.
 template <int NKS>
 __device__ __forceinline__ void train_forward(const u32x4* w, const float* b, const u32x4 (&x)[NKS][1], float (&ds)[32],
-                                              u32x4 (&h)[4][1], bf16_t* __restrict__ rows, int lane) {
-    const int q = lane >> 4, r = lane & 15;
+                                              u32x4 (&h)[4][1], bf16_t* __restrict__ rows, unsigned int at,
+                                              int lane) {
+    const int q = lane >> 4;
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-        f32x4 acc[1] = {*reinterpret_cast<const f32x4*>(b + t * 16 + 4 * q)};
+        f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
         row_tile<NKS, 1>(w, t, lane, x, acc);
+        const f32x4 bv = *reinterpret_cast<const f32x4*>(b + row_feature(t, 0) + 8 * q);
         float a[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float z = acc[0][e], s = sigmoid_f(z);
+            const float z = acc[0][e] + bv[e], u = 1.0f + expf(-z), s = 1.0f / u;
             ds[t * 4 + e] = s * (1.0f + z * (1.0f - s));
-            a[e] = z * s;
+            a[e] = z / u;
+            // computed here: left until the backward pass, z and u would both
+            // be held (and spilled)
+            asm volatile("" : "+v"(ds[t * 4 + e]));
         }
         const unsigned int p0 = pack_bf16(a[0], a[1]), p1 = pack_bf16(a[2], a[3]);
         h[t >> 1][0][(t & 1) * 2] = p0;
         h[t >> 1][0][(t & 1) * 2 + 1] = p1;
-        store_rows(rows, t * 16 + 4 * q, r, p0, p1);
+        store_rows(rows, t, at, lane, p0, p1);
     }
 }
 
@@ -331,9 +369,9 @@ __device__ __forceinline__ void train_forward(const u32x4* w, const float* b, co
 // target of output err_head is log10(|y0 - t0| * ln10 + 1e-5) of the current
 // prediction (no gradient through it).  Eight waves share the forward
 // fragments in LDS; the backward ones, read once per 16 cells, come from L2
-// (both sets do not fit in 160 KB).  Bound by the latency of those reads and
-// the SiLU: 87 us for 65,536 cells, at most one workgroup per CU so that the
-// 108 KB are staged once.
+// (both sets do not fit in 160 KB).  Bound by the SiLU's exponential and two
+// divisions per unit and the latency of those reads; at most one workgroup per
+// CU so that the 108 KB are staged once.
 // 128 registers hold the SiLU derivatives of the four layers, which leaves
 // two waves per SIMD.
 __global__ __launch_bounds__(TRAIN_THREADS) void mlp_train_kernel(const bf16_t* __restrict__ packed,
@@ -341,98 +379,74 @@ __global__ __launch_bounds__(TRAIN_THREADS) void mlp_train_kernel(const bf16_t* 
                                                                  const float* __restrict__ feat,
                                                                  const float* __restrict__ target, int B, float m0,
                                                                  float m1, float m2, int err_head, TrainBuffers tb) {
-    __shared__ TrainLDS s;
+    __shared__ NetLDS net;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar addresses
     const int q = lane >> 4, r = lane & 15;
-    stage_net(s.net, packed, bias, tid, TRAIN_THREADS);
+    const bf16_t* fwd = packed + MLP_NFF * MLP_FRAG;
+    stage_net(net, fwd, bias, tid, TRAIN_THREADS);
     const int ntiles = 2 * ((B + 31) / 32);  // whole blocks of 32 cells: padding cells get zero gradients
-    float gb[4][2] = {}, gbo[3] = {0.f, 0.f, 0.f};
-    float loss = 0.f;
     for (int tile = blockIdx.x * TRAIN_WAVES + wave; tile < ntiles; tile += gridDim.x * TRAIN_WAVES) {
         // as in the inference kernel; the backward fragments' base is made
         // opaque here too, or their addresses are hoisted and spill
-        const u32x4* wb = reinterpret_cast<const u32x4*>(packed + MLP_NFF * MLP_FRAG);
+        const u32x4* wb = reinterpret_cast<const u32x4*>(fwd + MLP_NFF * MLP_FRAG);
         asm volatile("" : "+s"(wb) : : "memory");
-        const int c = tile * 16 + r;
         const long long blk = tile >> 1;
-        const int half = (tile & 1) * 16;
-        const auto rows = [&](bf16_t* base) { return base + blk * (MLP_H * 32) + half; };
+        const int cb = tile_cell(tile & 1, r);
+        const long long c = blk * 32 + cb;
+        const unsigned int at = row_place(q, cb);
+        const auto rows = [&](bf16_t* base) { return base + blk * (MLP_H * 32); };
+        float* sums = tb.bsum + (long long)tile * (4 * MLP_H);
         u32x4 x1[1][1], ha[4][1], hb[4][1];
         x1[0][0] = load_features(feat, c, B, q);
         if (q == 0) {
-            bf16_t* d = tb.h[0] + blk * (MLP_IN * 32) + half + r;
+            bf16_t* d = tb.h[0] + blk * (MLP_IN * 32) + cb;
 #pragma unroll
             for (int i = 0; i < MLP_IN; ++i) d[i * 32] = (bf16_t)(x1[0][0][i >> 1] >> ((i & 1) * 16));
         }
         float z1[32], z2[32], z3[32], z4[32];
-        train_forward<1>(s.net.w, s.net.b, x1, z1, ha, rows(tb.h[1]), lane);
-        train_forward<4>(s.net.w + 8 * 64, s.net.b + MLP_H, ha, z2, hb, rows(tb.h[2]), lane);
-        train_forward<4>(s.net.w + 40 * 64, s.net.b + 2 * MLP_H, hb, z3, ha, rows(tb.h[3]), lane);
-        train_forward<4>(s.net.w + 72 * 64, s.net.b + 3 * MLP_H, ha, z4, hb, rows(tb.h[4]), lane);
-        f32x4 y[1] = {*reinterpret_cast<const f32x4*>(s.net.b + 4 * MLP_H + 4 * q)};
-        row_tile<4, 1>(s.net.w + 104 * 64, 0, lane, hb, y);
+        train_forward<1>(net.w, net.b, x1, z1, ha, rows(tb.h[1]), at, lane);
+        train_forward<4>(net.w + 8 * 64, net.b + MLP_H, ha, z2, hb, rows(tb.h[2]), at, lane);
+        train_forward<4>(net.w + 40 * 64, net.b + 2 * MLP_H, hb, z3, ha, rows(tb.h[3]), at, lane);
+        train_forward<4>(net.w + 72 * 64, net.b + 3 * MLP_H, ha, z4, hb, rows(tb.h[4]), at, lane);
+        f32x4 y[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+        row_tile<4, 1>(net.w + 104 * 64, 0, lane, hb, y);
+        y[0] += *reinterpret_cast<const f32x4*>(net.b + 4 * MLP_H + 4 * q);
         // lane group 0 holds the outputs of cell c
-        float dy[3] = {0.f, 0.f, 0.f};
+        f32x4 dy = {0.f, 0.f, 0.f, 0.f};  // and the cell's loss
         if (q == 0 && c < B) {
             const float ms[3] = {m0, m1, m2};
-            const float t0 = target[(long long)c * MLP_NOUT];
+            const float t0 = target[c * MLP_NOUT];
 #pragma unroll
             for (int o = 0; o < MLP_NOUT; ++o) {
-                float t = target[(long long)c * MLP_NOUT + o];
+                float t = target[c * MLP_NOUT + o];
                 if (o == err_head) t = log10f(fabsf(y[0][0] - t0) * 2.302585093f + 1e-5f);
                 const float d = y[0][o] - t;
-                loss += 0.5f * ms[o] * d * d;
+                dy[3] += 0.5f * ms[o] * d * d;
                 dy[o] = ms[o] * d / (float)B;
             }
         }
         u32x4 g[1][1] = {{u32x4{pack_bf16(dy[0], dy[1]), pack_bf16(dy[2], 0.f), 0u, 0u}}};
         if (q == 0) {
-            bf16_t* d = tb.dz[5] + blk * (4 * 32) + half + r;
+            tb.cell[c] = dy;
+            bf16_t* d = tb.dz[5] + blk * (4 * 32) + cb;
 #pragma unroll
             for (int o = 0; o < MLP_NOUT; ++o) d[o * 32] = (bf16_t)(g[0][0][o >> 1] >> ((o & 1) * 16));
         }
-#pragma unroll
-        for (int o = 0; o < MLP_NOUT; ++o) gbo[o] += dy[o];
-        train_backward<1>(wb, g, z4, ha, rows(tb.dz[4]), gb[3], lane);
-        train_backward<4>(wb + 72 * 64, ha, z3, hb, rows(tb.dz[3]), gb[2], lane);
-        train_backward<4>(wb + 40 * 64, hb, z2, ha, rows(tb.dz[2]), gb[1], lane);
-        train_backward<4>(wb + 8 * 64, ha, z1, hb, rows(tb.dz[1]), gb[0], lane);
-    }
-#pragma unroll
-    for (int l = 0; l < 4; ++l)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) s.gb[wave][l * MLP_H + 64 * i + 16 * (r >> 2) + 4 * q + (r & 3)] = gb[l][i];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        loss += __shfl_xor(loss, off, 64);
-#pragma unroll
-        for (int o = 0; o < MLP_NOUT; ++o) gbo[o] += __shfl_xor(gbo[o], off, 64);
-    }
-    if (lane == 0) {
-        s.loss[wave] = loss;
-#pragma unroll
-        for (int o = 0; o < MLP_NOUT; ++o) s.gb[wave][4 * MLP_H + o] = gbo[o];
-    }
-    __syncthreads();
-    for (int i = tid; i < (int)MLP_NB; i += TRAIN_THREADS) {
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < TRAIN_WAVES; ++w) v += s.gb[w][i];
-        tb.bpart[(long long)blockIdx.x * MLP_NB + i] = v;
-    }
-    if (tid == 0) {
-        float v = 0.f;
-        for (int w = 0; w < TRAIN_WAVES; ++w) v += s.loss[w];
-        tb.loss_part[blockIdx.x] = v;
+        train_backward<1>(wb, g, z4, ha, rows(tb.dz[4]), sums + 3 * MLP_H, at, lane);
+        train_backward<4>(wb + 72 * 64, ha, z3, hb, rows(tb.dz[3]), sums + 2 * MLP_H, at, lane);
+        train_backward<4>(wb + 40 * 64, hb, z2, ha, rows(tb.dz[2]), sums + MLP_H, at, lane);
+        train_backward<4>(wb + 8 * 64, ha, z1, hb, rows(tb.dz[1]), sums, at, lane);
     }
 }
 
 // Fragment of 16 feature rows x 32 cells of block `blk`: lane (q, r) takes
-// the 8 cells 8q.. of row m + r, zero for rows past `rows`.
-__device__ __forceinline__ bf16x8 load_rows(const bf16_t* __restrict__ a, long long blk, int rows, int m, int q, int r) {
+// the 8 cells 8q.. of row m + r, zero for rows past `valid` of the `rows`
+// stored.
+__device__ __forceinline__ bf16x8 load_rows(const bf16_t* __restrict__ a, long long blk, int rows, int valid, int m, int q,
+                                            int r) {
     u32x4 v = {0u, 0u, 0u, 0u};
-    if (m + r < rows) v = *reinterpret_cast<const u32x4*>(a + (blk * rows + m + r) * 32 + q * 8);
+    if (valid >= MLP_H || m + r < valid) v = *reinterpret_cast<const u32x4*>(a + (blk * rows + m + r) * 32 + q * 8);
     return as_bf16x8(v);
 }
 
@@ -444,70 +458,109 @@ __device__ __forceinline__ void store_tile(float* __restrict__ p, int ldn, int r
         if (m + 4 * q + e < rows && n + r < ldn) p[(m + 4 * q + e) * ldn + n + r] = c[e];
 }
 
-// Weight gradients of chunk blockIdx.x (`nblk` blocks of 32 cells): job 0..2
-// the 128 x 128 layers (a 64 x 64 quadrant per wave), job 3 the first and the
-// output layer.  Bound by the latency of the fragment reads: two blocks in
-// flight and up to 128 chunks took 65,536 cells from 66 to 33 us, and the
-// longer sum of partials in reduce_adam_kernel from 10 to 13.
-__global__ __launch_bounds__(256) void mlp_wgrad_kernel(int blocks, int nblk, TrainBuffers tb) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int q = lane >> 4, r = lane & 15, job = blockIdx.y;
-    const long long b0 = (long long)blockIdx.x * nblk, b1 = min((long long)blocks, b0 + nblk);
-    float* part = tb.wpart + (long long)blockIdx.x * MLP_NW;
-    if (job < 3) {
-        const bf16_t* dz = tb.dz[job + 2];
-        const bf16_t* h = tb.h[job + 1];
-        const int m0 = (wave >> 1) * 64, n0 = (wave & 1) * 64;
-        f32x4 acc[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-        for (long long blk = b0; blk < b1; ++blk) {
-            bf16x8 a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = load_rows(dz, blk, MLP_H, m0 + i * 16, q, r);
-                b[i] = load_rows(h, blk, MLP_H, n0 + i * 16, q, r);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        float* p = part + MLP_H * MLP_IN + job * MLP_H * MLP_H;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) store_tile(p, MLP_H, MLP_H, m0 + i * 16, n0 + j * 16, q, r, acc[i][j]);
+// Loss and output-bias gradient of 256 cells: the loss as a binary tree, each
+// output's gradient one cell after another.
+__device__ __forceinline__ void output_sums(const TrainBuffers& tb, int blk, int B) {
+    __shared__ f32x4 v[256];
+    __shared__ float tree[256];
+    const int tid = threadIdx.x;
+    const long long c = (long long)blk * 256 + tid;
+    const f32x4 x = c < B ? tb.cell[c] : f32x4{0.f, 0.f, 0.f, 0.f};
+    v[tid] = x;
+    tree[tid] = x[3];
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if (tid < s) tree[tid] += tree[tid + s];
+        __syncthreads();
+    }
+    if (tid == 0) tb.loss_part[blk] = tree[0];
+    if (tid < MLP_NOUT) {
+        const float* col = reinterpret_cast<const float*>(v) + tid;
+        float s = 0.f;
+#pragma unroll 16
+        for (int i = 0; i < 256; ++i) s += col[4 * i];  // zeros past the last cell
+        tb.opart[(long long)blk * MLP_NOUT + tid] = s;
+    }
+}
+
+// Weight gradients of `nblk` blocks of 32 cells: workgroup (chunk, job) of
+// the first nz * WGRAD_JOBS, jobs 0 .. 11 a 64 x 64 quadrant of a 128 x 128
+// layer (32 x 32 per wave), jobs 12 and 13 half of the first and the output
+// layer; the workgroups past them sum the outputs of 256 cells each.  Bound
+// by the latency of the fragment reads, several blocks in flight per wave.
+// At most 32 chunks, whose sums are then added in order: a gradient is the
+// same however the batch is spread over the chip.
+constexpr int WGRAD_JOBS = 14, WGRAD_AHEAD = 8;
+__global__ __launch_bounds__(256) void mlp_wgrad_kernel(int B, int blocks, int nblk, int nz, TrainBuffers tb) {
+    if ((int)blockIdx.x >= nz * WGRAD_JOBS) {
+        output_sums(tb, (int)blockIdx.x - nz * WGRAD_JOBS, B);
         return;
     }
-    f32x4 c1[2], c5[2];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane >> 4, r = lane & 15, job = blockIdx.x % WGRAD_JOBS, chunk = blockIdx.x / WGRAD_JOBS;
+    const long long b0 = (long long)chunk * nblk, b1 = min((long long)blocks, b0 + nblk);
+    float* part = tb.wpart + (long long)chunk * MLP_NW;
+    if (job < 12) {
+        const int l = job >> 2;
+        const bf16_t* dz = tb.dz[l + 2];
+        const bf16_t* h = tb.h[l + 1];
+        const int m0 = ((job >> 1) & 1) * 64 + (wave >> 1) * 32, n0 = (job & 1) * 64 + (wave & 1) * 32;
+        f32x4 acc[2][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) c1[i] = c5[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long long blk = b0; blk < b1; ++blk) {
-        const bf16x8 x = load_rows(tb.h[0], blk, MLP_IN, 0, q, r);
-        bf16x8 dy;
-        {
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (r < MLP_NOUT) v = *reinterpret_cast<const u32x4*>(tb.dz[5] + (blk * 4 + r) * 32 + q * 8);
-            dy = as_bf16x8(v);
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const auto step = [&](auto nb, long long blk) {  // nb blocks, their loads first
+            constexpr int N = decltype(nb)::value;
+            bf16x8 a[N][2], b[N][2];
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[k][i] = load_rows(dz, blk + k, MLP_H, MLP_H, m0 + i * 16, q, r);
+                    b[k][i] = load_rows(h, blk + k, MLP_H, MLP_H, n0 + i * 16, q, r);
+                }
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k][i], b[k][j], acc[i][j], 0, 0, 0);
+        };
+        long long blk = b0;
+        for (; blk + WGRAD_AHEAD <= b1; blk += WGRAD_AHEAD) step(std::integral_constant<int, WGRAD_AHEAD>{}, blk);
+        for (; blk < b1; ++blk) step(std::integral_constant<int, 1>{}, blk);
+        float* p = part + MLP_H * MLP_IN + l * MLP_H * MLP_H;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) store_tile(p, MLP_H, MLP_H, m0 + i * 16, n0 + j * 16, q, r, acc[i][j]);
+        return;
+    }
+    const int f = ((job - 12) * 4 + wave) * 16;
+    f32x4 c1 = {0.f, 0.f, 0.f, 0.f}, c5 = c1;
+    const auto step = [&](auto nb, long long blk) {
+        constexpr int N = decltype(nb)::value;
+        bf16x8 a1[N], b1[N], a5[N], b5[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            a1[k] = load_rows(tb.dz[1], blk + k, MLP_H, MLP_H, f, q, r);
+            b1[k] = load_rows(tb.h[0], blk + k, MLP_IN, MLP_IN, 0, q, r);
+            a5[k] = load_rows(tb.dz[5], blk + k, 4, MLP_NOUT, 0, q, r);
+            b5[k] = load_rows(tb.h[4], blk + k, MLP_H, MLP_H, f, q, r);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int f = (wave * 2 + i) * 16;
-            c1[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_rows(tb.dz[1], blk, MLP_H, f, q, r), x, c1[i], 0, 0, 0);
-            c5[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dy, load_rows(tb.h[4], blk, MLP_H, f, q, r), c5[i], 0, 0, 0);
+        for (int k = 0; k < N; ++k) {
+            c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[k], b1[k], c1, 0, 0, 0);
+            c5 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a5[k], b5[k], c5, 0, 0, 0);
         }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int f = (wave * 2 + i) * 16;
-        store_tile(part, MLP_IN, MLP_H, f, 0, q, r, c1[i]);
-        store_tile(part + MLP_H * MLP_IN + 3 * MLP_H * MLP_H, MLP_H, MLP_NOUT, 0, f, q, r, c5[i]);
-    }
+    };
+    long long blk = b0;
+    for (; blk + WGRAD_AHEAD <= b1; blk += WGRAD_AHEAD) step(std::integral_constant<int, WGRAD_AHEAD>{}, blk);
+    for (; blk < b1; ++blk) step(std::integral_constant<int, 1>{}, blk);
+    store_tile(part, MLP_IN, MLP_H, f, 0, q, r, c1);
+    store_tile(part + MLP_H * MLP_IN + 3 * MLP_H * MLP_H, MLP_H, MLP_NOUT, 0, f, q, r, c5);
 }
 
 // Adam on one fp32 master parameter; returns its new value.
@@ -521,14 +574,21 @@ __device__ __forceinline__ float adam_step(const AdamArgs& a, float p, float g, 
 }
 
 constexpr int REDUCE_WBLOCKS = (int)((MLP_NW + 255) / 256);
+constexpr int REDUCE_BIAS = 16;                               // hidden biases per workgroup
+constexpr int REDUCE_BBLOCKS = 4 * MLP_H / REDUCE_BIAS + 1;   // the last: the output biases
+constexpr int REDUCE_CHUNK = 512;
 
-// Gradients from the partials: a thread per weight (chunks in ascending
-// order), then a wave per bias (64 interleaved sums, added by a shuffle
-// tree); with a.update also Adam and the new weights' fragments.
-__global__ __launch_bounds__(256) void reduce_adam_kernel(TrainBuffers tb, int nz, int nwg, float* __restrict__ gW,
+// Gradients from the partials, each sum from the first to the last: a thread
+// per weight; 16 hidden biases per workgroup, whose terms of 64 cells (four
+// tiles, added in pairs) all its threads load into LDS for one thread per bias to
+// add up; the output biases likewise from their sums of 256 cells.  With
+// a.update also Adam and the new weights' fragments.
+__global__ __launch_bounds__(256) void reduce_adam_kernel(TrainBuffers tb, int B, int nz, float* __restrict__ gW,
                                                           float* __restrict__ gb, AdamArgs a) {
+    __shared__ f32x4 term[REDUCE_CHUNK][REDUCE_BIAS / 4];
+    const int tid = threadIdx.x;
     if (blockIdx.x < REDUCE_WBLOCKS) {
-        const int i = blockIdx.x * 256 + threadIdx.x;
+        const int i = blockIdx.x * 256 + tid;
         if (i >= (int)MLP_NW) return;
         float g = 0.f;
 #pragma unroll 8
@@ -541,13 +601,40 @@ __global__ __launch_bounds__(256) void reduce_adam_kernel(TrainBuffers tb, int n
         }
         return;
     }
-    const int i = (blockIdx.x - REDUCE_WBLOCKS) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (i >= (int)MLP_NB) return;
+    const int i0 = (blockIdx.x - REDUCE_WBLOCKS) * REDUCE_BIAS;
+    const bool out = i0 == 4 * MLP_H;
+    const int nbias = out ? MLP_NOUT : REDUCE_BIAS;
+    const int tiles = 2 * ((B + 31) / 32);
+    const long long n = out ? ((long long)B + 255) / 256 : ((long long)B + 63) / 64;
+    const float* col = reinterpret_cast<const float*>(term) + tid;
     float g = 0.f;
-    for (int k = lane; k < nwg; k += 64) g += tb.bpart[(long long)k * MLP_NB + i];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) g += __shfl_xor(g, off, 64);
-    if (lane == 0) {
+    for (long long t0 = 0; t0 < n; t0 += REDUCE_CHUNK) {
+        const int m = (int)min((long long)REDUCE_CHUNK, n - t0);
+        __syncthreads();
+        if (out) {
+            for (int j = tid; j < m; j += 256) {
+                const float* p = tb.opart + (t0 + j) * MLP_NOUT;
+                term[j][0] = f32x4{p[0], p[1], p[2], 0.f};
+            }
+        } else {
+            const int b4 = tid % (REDUCE_BIAS / 4);
+#pragma unroll 4
+            for (int j = tid / (REDUCE_BIAS / 4); j < m; j += 256 / (REDUCE_BIAS / 4)) {
+                const long long t = 4 * (t0 + j);
+                const f32x4* p = reinterpret_cast<const f32x4*>(tb.bsum + t * (4 * MLP_H) + i0) + b4;
+                f32x4 lo = p[0] + p[MLP_H], hi = {0.f, 0.f, 0.f, 0.f};  // p[MLP_H]: the next tile
+                if (t + 2 < tiles) hi = p[2 * MLP_H] + p[3 * MLP_H];
+                term[j][b4] = lo + hi;
+            }
+        }
+        __syncthreads();
+        if (tid < nbias) {
+#pragma unroll 16
+            for (int j = 0; j < m; ++j) g += col[j * REDUCE_BIAS];
+        }
+    }
+    if (tid < nbias) {
+        const int i = i0 + tid;
         gb[i] = g;
         if (a.update) a.b[i] = adam_step(a, a.b[i], g, a.mb + i, a.vb + i, 0.f);
     }
@@ -562,12 +649,11 @@ hipError_t launch_mlp_pack(const float* W, uint16_t* packed, hipStream_t stream)
 }
 
 hipError_t launch_mlp_train_fused(const uint16_t* packed, const float* bias, const float* feat, const float* target,
-                                  int B, float m0, float m1, float m2, int err_head, const TrainBuffers& t, int* nwg,
+                                  int B, float m0, float m1, float m2, int err_head, const TrainBuffers& t,
                                   hipStream_t stream) {
     const int tiles = 2 * ((B + 31) / 32);
     int nb = (tiles + TRAIN_WAVES - 1) / TRAIN_WAVES;
     if (nb > MLP_TRAIN_MAX_WG) nb = MLP_TRAIN_MAX_WG;
-    *nwg = nb;
     hipLaunchKernelGGL(mlp_train_kernel, dim3((unsigned)nb), dim3(TRAIN_THREADS), 0, stream, packed, bias, feat,
                        target, B, m0, m1, m2, err_head, t);
     return hipGetLastError();
@@ -577,14 +663,15 @@ hipError_t launch_mlp_weight_grad(int B, const TrainBuffers& t, int* nz, hipStre
     const int blocks = (B + 31) / 32;
     const int nblk = (blocks + MLP_TRAIN_MAX_NZ - 1) / MLP_TRAIN_MAX_NZ;
     *nz = (blocks + nblk - 1) / nblk;
-    hipLaunchKernelGGL(mlp_wgrad_kernel, dim3((unsigned)*nz, 4), dim3(256), 0, stream, blocks, nblk, t);
+    hipLaunchKernelGGL(mlp_wgrad_kernel, dim3((unsigned)(*nz * WGRAD_JOBS + (B + 255) / 256)), dim3(256), 0, stream, B,
+                       blocks, nblk, *nz, t);
     return hipGetLastError();
 }
 
-hipError_t launch_mlp_reduce_adam(const TrainBuffers& t, int nz, int nwg, float* gW, float* gb, const AdamArgs& a,
+hipError_t launch_mlp_reduce_adam(int B, const TrainBuffers& t, int nz, float* gW, float* gb, const AdamArgs& a,
                                   hipStream_t stream) {
-    hipLaunchKernelGGL(reduce_adam_kernel, dim3(REDUCE_WBLOCKS + (unsigned)((MLP_NB + 3) / 4)), dim3(256), 0, stream, t,
-                       nz, nwg, gW, gb, a);
+    hipLaunchKernelGGL(reduce_adam_kernel, dim3(REDUCE_WBLOCKS + REDUCE_BBLOCKS), dim3(256), 0, stream, t, B, nz, gW, gb,
+                       a);
     return hipGetLastError();
 }
 

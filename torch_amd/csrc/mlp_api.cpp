@@ -46,17 +46,17 @@ int loss_grad(torchgpu_mlp* m, const float* feat, const float* target, int B, co
               float* loss, const tg::AdamArgs& adam) {
     if (B <= 0 || B > m->max_batch) return TORCHGPU_ERR_INVALID_ARG;
     const float w0 = w3 ? w3[0] : 1.f, w1 = w3 ? w3[1] : 1.f, w2 = w3 ? w3[2] : 1.f;
-    int nwg = 0, nz = 0;
-    HIP_CHECK(tg::launch_mlp_train_fused(m->packed, m->b, feat, target, B, w0, w1, w2, err_head ? 2 : -1, m->t, &nwg,
+    int nz = 0;
+    HIP_CHECK(tg::launch_mlp_train_fused(m->packed, m->b, feat, target, B, w0, w1, w2, err_head ? 2 : -1, m->t,
                                          m->stream));
     HIP_CHECK(tg::launch_mlp_weight_grad(B, m->t, &nz, m->stream));
-    HIP_CHECK(tg::launch_mlp_reduce_adam(m->t, nz, nwg, m->gW, m->gb, adam, m->stream));
+    HIP_CHECK(tg::launch_mlp_reduce_adam(B, m->t, nz, m->gW, m->gb, adam, m->stream));
     if (loss) {
-        float lp[tg::MLP_TRAIN_MAX_WG];
-        HIP_CHECK(hipMemcpyAsync(lp, m->t.loss_part, nwg * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+        std::vector<float> lp((B + 255LL) / 256);
+        HIP_CHECK(hipMemcpyAsync(lp.data(), m->t.loss_part, lp.size() * sizeof(float), hipMemcpyDeviceToHost, m->stream));
         HIP_CHECK(hipStreamSynchronize(m->stream));
         double s = 0;
-        for (int i = 0; i < nwg; ++i) s += lp[i];
+        for (float v : lp) s += v;
         *loss = (float)(s / B);
     }
     return TORCHGPU_OK;
@@ -94,9 +94,12 @@ int torchgpu_mlp_create(int max_batch, void* stream, torchgpu_mlp** out) {
         alloc((void**)&m->t.dz[L], blocks * 32 * MLP_H * 2);
     }
     alloc((void**)&m->t.dz[5], blocks * 32 * 4 * 2);
-    alloc((void**)&m->t.wpart, (size_t)tg::MLP_TRAIN_MAX_NZ * MLP_NW * 4);
-    alloc((void**)&m->t.bpart, (size_t)tg::MLP_TRAIN_MAX_WG * MLP_NB * 4);
-    alloc((void**)&m->t.loss_part, tg::MLP_TRAIN_MAX_WG * 4);
+    const long long nz = blocks < tg::MLP_TRAIN_MAX_NZ ? blocks : tg::MLP_TRAIN_MAX_NZ;
+    alloc((void**)&m->t.cell, blocks * 32 * sizeof(tg::mlp_f32x4));
+    alloc((void**)&m->t.bsum, blocks * 2 * 4 * MLP_H * 4);
+    alloc((void**)&m->t.wpart, nz * MLP_NW * 4);
+    alloc((void**)&m->t.opart, (max_batch + 255LL) / 256 * tg::MLP_NOUT * 4);
+    alloc((void**)&m->t.loss_part, (max_batch + 255LL) / 256 * 4);
     if (!ok) {
         torchgpu_mlp_destroy(m);
         return TORCHGPU_ERR_HIP;
@@ -114,8 +117,8 @@ int torchgpu_mlp_create(int max_batch, void* stream, torchgpu_mlp** out) {
 void torchgpu_mlp_destroy(torchgpu_mlp* m) {
     if (!m) return;
     (void)hipStreamSynchronize(m->stream);
-    std::vector<void*> ptrs = {m->W, m->b, m->packed, m->gW, m->gb, m->mW, m->vW, m->mb, m->vb, m->t.wpart,
-                               m->t.bpart, m->t.loss_part};
+    std::vector<void*> ptrs = {m->W, m->b, m->packed, m->gW, m->gb, m->mW, m->vW, m->mb, m->vb, m->t.cell,
+                               m->t.bsum, m->t.wpart, m->t.opart, m->t.loss_part};
     for (int L = 0; L <= 4; ++L) ptrs.push_back(m->t.h[L]);
     for (int L = 1; L <= 5; ++L) ptrs.push_back(m->t.dz[L]);
     for (void* p : ptrs)
