@@ -71,6 +71,38 @@ def test_thermo_cells_vs_oracle_workload_sample(gpu, orc):
     assert np.median(rel) < 1e-14 and rel.max() < 1e-6, np.quantile(rel, [0.5, 0.99, 1.0])
 
 
+@pytest.mark.parametrize("knots", ["own", "lower", "between", "narrow", "wide", "uneven"])
+def test_cooling_spline_takes_its_own_abscissae(gpu, orc, knots):
+    """Spline tables whose abscissae are not the operator's own 3.5 .. 6.0:
+    moved, of another spacing near 0.1, or uneven.  Pre-step rates of cells
+    between 300 and 1e7 K against the oracle's bracketing search, both within
+    a few ulp of log10 T on a spline of slope 60: 1e-12 of the terms."""
+    import torch
+
+    k = np.arange(26)
+    x = {"own": None, "lower": 3.0 + 0.1 * k, "between": 3.55 + 0.1 * k, "narrow": 3.5 + 0.0985 * k,
+         "wide": 3.4 + 0.1035 * k, "uneven": 3.5 + 0.1 * k + 0.04 * np.sin(2.1 * k)}[knots]
+    c = orc.converter(1e-20, 1e-28, 1e11)
+    tc = lambda v, m, l, t: orc.to_code(c, v, m, l, t)  # noqa: E731
+    s = cooling_inputs.sample_cgs(4096, seed=21)
+    inp = cooling_inputs.to_code_inputs(s, tc)
+    T = 10.0 ** np.linspace(2.5, 7.0, 4096)
+    inp[:, 1] = inp[:, 0] * tc(8.314462e7, 0, 2, -2) * (inp[:, 2] + 1.0) * T
+    inp[:, 4] = inp[:, 1] / (1.67 - 1.0)
+    t = orc.thermo_params(c, subcycling=False)
+    p = gpu.thermo_params(subcycling=False)
+    if x is not None:
+        for i in range(26):
+            t.spl_x[i] = p.spl_x[i] = x[i]
+    p.pfloor = t.pfloor
+    ref = orc.thermo_batch(t, inp, nthreads=8)
+    out, _ = gpu.Cooling(p).thermo_cells(torch.from_numpy(np.ascontiguousarray(inp.T)).cuda())
+    out = out.cpu().numpy()
+    scale = np.abs(ref[:, 0]) + np.abs(ref[:, 1])
+    err = np.abs(out[1] - ref[:, 1]) / scale
+    assert err.max() < 1e-12, (err.max(), T[err.argmax()])
+
+
 def test_thermo_gate_and_no_subcycling(gpu, orc):
     import torch
 

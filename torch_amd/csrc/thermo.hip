@@ -31,6 +31,7 @@
 //   fallback  the persistent FP64 kernel over the fallback queue
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -1104,6 +1105,10 @@ tg::ThermoConsts to_consts(const torchgpu_thermo_params& p) {
     t.spl_min_slope = p.spl_min_slope;
     t.spl_max_slope = p.spl_max_slope;
     t.icxhi = 1.0 / p.cxhi_damp;
+    t.spl_k0 = 1.0 - 10.0 * p.spl_x[0];
+    t.spl_even = 1;
+    for (int k = 1; k < 26; ++k)
+        if (!(std::fabs(p.spl_x[k] - (p.spl_x[0] + 0.1 * k)) < 1.0e-9)) t.spl_even = 0;
     t.subcycling = p.subcycling;
     return t;
 }

@@ -21,8 +21,9 @@ struct ThermoConsts {
     double fuvh_a, fuvh_b, fuvh_c, irh_a, irh_b, crh;
     double spl_min_slope, spl_max_slope;
     double icxhi;  // 1 / cxhi_damp
+    double spl_k0; // 1 - 10 spl_x[0]: the spline piece at log10 T is 10 log10 T + spl_k0
     int subcycling;
-    int pad;
+    int spl_even;  // the abscissae are spl_x[0] + k / 10 to 1e-9
 };
 
 // ---------------------------------------------------------------------------
@@ -131,17 +132,27 @@ __device__ __forceinline__ double rcp_t(double x) {
 }
 
 // The cooling spline (LogSplineData::interpolate) at log10 T for ln T = hi +
-// lo: the piece from the uniform 0.1 spacing of the abscissae (two pieces
-// agree at their knot to rounding, so a neighbour chosen by rounding there
-// changes nothing).  The spline is steep (20 decades in 1.5 of T): the offset
-// from the knot is formed from both parts, or the rounding of log10 T alone
-// would be 2e-14 of the rate.
-__device__ __forceinline__ double log_spline_t(const double* tab, double hi, double lo) {
+// lo: the piece from the 0.1 spacing of the abscissae (two pieces agree at
+// their knot to rounding, so a neighbour chosen by rounding there changes
+// nothing), corrected by one against the stored ones, as log_spline does,
+// where they are not that even.  The spline is steep (20 decades in 1.5 of T):
+// the offset from the knot is formed from both parts, or the rounding of log10
+// T alone would be 2e-14 of the rate.
+__device__ __forceinline__ double log_spline_t(const ThermoConsts& t, const double* tab, double hi, double lo) {
     const double x = hi * 0x1.bcb7b1526e50ep-2;
     const double xl = __builtin_fma(lo, 0x1.bcb7b1526e50ep-2,
                                     __builtin_fma(hi, 0x1.95355baaafad3p-57, __builtin_fma(hi, 0x1.bcb7b1526e50ep-2, -x)));
-    int k = (int)__builtin_fma(x + xl, 10.0, -34.0);  // 0 below 3.5, 26 from 6.0 on
+    int k = (int)__builtin_fma(x + xl, 10.0, t.spl_k0);  // 0 below the first knot, 26 from the last on
     k = k < 0 ? 0 : (k > TT_NSPL - 1 ? TT_NSPL - 1 : k);
+    if (__builtin_expect(!t.spl_even, 0)) {  // piece 0 starts at knot 0, piece j at knot j - 1
+        const double* knot = tab + TT_SPL + 1;
+        const double v = x + xl;
+        k = k < 1 ? 1 : (k > TT_NSPL - 2 ? TT_NSPL - 2 : k);
+        if (knot[k - 1] > v) --k;
+        else if (knot[k] <= v) ++k;
+        if (knot[0] > v) k = 0;
+        if (knot[TT_NSPL - 2] < v) k = TT_NSPL - 1;
+    }
     const double* p = tab + TT_SPL + k;
     const double s = (x - p[0]) + xl;
     double r = __builtin_fma(p[4 * TT_NSPL], s, p[3 * TT_NSPL]);
@@ -151,8 +162,8 @@ __device__ __forceinline__ double log_spline_t(const double* tab, double hi, dou
 
 // Natural cubic spline in log10 space: LogSplineData::interpolate +
 // SplineData::splint (SplineData.cpp:57-81,142-151).  x, y, y2 are 26-entry
-// tables (LDS) whose abscissae are log10 T = 3.5, 3.6, ..., 6.0 up to
-// rounding: the bracketing interval of the reference's bisection (largest
+// tables (LDS) whose abscissae are 0.1 apart (log10 T = 3.5, 3.6, ..., 6.0, the
+// operator's own) up to rounding: the bracketing interval of the reference's bisection (largest
 // klo <= 24 with x[klo] <= x) is found from the spacing and corrected by one
 // step against the stored abscissae, which gives the same klo.
 __device__ __forceinline__ double log_spline(const ThermoConsts& t, const double* sx, const double* sy,
@@ -229,7 +240,7 @@ __device__ __forceinline__ double subtract_cooling(const ThermoConsts& t, const 
     log_t(tab, T, hi, lo);
     const double a1 = t.T2 * iT, a2 = t.T4 * iT, a3 = T * t.icxhi;
     double e[4] = {exp_floor(__builtin_fma(-a1, a1, -t.T1 * iT)), exp_floor(__builtin_fma(-a2, a2, -t.T3 * iT)),
-                   exp_floor(__builtin_fma(2.302585093, log_spline_t(tab, hi, lo), -(a3 * a3))),
+                   exp_floor(__builtin_fma(2.302585093, log_spline_t(t, tab, hi, lo), -(a3 * a3))),
                    exp_floor(__builtin_fma(0.5, lo, __builtin_fma(-c.nmc_T0, iT, 0.5 * hi)))};
     exp_n<4>(tab, e);
     rate -= c.imlc_k * e[0];
