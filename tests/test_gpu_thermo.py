@@ -103,6 +103,32 @@ def test_cooling_spline_takes_its_own_abscissae(gpu, orc, knots):
     assert err.max() < 1e-12, (err.max(), T[err.argmax()])
 
 
+def test_cooling_rate_of_extreme_temperatures(gpu, orc):
+    """Pre-step rates of neutral, half and fully ionised cells from 1e-300 to
+    1e290 K (and some at the operator's own temperatures) against the
+    oracle: ln T up to 690 times half an ulp in an exponent is 1e-13."""
+    import torch
+
+    c = orc.converter(1e-20, 1e-28, 1e11)
+    t = orc.thermo_params(c, subcycling=False)
+    p = gpu.thermo_params(subcycling=False)
+    p.pfloor = t.pfloor
+    T = np.concatenate([10.0 ** np.linspace(-300, 290, 1181), 10.0 ** np.linspace(1, 9, 161)])
+    T, x = (a.ravel() for a in np.meshgrid(T, [0.0, 0.5, 1.0]))
+    inp = np.zeros((T.size, 9))
+    inp[:, 0] = 1e-10
+    inp[:, 1] = inp[:, 0] * t.spec_gas_const * (x + 1.0) * T
+    inp[:, 2], inp[:, 3], inp[:, 5] = x, 1.0, 100.0
+    inp[:, 4] = inp[:, 1] / (1.67 - 1.0)
+    inp[:, 8] = 1e-3
+    ref = orc.thermo_batch(t, inp, nthreads=8)
+    assert np.isfinite(ref[:, 1]).all()
+    out, _ = gpu.Cooling(p).thermo_cells(torch.from_numpy(np.ascontiguousarray(inp.T)).cuda())
+    out = out.cpu().numpy()
+    err = np.abs(out[1] - ref[:, 1]) / (np.abs(ref[:, 0]) + np.abs(ref[:, 1]))
+    assert err.max() < 1e-12, (err.max(), T[np.nanargmax(err)])
+
+
 def test_thermo_gate_and_no_subcycling(gpu, orc):
     import torch
 

@@ -123,7 +123,8 @@ __device__ __forceinline__ double pow_t(const double* tab, double x, double y) {
     return __builtin_fma(e, x2, e);
 }
 
-// 1/x for a normal x of magnitude 2^-900 .. 2^900, within one ulp: the
+// 1/x for a normal x of magnitude 2^-900 .. 2^900 (T within 1e-100 .. 1e100
+// and its power 1.63), within one ulp: the
 // hardware reciprocal and two Newton steps
 __device__ __forceinline__ double rcp_t(double x) {
     double r = __builtin_amdgcn_rcp(x);
@@ -218,6 +219,29 @@ __device__ __forceinline__ CoolingCell cooling_cell(const ThermoConsts& t, const
     return c;
 }
 
+// subtract_cooling where its shared forms end: outside 1e-100 .. 1e100 K a
+// reciprocal, a square or e^(1.63 ln T) leaves the double range and meets its
+// opposite as 0 x infinity.  Each term by its own exponential, whose exponent
+// is clamped where the result is 0 or infinity anyway.
+__device__ __forceinline__ double subtract_cooling_far(const ThermoConsts& t, const CoolingCell& c, const double* tab,
+                                                       double rate, double T) {
+    if (!(T > 0.0)) return T == 0.0 ? rate : __builtin_nan("");  // all terms vanish towards 0; no rate below it, or of NaN
+    if (T > 0x1.fffffffffffffp1023) return rate - c.imlc_k - c.nmlc_k - c.nmc_k * T;
+    const double iT = 1.0 / T;
+    double hi, lo;
+    log_t(tab, T, hi, lo);
+    const double ln = hi + lo, a1 = t.T2 * iT, a2 = t.T4 * iT, a3 = T * t.icxhi;
+    rate -= c.imlc_k * exp_any(tab, -t.T1 * iT - a1 * a1);
+    rate -= c.nmlc_k * exp_any(tab, -t.T3 * iT - a2 * a2);
+    rate -= c.cehi_k * exp_any(tab, 2.302585093 * log_spline_t(t, tab, hi, lo) - a3 * a3);
+    if (T > t.ciec_minT) {
+        const double p163 = exp_any(tab, 1.63 * (ln - 11.512925464970228420));
+        const double smoothing = (T - 5.0e4) / 2.0e4;
+        rate -= c.ciec_k * exp_any(tab, -0.63 * ln) * (1.0 - exp_any(tab, -p163)) * (smoothing < 1.0 ? smoothing : 1.0);
+    }
+    return rate - c.nmc_k * exp_any(tab, 0.5 * ln - c.nmc_T0 * iT);
+}
+
 // Sum of the five cooling terms, subtracted in the reference's order from
 // `rate` (Thermodynamics.cpp:255-259 / 315-319).  The transcendental work is
 // shared between the terms: one reciprocal and one natural log of T feed
@@ -229,12 +253,7 @@ __device__ __forceinline__ CoolingCell cooling_cell(const ThermoConsts& t, const
 // term).
 __device__ __forceinline__ double subtract_cooling(const ThermoConsts& t, const CoolingCell& c, const double* tab,
                                                    double rate, double T) {
-    if (!(T >= 1e-280 && T <= 1e280)) {
-        // every term underflows towards T = 0; the last one grows as sqrt(T)
-        // at infinity; negative and NaN temperatures have no rate
-        if (T >= 0.0) return T <= 1.0 ? rate : rate - c.nmc_k * sqrt(T);
-        return __builtin_nan("");
-    }
+    if (!(T >= 1e-100 && T <= 1e100)) return subtract_cooling_far(t, c, tab, rate, T);
     const double iT = rcp_t(T);
     double hi, lo;
     log_t(tab, T, hi, lo);
