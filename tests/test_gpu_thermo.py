@@ -129,6 +129,27 @@ def test_cooling_rate_of_extreme_temperatures(gpu, orc):
     assert err.max() < 1e-12, (err.max(), T[np.nanargmax(err)])
 
 
+def test_infinite_rate_lands_softly(gpu, orc):
+    """A cooling rate that overflows stays -inf within 200 K of the floor (as a
+    division by 200 leaves it), and its subcycle count is refused."""
+    import torch
+
+    c = orc.converter(1e-20, 1e-28, 1e11)
+    t = orc.thermo_params(c, subcycling=False)
+    inp = np.zeros((64, 9))
+    T = np.linspace(110.0, 500.0, 64)
+    inp[:, 0], inp[:, 2], inp[:, 3], inp[:, 5], inp[:, 8] = 1e147, 0.5, 1.0, 100.0, 1e-3
+    inp[:, 1] = inp[:, 0] * t.spec_gas_const * 1.5 * T
+    inp[:, 4] = inp[:, 1] / (1.67 - 1.0)
+    ref = orc.thermo_batch(t, inp, nthreads=1)
+    assert (ref[:, 1] == -np.inf).all()
+    dev = torch.from_numpy(np.ascontiguousarray(inp.T)).cuda()
+    out, _ = _cooling(gpu, pfloor=t.pfloor, subcycling=False).thermo_cells(dev)
+    np.testing.assert_array_equal(out[1].cpu().numpy(), ref[:, 1])
+    with pytest.raises(gpu.TorchGpuError):
+        _cooling(gpu, pfloor=t.pfloor).thermo_cells(dev)
+
+
 def test_thermo_gate_and_no_subcycling(gpu, orc):
     import torch
 

@@ -187,9 +187,11 @@ __device__ __forceinline__ double soft_landing(double rate, double T, double T_m
     if (rate < 0.0) {
         if (T <= T_min) result = 0;
         else if (T <= T_min + 200) {
-            // rate (T - T_min) / 200, rounded as the division rounds it
+            // rate (T - T_min) / 200, rounded as the division rounds it; the
+            // correction of an infinite q is NaN
             const double x = rate * (T - T_min), q = x * 0.005;
-            result = __builtin_fma(__builtin_fma(-200.0, q, x), 0.005, q);
+            const double r = __builtin_fma(__builtin_fma(-200.0, q, x), 0.005, q);
+            result = r == r ? r : q;
         }
     }
     return result;
