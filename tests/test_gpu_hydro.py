@@ -77,6 +77,32 @@ def test_solver_limiter_variants_ragged_grid(gpu, orc, solver, limiter, order):
     np.testing.assert_array_equal(Ug, Uo)
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("solver", ["HLL", "HLLC", "RotatedHLLC"])
+def test_negative_face_pressure_raises(gpu, orc, solver, precision, axis):
+    """maxmod takes the larger of two one-sided slopes, which a pressure jump of
+    1 to 1,000 carries below zero at the face before it: the square of the sound
+    speed there is negative and the flux is NaN, which the reference throws on
+    and every solver of either precision reports."""
+    Q = np.zeros((7, 12, 12, 12))
+    Q[0], Q[1] = 1.0, 1.0
+    Q[2], Q[3] = 0.5, 1.0
+    P = np.moveaxis(Q[1], 2 - axis, 0)
+    P[6], P[7:] = 1.1, 1000.0
+    kw = dict(solver=solver, limiter="maxmod")
+    p = _oparams(orc, (12, 12, 12), dx=1.0 / 12, **kw)
+    with pytest.raises(RuntimeError) as e:
+        orc.run_hydro(p, _u0(orc, p, Q), 1)
+    assert "code 1" in str(e.value)
+    g = _grid(gpu, (12, 12, 12), precision=gpu.MIXED if precision == "mixed" else gpu.FP64, **kw)
+    g.set_primitive(Q)
+    g.run(1)
+    with pytest.raises(gpu.TorchGpuError) as ge:
+        g.synchronize()
+    assert ge.value.code == 3, ge.value
+
+
 # sizes on both sides of the two FP64 layouts' rule (8 x 4 x 4 tiles below about
 # a quarter of a million cells, 16 x 16 columns marched along z above), none a
 # multiple of a tile, a column or a column's planes

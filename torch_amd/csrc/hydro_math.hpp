@@ -534,7 +534,8 @@ struct NormalFlux {
 __device__ __forceinline__ NormalFlux hll_f(const SideF& L, const SideF& R, const RoeF& r, float unl, float unr,
                                             float g2) {
     const float ut = (L.sr * unl + R.sr * unr) * r.is, du = unr - unl;
-    const float d = fsqrt(fmaxf(r.base2 + r.nu2 * du * du, 1.0e-37f));
+    const float d2 = r.base2 + r.nu2 * du * du;
+    const float d = fsqrt(fmaxf(d2, 1.0e-37f));
     const float S_l = ut - d, S_r = ut + d;
     const float wr = __builtin_amdgcn_fmed3f(S_r * frcp(S_r - S_l), 0.f, 1.f), wl = 1.f - wr;
     NormalFlux f;
@@ -543,7 +544,7 @@ __device__ __forceinline__ NormalFlux hll_f(const SideF& L, const SideF& R, cons
     f.s = fminf(S_l, 0.f) * wr;
     f.c = wr * L.p + wl * R.p;
     f.e = f.hl * (g2 * L.p + L.ke) + f.hr * (g2 * R.p + R.ke) + f.s * (R.E - L.E);
-    f.nan = !(fabsf(ut) + d < INFINITY);  // the limits above drop a NaN
+    f.nan = !(d2 >= 0.f && fabsf(ut) + d < INFINITY);  // the limits above drop a NaN and a negative square
     return f;
 }
 
