@@ -103,6 +103,34 @@ def test_negative_face_pressure_raises(gpu, orc, solver, precision, axis):
     assert ge.value.code == 3, ge.value
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_pure_hll_face_of_negative_pressure(gpu, orc, precision, axis):
+    """As above, with two streams meeting along the axis at the jump: the
+    rotated solver's normal is the axis, so its HLL solve, whose squared sound
+    speed the velocity jump keeps positive, is all the face takes.  The mixed
+    fluxes are sums of FP32 terms of the momentum flux's size (6^2 + 10 against
+    a state of up to 34): 1e-4 of the largest value after two steps."""
+    Q = np.zeros((7, 12, 12, 12))
+    Q[0], Q[1] = 1.0, 1.0
+    Q[2], Q[3] = 0.5, 1.0
+    P, V = (np.moveaxis(Q[v], 2 - axis, 0) for v in (1, 4 + axis))
+    P[6], P[7:] = 1.1, 10.0
+    V[:6], V[6:] = 6.0, -6.0
+    kw = dict(limiter="maxmod")
+    p = _oparams(orc, (12, 12, 12), dx=1.0 / 12, **kw)
+    ref, _, _ = orc.run_hydro(p, _u0(orc, p, Q), 2)
+    g = _grid(gpu, (12, 12, 12), precision=gpu.MIXED if precision == "mixed" else gpu.FP64, **kw)
+    g.set_primitive(Q)
+    g.run(2)
+    g.synchronize()
+    U = g.get_conserved()
+    if precision == "fp64":
+        np.testing.assert_array_equal(U, ref)
+    else:
+        assert np.abs(U - ref).max() < 1e-4 * np.abs(ref).max()
+
+
 # sizes on both sides of the two FP64 layouts' rule (8 x 4 x 4 tiles below about
 # a quarter of a million cells, 16 x 16 columns marched along z above), none a
 # multiple of a tile, a column or a column's planes

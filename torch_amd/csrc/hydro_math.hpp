@@ -608,11 +608,14 @@ __device__ __forceinline__ bool riemann_f(float F[7], const float* Ql, const flo
         nd = axis ? 1.f : nd * in;
         const float is = __builtin_amdgcn_rsqf(s2);
         // n2 = s d - k (nA, nB), and its weight s; pure HLL: s = 0, and the
-        // solve at rest whose result has no weight stays finite
+        // solve whose result has no weight is at rest with a sound speed of 1,
+        // finite whatever the states
+        RoeF r2 = r;
+        r2.base2 = axis && !small ? 1.f : r.base2;
         const float s = axis ? (small ? 1.f : 0.f) : s2 * is, k = axis ? 0.f : nd * is;
         const float ql = L.v[A] * nA + L.v[B] * nB, qr = R.v[A] * nA + R.v[B] * nB;
         const NormalFlux f1 = hll_f(L, R, r, nd * L.v[DIM] + ql, nd * R.v[DIM] + qr, c.g2);
-        const NormalFlux f2 = hllc_f(L, R, r, s * L.v[DIM] - k * ql, s * R.v[DIM] - k * qr);
+        const NormalFlux f2 = hllc_f(L, R, r2, s * L.v[DIM] - k * ql, s * R.v[DIM] - k * qr);
         const float w1 = small ? 0.f : nd;
         hl = w1 * f1.hl + s * f2.hl;
         hr = w1 * f1.hr + s * f2.hr;
