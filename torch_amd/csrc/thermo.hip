@@ -1207,8 +1207,10 @@ int ensure_fallback(torchgpu_cooling* c, long long n) {
 }
 
 int ensure_queues(torchgpu_cooling* c, long long n) {
-    if (n <= c->cap) return TORCHGPU_OK;
-    int rc;
+    // the fallback queue has a capacity of its own: the FP64 grid step grows
+    // it too, and may have lost it in trying
+    const int rc = ensure_fallback(c, n);
+    if (rc || n <= c->cap) return rc;
     (void)hipStreamSynchronize(c->stream);
     if (c->mlp_list) (void)hipFree(c->mlp_list);
     if (c->long_list) (void)hipFree(c->long_list);
@@ -1220,7 +1222,6 @@ int ensure_queues(torchgpu_cooling* c, long long n) {
     c->sdata = nullptr;
     c->cap = 0;
     HIP_OK(hipMalloc(&c->mlp_list, n * sizeof(long long)));
-    if ((rc = ensure_fallback(c, n))) return rc;
     HIP_OK(hipMalloc(&c->long_list, n * sizeof(long long)));
     HIP_OK(hipMalloc(&c->feat, n * 8 * sizeof(float)));
     HIP_OK(hipMalloc(&c->y, n * 3 * sizeof(float)));
