@@ -1,12 +1,14 @@
 """The mixed-precision kernel evaluates the rotated hybrid HLLC-HLL flux
 without rotation matrices (hydro_math.hpp, riemann_f): solving along a unit
-normal n in the original frame with u_n = v.n, and n2 = (d - n1_d n1) / s.
-This test restates that formulation in float64 numpy and checks it against
-the oracle's literal rotate-solve-rotate-back solver
-(Riemann.cpp:154-244) on the reference-derived KAT inputs of
-tests/golden/riemann.npz: the two must agree to rounding (the identity is
-exact in real arithmetic), so a wrong sign of n2, a dropped p n term in the
-momentum flux or a wrong star-state velocity fails it."""
+normal n in the original frame with u_n = v.n, and n2 = (d - n1_d n1) / s; and
+it sums the two solvers' fluxes as scalars (NormalFlux: a mass flux per side, a
+conserved jump, a pressure term along the normal and the energy flux) before it
+forms the one flux vector.  This test restates that in float64 numpy, the
+combination line for line, and checks it against the oracle's literal
+rotate-solve-rotate-back solver (Riemann.cpp:154-244) on the
+reference-derived KAT inputs of tests/golden/riemann.npz: the two must agree
+to rounding (the identity is exact in real arithmetic), so a wrong sign of n2,
+a dropped pressure term or jump, or a wrong star-state velocity fails it."""
 import os
 
 import numpy as np
@@ -25,27 +27,6 @@ def _side(q, g):
                 E=p / (g - 1.0) + ke)
 
 
-def _flux(s, un, n, g2):
-    m = s["rho"] * un
-    F = np.empty((un.shape[0], 7))
-    F[:, DEN] = m
-    F[:, PRE] = un * (g2 * s["p"] + s["ke"])
-    F[:, HII] = m * s["x"]
-    F[:, ADV] = m * s["a"]
-    F[:, VEL:] = m[:, None] * s["v"] + s["p"][:, None] * n
-    return F
-
-
-def _cons(s):
-    U = np.empty((s["rho"].shape[0], 7))
-    U[:, DEN] = s["rho"]
-    U[:, PRE] = s["E"]
-    U[:, HII] = s["rho"] * s["x"]
-    U[:, ADV] = s["rho"] * s["a"]
-    U[:, VEL:] = s["rho"][:, None] * s["v"]
-    return U
-
-
 def _speeds(L, R, unl, unr):
     is_ = 1.0 / (L["sr"] + R["sr"])
     ut = (L["sr"] * unl + R["sr"] * unr) * is_
@@ -53,70 +34,76 @@ def _speeds(L, R, unl, unr):
     return ut - d, ut + d
 
 
-def _hll(L, R, n, g2):
-    unl, unr = (L["v"] * n).sum(1), (R["v"] * n).sum(1)
+def _hll(L, R, unl, unr, g2):
+    """(hl, hr, s, c, e) of the HLL flux along a normal."""
     Sl, Sr = _speeds(L, R, unl, unr)
-    Fl, Fr = _flux(L, unl, n, g2), _flux(R, unr, n, g2)
-    Ul, Ur = _cons(L), _cons(R)
-    with np.errstate(all="ignore"):
-        Fh = (Sr[:, None] * Fl - Sl[:, None] * Fr + (Sl * Sr)[:, None] * (Ur - Ul)) / (Sr - Sl)[:, None]
-    return np.where((Sr <= 0)[:, None], Fr, np.where((Sl >= 0)[:, None], Fl, Fh))
+    wr = np.clip(Sr / (Sr - Sl), 0.0, 1.0)
+    wl = 1.0 - wr
+    hl, hr, s = wr * unl, wl * unr, np.minimum(Sl, 0.0) * wr
+    e = hl * (g2 * L["p"] + L["ke"]) + hr * (g2 * R["p"] + R["ke"]) + s * (R["E"] - L["E"])
+    return hl, hr, s, wr * L["p"] + wl * R["p"], e
 
 
-def _hllc(L, R, n, g2):
-    unl, unr = (L["v"] * n).sum(1), (R["v"] * n).sum(1)
+def _hllc(L, R, unl, unr, g2):
     Sl, Sr = _speeds(L, R, unl, unr)
     wl, wr = L["rho"] * (Sl - unl), R["rho"] * (Sr - unr)
-    with np.errstate(all="ignore"):
-        Sc = (R["p"] - L["p"] + wl * unl - wr * unr) / (wl - wr)
+    Sc = (R["p"] - L["p"] + wl * unl - wr * unr) / (wl - wr)
     sub = ~(Sl >= 0) & ~(Sr <= 0)
     left = (Sl >= 0) | (sub & (Sc >= 0))
-    K = {k: np.where(left[:, None] if L[k].ndim == 2 else left, L[k], R[k]) for k in L}
-    un = np.where(left, unl, unr)
-    S = np.where(left, Sl, Sr)
-    F = _flux(K, un, n, g2)
-    with np.errstate(all="ignore"):
-        w = S - un
-        A = K["rho"] * w / (S - Sc)
-        dsc = Sc - un
-        dU = np.empty_like(F)
-        dU[:, DEN] = A - K["rho"]
-        dU[:, PRE] = A * (K["E"] / K["rho"] + dsc * (Sc + K["p"] / (K["rho"] * w))) - K["E"]
-        dU[:, HII] = (A - K["rho"]) * K["x"]
-        dU[:, ADV] = (A - K["rho"]) * K["a"]
-        dU[:, VEL:] = A[:, None] * (K["v"] + dsc[:, None] * n) - K["rho"][:, None] * K["v"]
-        Fs = F + S[:, None] * dU
-    return np.where(sub[:, None], Fs, F)
+    rho, p, E = (np.where(left, L[k], R[k]) for k in ("rho", "p", "E"))
+    un, S = np.where(left, unl, unr), np.where(left, Sl, Sr)
+    iss = np.where(sub, 1.0 / np.where(sub, S - Sc, 1.0), 0.0)
+    wi = (S - un) * iss
+    t = np.where(sub, wi * Sc, un)
+    dsc = np.where(sub, Sc - un, 0.0)
+    sd = S * dsc
+    e = t * E + p * (un + sd * iss) + sd * (rho * t)
+    return np.where(left, t, 0.0), np.where(left, 0.0, t), np.zeros_like(t), p + sd * (rho * wi), e
 
 
-def rotation_free(Ql, Qr, dims, g):
-    """Rotated hybrid flux along axis dims[i] of each face, rotation-free."""
+def normal_flux(solver, Ql, Qr, dims, g):
+    """Flux along axis dims[i] of each face as riemann_f forms it."""
     L, R = _side(Ql, g), _side(Qr, g)
     g2 = g / (g - 1.0)
-    n = Ql.shape[0]
-    d = np.zeros((n, 3))
-    d[np.arange(n), dims] = 1.0
-    n1 = R["v"] - L["v"]
-    n1d = n1[np.arange(n), dims]
-    n1 = np.where((n1d < 0)[:, None], -n1, n1)
-    nn = (n1 * n1).sum(1)
-    pure_hllc = np.sqrt(nn) < 1e-6
-    with np.errstate(all="ignore"):
-        n1 = n1 / np.sqrt(nn)[:, None]
-        n1d = n1[np.arange(n), dims]
-        s2 = (n1 * n1).sum(1) - n1d * n1d
-        s2 = np.maximum(s2, 0.0)
-        pure_hll = ~pure_hllc & (s2 == 0)
-        s = np.sqrt(s2)
-        n2 = (d - n1d[:, None] * n1) / s[:, None]
-    hyb = ~pure_hllc & ~pure_hll
-    n1s = np.where(hyb[:, None], n1, d)
-    n2s = np.where(hyb[:, None], n2, d)
-    F1 = _hll(L, R, n1s, g2)
-    F2 = _hllc(L, R, n2s, g2)
-    Fh = n1d[:, None] * F1 + s[:, None] * F2
-    out = np.where(pure_hllc[:, None], _hllc(L, R, d, g2), np.where(pure_hll[:, None], _hll(L, R, d, g2), Fh))
-    return out
+    i = np.arange(Ql.shape[0])
+    D, A, B = dims, np.where(dims == 0, 1, 0), np.where(dims == 2, 1, 2)
+    lv, rv = L["v"], R["v"]
+    zero = np.zeros(i.size)
+    nA = nB = ct = zero
+    if solver != "RotatedHLLC":
+        hl, hr, sj, cd, e = (_hll if solver == "HLL" else _hllc)(L, R, lv[i, D], rv[i, D], g2)
+    else:
+        nd, nA, nB = (rv[i, X] - lv[i, X] for X in (D, A, B))
+        nn = nd * nd + nA * nA + nB * nB
+        small = nn < 1.0e-12
+        n = np.where(small, 0.0, np.copysign(1.0 / np.sqrt(np.where(small, 1.0, nn)), nd))
+        nA, nB = nA * n, nB * n
+        s2 = nA * nA + nB * nB
+        axis = s2 == 0.0
+        nd = np.where(axis, 1.0, nd * n)
+        is_ = 1.0 / np.sqrt(np.where(axis, 1.0, s2))
+        s = np.where(axis, np.where(small, 1.0, 0.0), s2 * is_)
+        k = np.where(axis, 0.0, nd * is_)
+        ql, qr = lv[i, A] * nA + lv[i, B] * nB, rv[i, A] * nA + rv[i, B] * nB
+        f1 = _hll(L, R, nd * lv[i, D] + ql, nd * rv[i, D] + qr, g2)
+        f2 = _hllc(L, R, s * lv[i, D] - k * ql, s * rv[i, D] - k * qr, g2)
+        w1 = np.where(small, 0.0, nd)
+        hl, hr, sj = w1 * f1[0] + s * f2[0], w1 * f1[1] + s * f2[1], w1 * f1[2]
+        e = w1 * f1[4] + s * f2[4]
+        c1, c2 = w1 * f1[3], s * f2[3]
+        cd, ct = c1 * nd + c2 * s, c1 - c2 * k
+    ml, mr = L["rho"] * hl, R["rho"] * hr
+
+    def flux(l, r, c=zero):
+        return ml * l + (mr * r + (sj * (R["rho"] * r - L["rho"] * l) + c))
+
+    F = np.empty((i.size, 7))
+    F[:, DEN] = ml + mr + sj * (R["rho"] - L["rho"])
+    F[:, PRE] = e
+    F[:, HII], F[:, ADV] = flux(L["x"], R["x"]), flux(L["a"], R["a"])
+    for X, c in ((D, cd), (A, ct * nA), (B, ct * nB)):
+        F[i, VEL + X] = flux(lv[i, X], rv[i, X], c)
+    return F
 
 
 @pytest.mark.parametrize("solver", ["RotatedHLLC", "HLL", "HLLC"])
@@ -125,16 +112,7 @@ def test_rotation_free_matches_rotated_solver(solver):
     Ql, Qr, dims, g = f["Ql"], f["Qr"], f["dims"].astype(int), float(f["gamma"])
     ref, st = oracle.riemann(solver, Ql, Qr, dims, g)
     ok = st == 0
-    L, R = _side(Ql, g), _side(Qr, g)
-    n = Ql.shape[0]
-    d = np.zeros((n, 3))
-    d[np.arange(n), dims] = 1.0
-    if solver == "RotatedHLLC":
-        got = rotation_free(Ql, Qr, dims, g)
-    elif solver == "HLL":
-        got = _hll(L, R, d, g / (g - 1.0))
-    else:
-        got = _hllc(L, R, d, g / (g - 1.0))
+    got = normal_flux(solver, Ql, Qr, dims, g)
     # relative to the face's flux scale (momentum flux ~ p + rho v^2)
     scale = np.abs(ref[ok]).max(1, keepdims=True) + 1e-300
     err = np.abs(got[ok] - ref[ok]) / scale
