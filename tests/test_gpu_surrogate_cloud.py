@@ -78,14 +78,17 @@ def test_cloud_grid_at_100x_dt_goes_to_the_network(gpu):
     del mlp
 
 
-@pytest.mark.skipif(not os.path.exists(WEIGHTS), reason="cloud surrogate weights not trained yet")
-def test_grid_substep_forms_inputs_in_the_prepass(gpu):
-    """A surrogate thermo sub-step on the grid forms each cell's inputs in the
-    prepass from U (writing the gathered array only for the cells it queues);
-    with the heating record on it gathers the whole array first.  Both give
-    the same state bit for bit (mixed and FP64 grids), at the loop's dt and
-    at 100x it, where cells go to the network and the FP64 fallback, and the
-    thermo time step agrees too."""
+@pytest.mark.parametrize("surrogate", [
+    pytest.param(True, marks=pytest.mark.skipif(not os.path.exists(WEIGHTS),
+                                                reason="cloud surrogate weights not trained yet")), False])
+def test_grid_substep_forms_inputs_in_the_prepass(gpu, surrogate):
+    """A thermo sub-step on the grid forms each cell's inputs in the prepass
+    from U (writing the gathered array only for the cells it queues); with the
+    heating record on it gathers the whole array first.  Both give the same
+    state bit for bit (mixed and FP64 grids), at the loop's dt and at 100x it,
+    where cells are queued (for the network and the FP64 fallback, or, more
+    than 8 subcycles, for the FP64 integrator), and the thermo time step agrees
+    too."""
     import torch
 
     from torch_amd import cloud
@@ -97,13 +100,16 @@ def test_grid_substep_forms_inputs_in_the_prepass(gpu):
             p, g, cool, thermo = cloud.build(48, precision)
             if track:
                 g.heating_track(True)
-            mlp = sg.attach(cool, WEIGHTS, gate=0.01)
-            cool.run_split(g, 6, surrogate=True, **thermo)
+            mlp = sg.attach(cool, WEIGHTS, gate=0.01) if surrogate else None
+            cool.run_split(g, 6, surrogate=surrogate, **thermo)
             g.synchronize()
             t, dt, _ = g.clock()
             dts.append(cool.grid_timestep(g, p.dt_max, **thermo))
+            inp = cloud.cooling_inputs(g, p, thermo["col_den"], thermo["F_FUV"], thermo["excluded"], 100.0 * dt)
+            steps = sg.subcycles(cool, inp)
+            assert int((steps > 8).sum()) > 100 and int((steps <= 8).sum()) > 100
             for mult in (1.0, 100.0):
-                cool.grid_substep(g, mult * dt, surrogate=True, **thermo)
+                cool.grid_substep(g, mult * dt, surrogate=surrogate, **thermo)
             g.stage_dt(0, 0.5 * dt)   # a hydro sub-step on the float Q the cooling wrote
             g.synchronize()
             states.append(g.get_conserved())
