@@ -1381,7 +1381,7 @@ int torchgpu_cooling_set_surrogate(torchgpu_cooling* c, torchgpu_mlp* m, const t
 }  // extern "C"
 
 // Where a grid surrogate step writes the cooling update of the cells its
-// prepass finishes (surrogate_prepass_kernel<true, true>): the state, its float Q
+// prepass finishes (surrogate_prepass_kernel<true, ...>): the state, its float Q
 // (NULL for FP64 grids) and the step state.
 struct ApplyDst {
     double* U;
@@ -1391,12 +1391,13 @@ struct ApplyDst {
 };
 
 // The FP64 step on the grid state: as the surrogate's, with every cell past
-// SHORT_STEPS subcycles integrated by the persistent kernel.
+// SHORT_STEPS subcycles integrated by the persistent kernel (the caller has
+// seen to the fallback queue).
 static int fp64_grid_step(torchgpu_cooling* c, int64_t n, double* in, double* out, uint8_t* path, const tg::GridSrc& gs,
                           const ApplyDst& apply) {
     if (n == 0) return TORCHGPU_OK;
-    int rc = ensure_fallback(c, n);
-    if (rc || (rc = zero_counters(c))) return rc;
+    int rc = zero_counters(c);
+    if (rc) return rc;
     tg::SurrogateConsts sc{};
     sc.nexact = tg::SHORT_STEPS;
     long long nb = (n + 255) / 256;
@@ -1584,30 +1585,35 @@ static int gather(torchgpu_cooling* c, torchgpu_ctx* ctx, const double* T_min, c
 // of min |f E/RATE| over the gated cells, 0x7fef... when none), no host sync.
 // The thermo time step of the grid state; with cfl_st, the kernel also
 // reduces the hydro CFL maximum of the same state (launch_cfl's); with
-// keep_rate, it keeps each cell's heating rate and pre-step RATE in
-// c->rcache for a cooling sub-step that follows on the same state.
+// *keep_rate, it keeps each cell's heating rate and pre-step RATE in
+// c->rcache for a cooling sub-step that follows on the same state, or clears
+// the flag where there is no memory for them.
 static int grid_timestep_dev(torchgpu_ctx* ctx, torchgpu_cooling* c, const double* T_min, const double* col_den,
                              const double* F, int64_t excluded, tg::StepState* cfl_st = nullptr,
-                             bool keep_rate = false) {
+                             bool* keep_rate = nullptr) {
     // the inputs are formed in the kernel
     tg::GridSrc gs;
     int rc = grid_src(c, ctx, T_min, col_den, F, excluded, 0.0, gs);
     if (rc) return rc;
     const long long n = tg::ctx_view(ctx).g->ncell;
-    if (keep_rate && n > c->rcache_cap) {
+    if (keep_rate && *keep_rate && n > c->rcache_cap) {
         (void)hipStreamSynchronize(c->stream);
         if (c->rcache) (void)hipFree(c->rcache);
         c->rcache = nullptr;
         c->rcache_cap = 0;
-        HIP_OK(hipMalloc(&c->rcache, 2 * n * sizeof(double)));
-        c->rcache_cap = n;
+        if (hipMalloc(&c->rcache, 2 * n * sizeof(double)) == hipSuccess) {
+            c->rcache_cap = n;
+        } else {
+            (void)hipGetLastError();
+            *keep_rate = false;
+        }
     }
     hipLaunchKernelGGL(tg::set_u64_kernel, dim3(1), dim3(1), 0, c->stream, c->dtbits, 0x7fefffffffffffffull);
     long long nb = (n + 255) / 256;
     if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
     hipLaunchKernelGGL(tg::thermo_timestep_kernel<true>, dim3((unsigned)nb), dim3(256), 0, c->stream, c->t,
                        c->tables, n, (const double*)nullptr, c->dtbits, c->err, gs, cfl_st,
-                       keep_rate ? c->rcache : (double*)nullptr);
+                       keep_rate && *keep_rate ? c->rcache : (double*)nullptr);
     HIP_OK(hipGetLastError());
     return TORCHGPU_OK;
 }
@@ -1623,8 +1629,13 @@ static int grid_substep_dev(torchgpu_ctx* ctx, torchgpu_cooling* c, const double
     // (Thermodynamics::updateSourceTerms + advSolution(dt) + fixSolution) to
     // the cells it finishes (the queued cells get it once the network and the
     // integrator have run), unless the heating record needs the gathered array
-    const bool direct = !(v.heat && c->t.subcycling);
+    // or there is no memory for the FP64 step's queue
+    bool direct = !(v.heat && c->t.subcycling);
     int rc;
+    if (direct && !surrogate && ensure_fallback(c, n)) {
+        (void)hipGetLastError();
+        direct = false;
+    }
     if (direct) {
         tg::GridSrc gs;
         if ((rc = grid_src(c, ctx, T_min, col_den, F, excluded, dt, gs))) return rc;
@@ -1900,8 +1911,9 @@ int torchgpu_run_full(torchgpu_ctx* ctx, torchgpu_cooling* c, torchgpu_radiation
         // which sees the same state (not with radiation, whose pre-step
         // comes in between, nor where the heating record has the inputs
         // gathered)
-        const bool share = c && !r && !(v.heat && c->t.subcycling) && order_first(comps, ncomps, (launched + 1) % ncomps) == THERMO;
-        if (c && (rc = grid_timestep_dev(ctx, c, T_min, col_den, F, excluded, v.st, share))) return rc;
+        bool share = c && !r && !(v.heat && c->t.subcycling) &&
+                     order_first(comps, ncomps, (launched + 1) % ncomps) == THERMO;
+        if (c && (rc = grid_timestep_dev(ctx, c, T_min, col_den, F, excluded, v.st, &share))) return rc;
         if (r && ((rc = tg::rad_pre_step_dev(r, 1)) || (rc = tg::rad_timestep_dev(r, 0.0, 1)))) return rc;
         HIP_OK(tg::launch_step_begin(v.st, 1, 0.0, v.stream, c ? c->dtbits : nullptr,
                                      r ? tg::rad_dt_bits(r) : nullptr));
