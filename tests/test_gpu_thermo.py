@@ -1,7 +1,8 @@
 """GPU subcycled cooling step against the reference fixtures and the oracle.
 
-The GPU uses the device math library (ocml) for exp/log/log10/pow/sqrt, the
-reference glibc's; agreement is therefore to a tolerance, stated per test."""
+The GPU's rates use table-driven exp, log and pow (thermo_math.hpp), within an
+ulp, and the reference glibc's; agreement is therefore to a tolerance, stated
+per test."""
 import os
 
 import numpy as np

@@ -495,8 +495,9 @@ __device__ __forceinline__ void march_column(const HydroGeom& g, MarchLDS& s, co
 
 template <int SOLVER, bool ALB, int STAGE, bool A32>
 // Four waves per SIMD (128 VGPRs; the 33 KB of LDS allow four workgroups
-// per CU): about 20 registers spill, which measured faster than three waves
-// per SIMD without spills (14.9 against 16.7 ms per 512^3 step).
+// per CU): 3 or 4 registers spill (up to 18 with 64-bit offsets).  With about
+// 20 spilled, four waves were faster than three per SIMD without spills (14.9
+// against 16.7 ms per 512^3 step).
 __global__ __launch_bounds__(MTHREADS) __attribute__((amdgpu_waves_per_eu(4))) void hydro_stage_mixed_kernel(HydroGeom g, int mtx, int mty, int mtz, int mz,
                                                                      const float* __restrict__ qin, const double* Ubase,
                                                                      double* Udst, float* __restrict__ qout,
@@ -567,7 +568,11 @@ __global__ __launch_bounds__(MTHREADS) __attribute__((amdgpu_waves_per_eu(4))) v
 // about 0.3 of a round unfilled.  Pieces of 2 .. 32 planes.  Us per step (two
 // stages) with 16 planes always, and so: 16^3 217 / 44; 64^3 225 / 71;
 // 96^3 234 / 128; 128^3 284 / 235; 150x97x118 308 / 249; 205x173x190 853 / 851;
-// 256^3 1,690 / 1,684.
+// 256^3 1,690 / 1,684.  On large grids the count hardly matters; 8 / 16 / 32
+// planes and the rule's own choice (32 at 512^3 and 384^3): 320^3 3,350 / 3,155
+// / 3,180 / 3,190; 500x300x400 6,610 / 6,270 / 6,440 / 6,060 (25); 384^3 5,710 /
+// 5,370 / 5,360 / 5,370; 512^3 13,300 / 12,560 / 12,610 / 12,590 (runs differ by
+// 0.3 %).
 static int march_planes(const HydroGeom& g) {
     const long long cols = (long long)((g.nx + MTX - 1) / MTX) * ((g.ny + MTY - 1) / MTY);
     int best_mz = g.nz < 16 ? g.nz : 16;

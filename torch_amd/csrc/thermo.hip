@@ -473,18 +473,17 @@ __device__ __forceinline__ void queue_cell(bool to_mlp, bool to_fb, long long ce
 // the deferred list, the others to its back.
 constexpr int COARSE_LONG = 64;
 
-// DEFER (long_list given): every cell routed to the network or the fallback
-// is queued in long_list instead, for surrogate_long_kernel, which estimates
-// its coarse end temperature (up to COARSE_STEPS iterations of two rate
-// evaluations) with every lane of a wave on such a cell; inline, one long
-// cell in a wave keeps its other 63 lanes idle, and the estimate's registers
-// would bound this kernel's occupancy.  Without DEFER (the training data)
-// the routing is done here.  The GRID instance (which also forms the inputs
-// and applies the update) runs at three waves per SIMD with a few spilled
-// registers: measured faster than two without spills and four with ~50.
-//
-// FALLBACK (a grid's FP64 step): every cell past nexact goes to the fallback
-// list.
+// PRE_ROUTE (the training data): every cell past nexact is routed here, to the
+// network or the fallback.
+// PRE_DEFER (long_list given): such a cell is queued in long_list instead, for
+// surrogate_long_kernel, which estimates its coarse end temperature (up to
+// COARSE_STEPS iterations of two rate evaluations) with every lane of a wave
+// on such a cell; inline, one long cell in a wave keeps its other 63 lanes
+// idle, and the estimate's registers would bound this kernel's occupancy.
+// PRE_FALLBACK (a grid's FP64 step): it goes to the fallback list.
+// The GRID instances (which also form the inputs and apply the update) run at
+// three waves per SIMD, 160 registers without spills; two and four waves (7
+// spilled registers) measured slower.
 enum PrepassMode { PRE_ROUTE, PRE_DEFER, PRE_FALLBACK };
 template <bool GRID, PrepassMode MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 4))) void surrogate_prepass_kernel(ThermoConsts t, const double* __restrict__ tables,
@@ -1525,9 +1524,6 @@ static int ensure_grid(torchgpu_cooling* c, long long n) {
     HIP_OK(hipMalloc(&c->in9, 9 * n * sizeof(double)));
     HIP_OK(hipMalloc(&c->out5, 5 * n * sizeof(double)));
     HIP_OK(hipMalloc(&c->gpath, n));
-    // finite contents everywhere: the ray trace reads columns of zero weight
-    hipLaunchKernelGGL(tg::zero_f64_kernel, dim3(1024), dim3(256), 0, c->stream, c->in9, 9 * n);
-    HIP_OK(hipGetLastError());
     if (!c->dtbits) HIP_OK(hipMalloc(&c->dtbits, sizeof(unsigned long long)));
     c->grid_cap = n;
     return TORCHGPU_OK;
