@@ -404,11 +404,12 @@ __device__ __forceinline__ void dstore_flux(ColumnLDS& s, int item, const double
 // workgroup that meets a cell or face out of their range ends before that
 // plane's update, having noted the plane in `resume`, and the instance with the full ones, launched
 // next, goes on from there (resume null: from the start), leaving at once
-// where nothing is left (4 us).  Us per step: 256^3 6,609 with full divisions
+// where nothing is left (4 us; 7 at 256^3, 27 at 512^3).  Us per step: 256^3 6,609 with full divisions
 // only, 5,715 so; 205x173x190 2,943 and 2,527; 128^3 864 and 750.  Both in one
 // kernel, chosen per plane, held 105 spilled registers and were slower than
 // full divisions alone (256^3 7,170).  What bounds the march is the latency of
-// its instruction stream: two waves per SIMD issue about half of the time.
+// its instruction stream: two waves per SIMD issue vector instructions 0.55 to
+// 0.63 of the time (3,800 per cell and stage).
 template <int SOLVER, bool ALB, int STAGE, bool FAST>
 __global__ __launch_bounds__(DTHREADS) __attribute__((amdgpu_waves_per_eu(2))) void hydro_march_kernel(
     HydroGeom g, int ntx, int nty, int ntz, int mz, const double* __restrict__ Usrc, const double* Ubase, double* Udst,

@@ -27,8 +27,9 @@
 // fixSolution, writes U, the float primitives of the output for the next
 // stage and (corrector) its CFL term.  34 KB LDS, 128 VGPRs: four waves per
 // SIMD, four workgroups per CU (neither the registers nor the LDS allow a
-// fifth).  Bound by vector instructions: 1,300 per cell and stage, issued on
-// four cycles of five (256^3, 0.8 ms per stage).
+// fifth).  Bound by vector instructions: 1,360 (predictor) and 1,440 per cell and
+// stage, issued 0.80 and 0.85 of the time at 512^3, 0.71 and 0.76 at 256^3 (0.8
+// ms per stage), and beside them the transcendentals' extra cycles.
 //
 // FP32 range: the float state is the FP64 state scaled by powers of two,
 // density by 2^kr and pressure by 2^kp with the grid's largest density and

@@ -32,10 +32,12 @@
 //                       weights into their fragments
 // A batch of 65,536 took 2,700 us per step as one tiled GEMM launch per
 // product with scalar operand loads, FP32 pre-activations in memory and a
-// serial sum of up to 1,024 bias partials per thread; it takes 156 us, the same
-// bits: every sum runs in that form's order.  (With the hardware exponential
-// and reciprocal in the SiLU, and sums in whatever order suits the launches, it
-// took 126 us, activations up to 1e-6 off and weights 5e-4 after four steps.)
+// serial sum of up to 1,024 bias partials per thread; it takes 156 us (101 in
+// the fused kernel, 38 in the weight gradients, 17 in the sums and Adam), the
+// same bits: every sum runs in that form's order.  With the hardware
+// exponential and reciprocal in the SiLU, and sums in whatever order suits the
+// launches, it took 126 us (87, 33, 13 in a trace), activations up to 1e-6 off and weights
+// 5e-4 after four steps.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -370,8 +372,8 @@ __device__ __forceinline__ void train_forward(const u32x4* w, const float* b, co
 // prediction (no gradient through it).  Eight waves share the forward
 // fragments in LDS; the backward ones, read once per 16 cells, come from L2
 // (both sets do not fit in 160 KB).  Bound by the SiLU's exponential and two
-// divisions per unit and the latency of those reads; at most one workgroup per
-// CU so that the 108 KB are staged once.
+// divisions per unit and the latency of those reads, 101 us for 65,536 cells; at
+// most one workgroup per CU so that the 108 KB are staged once.
 // 128 registers hold the SiLU derivatives of the four layers, which leaves
 // two waves per SIMD.
 __global__ __launch_bounds__(TRAIN_THREADS) void mlp_train_kernel(const bf16_t* __restrict__ packed,
@@ -487,7 +489,9 @@ __device__ __forceinline__ void output_sums(const TrainBuffers& tb, int blk, int
 // the first nz * WGRAD_JOBS, jobs 0 .. 11 a 64 x 64 quadrant of a 128 x 128
 // layer (32 x 32 per wave), jobs 12 and 13 half of the first and the output
 // layer; the workgroups past them sum the outputs of 256 cells each.  Bound
-// by the latency of the fragment reads, several blocks in flight per wave.
+// by the latency of the fragment reads, eight blocks in flight per wave: 38 us for
+// 65,536 cells (33 as 128 chunks of 64 x 64 tiles per wave, another order of
+// sums).
 // At most 32 chunks, whose sums are then added in order: a gradient is the
 // same however the batch is spread over the chip.
 constexpr int WGRAD_JOBS = 14, WGRAD_AHEAD = 8;
