@@ -84,8 +84,8 @@ def test_ray_trace_matches_oracle(gpu, shape, star, wind_r):
     in9b, dcolb = cool.grid_inputs(g)
     np.testing.assert_array_equal(in9b, in9)
     np.testing.assert_array_equal(dcolb, dcol)
-    # new densities set between calls (the x-face buffers hold the previous
-    # call's columns), each call against the oracle
+    # new densities set between calls (the columns hold the previous call's),
+    # each call against the oracle
     rng = np.random.default_rng(7)
     for rep in range(3):
         Q2 = Q.copy()
