@@ -62,7 +62,8 @@ struct CellState {
 // cell's heating rate and pre-step RATE as this function computed them on
 // the same state (pre_rate[pidx], pre_rate[pn + pidx]; thermo_timestep_kernel
 // stores them), taken instead of evaluating them again.
-__device__ __forceinline__ bool thermo_init(const ThermoConsts& t, const double* tab, const double* in, long long stride, long long cell,
+template <bool EVEN>
+__device__ __forceinline__ bool thermo_init(const RateConsts<EVEN>& t, const double* tab, const double* in, long long stride, long long cell,
                                             CellState& s, unsigned int* err, const double* pre_rate = nullptr,
                                             long long pidx = 0, long long pn = 0) {
     const double den = in[0 * stride + cell], pre = in[1 * stride + cell], hii = in[2 * stride + cell];
@@ -129,7 +130,8 @@ __device__ __forceinline__ bool thermo_init(const ThermoConsts& t, const double*
 }
 
 // One subcycle, :314-330.
-__device__ __forceinline__ void thermo_substep(const ThermoConsts& t, const double* tab, CellState& s) {
+template <bool EVEN>
+__device__ __forceinline__ void thermo_substep(const RateConsts<EVEN>& t, const double* tab, CellState& s) {
     double r = subtract_cooling(t, s.cc, tab, s.heat, s.subT);
     r = t.heating_amplification * soft_landing(r, s.subT, s.T_min);
     double pressure = s.pressure + r * s.rate2dpre;
@@ -191,7 +193,8 @@ __device__ __forceinline__ void load_spline(const double* __restrict__ tables, d
 
 // counters[0]: work counter; counters[1]: total subcycles.  Work items are
 // 0..count-1 (count = *count_dev when given), cell = order ? order[i] : i.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void thermo_cells_kernel(ThermoConsts t, const double* __restrict__ tables,
+template <bool EVEN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void thermo_cells_kernel(RateConsts<EVEN> t, const double* __restrict__ tables,
                                                           long long stride, long long count,
                                                           const unsigned long long* __restrict__ count_dev,
                                                           const long long* __restrict__ order,
@@ -278,7 +281,8 @@ __device__ __forceinline__ double residual_scale(long long nsub) { return 0.01 /
 
 // Rate of one subcycle step at temperature T (Thermodynamics.cpp:314-320),
 // as dp per subcycle.
-__device__ __forceinline__ double substep_dp(const ThermoConsts& t, const double* tab, const CellState& s, double T) {
+template <bool EVEN>
+__device__ __forceinline__ double substep_dp(const RateConsts<EVEN>& t, const double* tab, const CellState& s, double T) {
     const double r = subtract_cooling(t, s.cc, tab, s.heat, T);
     return t.heating_amplification * soft_landing(r, T, s.T_min) * s.rate2dpre;
 }
@@ -292,7 +296,8 @@ __device__ __forceinline__ double substep_dp(const ThermoConsts& t, const double
 // long subcycles (the explicit steps resolve the evolution) this is close to
 // the subcycle's own result; what remains is learned by the network.
 constexpr int COARSE_STEPS = 512;
-__device__ __forceinline__ double coarse_end_temperature(const ThermoConsts& t, const double* tab, const CellState& s) {
+template <bool EVEN>
+__device__ __forceinline__ double coarse_end_temperature(const RateConsts<EVEN>& t, const double* tab, const CellState& s) {
     double p = s.pressure;
     double kleft = (double)s.remaining;
     for (int it = 0; it < COARSE_STEPS && kleft > 0.0; ++it) {
@@ -404,7 +409,8 @@ __device__ __forceinline__ void apply_cell(const HydroGeom& g, double u[7], doub
 // A cell whose subcycle is longer than the exact limit: the coarse end
 // temperature, its raw features and the training-envelope test, which
 // route it to the network (to_mlp) or the FP64 fallback (to_fb).
-__device__ __forceinline__ void route_active(const ThermoConsts& t, const double* tab, const SurrogateConsts& sc, const double* cin,
+template <bool EVEN>
+__device__ __forceinline__ void route_active(const RateConsts<EVEN>& t, const double* tab, const SurrogateConsts& sc, const double* cin,
                                              long long cstride, long long ccell, const CellState& s, double& Tc,
                                              double u[8], bool& to_mlp, bool& to_fb) {
     Tc = coarse_end_temperature(t, tab, s);
@@ -485,8 +491,8 @@ constexpr int COARSE_LONG = 64;
 // three waves per SIMD, 160 registers without spills; two and four waves (7
 // spilled registers) measured slower.
 enum PrepassMode { PRE_ROUTE, PRE_DEFER, PRE_FALLBACK };
-template <bool GRID, PrepassMode MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 4))) void surrogate_prepass_kernel(ThermoConsts t, const double* __restrict__ tables,
+template <bool GRID, PrepassMode MODE, bool EVEN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 4))) void surrogate_prepass_kernel(RateConsts<EVEN> t, const double* __restrict__ tables,
                                                                SurrogateConsts sc, long long n,
                                                                double* __restrict__ in, double* __restrict__ out,
                                                                unsigned char* path, long long* __restrict__ mlp_list,
@@ -571,8 +577,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID ? 3 : 
 // per workgroup, so that a few hundred waves of such cells spread over all
 // CUs, and two waves per SIMD, which leave the coarse loop's registers
 // unspilled.
+template <bool EVEN>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void surrogate_long_kernel(
-    ThermoConsts t, const double* __restrict__ tables, SurrogateConsts sc, long long n, const double* __restrict__ in,
+    RateConsts<EVEN> t, const double* __restrict__ tables, SurrogateConsts sc, long long n, const double* __restrict__ in,
     unsigned char* path, long long* __restrict__ mlp_list, float* __restrict__ feat, SurrCell* __restrict__ sdata,
     long long* __restrict__ fb_list, unsigned long long* __restrict__ counters,
     const long long* __restrict__ long_list, unsigned int* __restrict__ err) {
@@ -714,8 +721,8 @@ __global__ void thermo_gather_kernel(GridSrc gs, double* __restrict__ in9) {
 // and a maximum, which any order of reduction gives bitwise); with rate_out,
 // each cell's heating rate and pre-step RATE ([2][n]) for a cooling sub-step
 // on the same state (thermo_init's pre_rate).
-template <bool GRID>
-__global__ __launch_bounds__(256) void thermo_timestep_kernel(ThermoConsts t, const double* __restrict__ tables,
+template <bool GRID, bool EVEN>
+__global__ __launch_bounds__(256) void thermo_timestep_kernel(RateConsts<EVEN> t, const double* __restrict__ tables,
                                                              long long n, const double* __restrict__ in9,
                                                              unsigned long long* __restrict__ dtmin_bits,
                                                              unsigned int* __restrict__ err, GridSrc gs,
@@ -727,7 +734,7 @@ __global__ __launch_bounds__(256) void thermo_timestep_kernel(ThermoConsts t, co
     double mc = 0.0;
     for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (long long)gridDim.x * blockDim.x) {
         CellState s;
-        ThermoConsts t1 = t;
+        RateConsts<EVEN> t1 = t;
         t1.subcycling = 0;  // pre-step rate only
         double lin[9], lu[7], lq[7];
         const double* cin = in9;
@@ -874,8 +881,9 @@ constexpr int LPT_NB = 64;
 constexpr unsigned char LPT_DONE = 255;
 constexpr int SHORT_STEPS = 8;
 
+template <bool EVEN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lpt_bucket_kernel(
-    ThermoConsts t, const double* __restrict__ tables, long long stride, long long count,
+    RateConsts<EVEN> t, const double* __restrict__ tables, long long stride, long long count,
     const unsigned long long* __restrict__ count_dev, const long long* __restrict__ list, const double* __restrict__ in,
     double* __restrict__ out, unsigned char* path, unsigned char* __restrict__ bucket,
     unsigned long long* __restrict__ hist, unsigned long long* __restrict__ counters, unsigned int* __restrict__ err) {
@@ -915,7 +923,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
 // the first, fixed by the pre-step rate): 0 for a cell that is not
 // subcycled, -1 where dt / dti is beyond the int range.  Nothing is
 // integrated and no error is raised.
-__global__ __launch_bounds__(256) void subcycle_count_kernel(ThermoConsts t, const double* __restrict__ tables,
+template <bool EVEN>
+__global__ __launch_bounds__(256) void subcycle_count_kernel(RateConsts<EVEN> t, const double* __restrict__ tables,
                                                             long long n, const double* __restrict__ in,
                                                             long long* __restrict__ count) {
     __shared__ double tab[TT_N];
@@ -970,6 +979,7 @@ __global__ __launch_bounds__(256) void lpt_scatter_kernel(long long count, const
 struct torchgpu_cooling {
     torchgpu_thermo_params p;
     tg::ThermoConsts t;
+    bool spl_even = true;                     // see tg::RateConsts
     hipStream_t stream = nullptr;
     double* tables = nullptr;                 // spline x, y, y2 (78 doubles), then the rate tables (TT_N)
     unsigned long long* counters = nullptr;   // [0] work, [1] subcycles, [2] surrogate queue, [3] fallback queue,
@@ -1085,6 +1095,13 @@ static void fill_rate_tables(const torchgpu_thermo_params& p, double* tab) {
 
 namespace {
 
+// launch(constants), as the kernels for the handle's spline take them
+template <class F>
+void with_rates(const torchgpu_cooling* c, F launch) {
+    if (c->spl_even) launch(tg::RateConsts<true>{c->t});
+    else launch(tg::RateConsts<false>{c->t});
+}
+
 tg::ThermoConsts to_consts(const torchgpu_thermo_params& p) {
     tg::ThermoConsts t{};
     t.thermo_hii_switch = p.thermo_hii_switch;
@@ -1105,9 +1122,6 @@ tg::ThermoConsts to_consts(const torchgpu_thermo_params& p) {
     t.spl_max_slope = p.spl_max_slope;
     t.icxhi = 1.0 / p.cxhi_damp;
     t.spl_k0 = 1.0 - 10.0 * p.spl_x[0];
-    t.spl_even = 1;
-    for (int k = 1; k < 26; ++k)
-        if (!(std::fabs(p.spl_x[k] - (p.spl_x[0] + 0.1 * k)) < 1.0e-9)) t.spl_even = 0;
     t.subcycling = p.subcycling;
     return t;
 }
@@ -1134,8 +1148,11 @@ int integrate(torchgpu_cooling* c, long long stride, long long count, const unsi
     const long long most = (long long)c->nsm * 16;
     if (blocks > most) blocks = most;
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(tg::lpt_bucket_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, c->t, c->tables,
-                       stride, count, count_dev, list, in, out, path, bucket, hist, c->counters, c->err);
+    with_rates(c, [&](auto t) {
+        hipLaunchKernelGGL((tg::lpt_bucket_kernel<decltype(t)::even>),
+                           dim3((unsigned)blocks), dim3(256), 0, c->stream, t, c->tables,
+                           stride, count, count_dev, list, in, out, path, bucket, hist, c->counters, c->err);
+    });
     HIP_OK(hipGetLastError());
     hipLaunchKernelGGL(tg::lpt_offsets_kernel, dim3(1), dim3(64), 0, c->stream, hist, hist + tg::LPT_NB);
     HIP_OK(hipGetLastError());
@@ -1145,9 +1162,12 @@ int integrate(torchgpu_cooling* c, long long stride, long long count, const unsi
     blocks = (count + 255) / 256;
     if (blocks > (long long)c->nsm * 8) blocks = (long long)c->nsm * 8;  // 32 waves per CU
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(tg::thermo_cells_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, c->t, c->tables,
-                       stride, count, (const unsigned long long*)hist, order, in, out, c->counters, c->err, path,
-                       list ? 2 : 0);
+    with_rates(c, [&](auto t) {
+        hipLaunchKernelGGL((tg::thermo_cells_kernel<decltype(t)::even>),
+                           dim3((unsigned)blocks), dim3(256), 0, c->stream, t, c->tables,
+                           stride, count, (const unsigned long long*)hist, order, in, out, c->counters, c->err, path,
+                           list ? 2 : 0);
+    });
     HIP_OK(hipGetLastError());
     return TORCHGPU_OK;
 }
@@ -1256,6 +1276,8 @@ int torchgpu_cooling_create(const torchgpu_thermo_params* p, void* stream, torch
     torchgpu_cooling* c = new torchgpu_cooling();
     c->p = *p;
     c->t = to_consts(*p);
+    for (int k = 1; k < 26; ++k)
+        if (!(std::fabs(p->spl_x[k] - (p->spl_x[0] + 0.1 * k)) < 1.0e-9)) c->spl_even = false;
     c->stream = (hipStream_t)stream;  // NULL: the null (default) stream
     double tab[78 + tg::TT_N];
     for (int i = 0; i < 26; ++i) { tab[i] = p->spl_x[i]; tab[26 + i] = p->spl_y[i]; tab[52 + i] = p->spl_y2[i]; }
@@ -1359,8 +1381,11 @@ int torchgpu_thermo_subcycles(torchgpu_cooling* c, int64_t n, const double* in, 
     if (n == 0) return TORCHGPU_OK;
     long long nb = (n + 255) / 256;
     if (nb > 65536) nb = 65536;
-    hipLaunchKernelGGL(tg::subcycle_count_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, c->t, c->tables, n, in,
-                       (long long*)count);
+    with_rates(c, [&](auto t) {
+        hipLaunchKernelGGL((tg::subcycle_count_kernel<decltype(t)::even>),
+                           dim3((unsigned)nb), dim3(256), 0, c->stream, t, c->tables, n, in,
+                           (long long*)count);
+    });
     HIP_OK(hipGetLastError());
     return TORCHGPU_OK;
 }
@@ -1401,10 +1426,13 @@ static int fp64_grid_step(torchgpu_cooling* c, int64_t n, double* in, double* ou
     sc.nexact = tg::SHORT_STEPS;
     long long nb = (n + 255) / 256;
     if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
-    hipLaunchKernelGGL((tg::surrogate_prepass_kernel<true, tg::PRE_FALLBACK>), dim3((unsigned)nb), dim3(256), 0,
-                       c->stream, c->t, c->tables, sc, (long long)n, in, out, path, (long long*)nullptr,
-                       (float*)nullptr, (tg::SurrCell*)nullptr, (float*)nullptr, c->fb_list, c->counters, c->err, gs,
-                       apply.U, apply.qf, apply.st, (long long*)nullptr, apply.pre_rate);
+    with_rates(c, [&](auto t) {
+        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<true, tg::PRE_FALLBACK, decltype(t)::even>),
+                           dim3((unsigned)nb), dim3(256), 0,
+                           c->stream, t, c->tables, sc, (long long)n, in, out, path, (long long*)nullptr,
+                           (float*)nullptr, (tg::SurrCell*)nullptr, (float*)nullptr, c->fb_list, c->counters, c->err, gs,
+                           apply.U, apply.qf, apply.st, (long long*)nullptr, apply.pre_rate);
+    });
     HIP_OK(hipGetLastError());
     return integrate_own(c, n, n, c->counters + 3, c->fb_list, in, out, path);
 }
@@ -1429,22 +1457,31 @@ static int surrogate_step(torchgpu_cooling* c, int64_t n, double* in, double* ou
     long long nb = (n + 255) / 256;
     if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
     if (gs)
-        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<true, tg::PRE_DEFER>), dim3((unsigned)nb), dim3(256), 0, c->stream, c->t,
-                           c->tables, sc, (long long)n, in, out, path, c->mlp_list, c->feat, c->sdata, (float*)nullptr,
-                           c->fb_list, c->counters, c->err, *gs, apply->U, apply->qf, apply->st, c->long_list,
-                           apply->pre_rate);
+        with_rates(c, [&](auto t) {
+            hipLaunchKernelGGL((tg::surrogate_prepass_kernel<true, tg::PRE_DEFER, decltype(t)::even>),
+                               dim3((unsigned)nb), dim3(256), 0, c->stream, t,
+                               c->tables, sc, (long long)n, in, out, path, c->mlp_list, c->feat, c->sdata, (float*)nullptr,
+                               c->fb_list, c->counters, c->err, *gs, apply->U, apply->qf, apply->st, c->long_list,
+                               apply->pre_rate);
+        });
     else
-        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, tg::PRE_DEFER>), dim3((unsigned)nb), dim3(256), 0, c->stream,
-                           c->t, c->tables, sc, (long long)n, in, out, path, c->mlp_list, c->feat, c->sdata,
-                           (float*)nullptr, c->fb_list, c->counters, c->err, tg::GridSrc{}, (double*)nullptr,
-                           (float*)nullptr, (tg::StepState*)nullptr, c->long_list, (const double*)nullptr);
+        with_rates(c, [&](auto t) {
+            hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, tg::PRE_DEFER, decltype(t)::even>),
+                               dim3((unsigned)nb), dim3(256), 0, c->stream,
+                               t, c->tables, sc, (long long)n, in, out, path, c->mlp_list, c->feat, c->sdata,
+                               (float*)nullptr, c->fb_list, c->counters, c->err, tg::GridSrc{}, (double*)nullptr,
+                               (float*)nullptr, (tg::StepState*)nullptr, c->long_list, (const double*)nullptr);
+        });
     HIP_OK(hipGetLastError());
     // the cells the prepass deferred (many remaining subcycles), densely
     long long nb64 = (n + 63) / 64;
     if (nb64 > (long long)c->nsm * 64) nb64 = (long long)c->nsm * 64;
-    hipLaunchKernelGGL(tg::surrogate_long_kernel, dim3((unsigned)nb64), dim3(64), 0, c->stream, c->t, c->tables, sc,
-                       (long long)n, (const double*)in, path, c->mlp_list, c->feat, c->sdata, c->fb_list, c->counters,
-                       (const long long*)c->long_list, c->err);
+    with_rates(c, [&](auto t) {
+        hipLaunchKernelGGL((tg::surrogate_long_kernel<decltype(t)::even>),
+                           dim3((unsigned)nb64), dim3(64), 0, c->stream, t, c->tables, sc,
+                           (long long)n, (const double*)in, path, c->mlp_list, c->feat, c->sdata, c->fb_list, c->counters,
+                           (const long long*)c->long_list, c->err);
+    });
     HIP_OK(hipGetLastError());
     HIP_OK(tg::launch_mlp_infer_dev(w16, b, c->feat, c->counters + 2, n, c->y, c->nsm, c->stream));
     hipLaunchKernelGGL(tg::surrogate_finish_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, c->t, sc,
@@ -1492,11 +1529,14 @@ int torchgpu_surrogate_training_data(torchgpu_cooling* c, int64_t n, const doubl
     };
     long long nb = (n + 255) / 256;
     if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
-    hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, tg::PRE_ROUTE>), dim3((unsigned)nb), dim3(256), 0, c->stream,
-                       c->t, c->tables, sc, (long long)n, const_cast<double*>(in), scratch, (unsigned char*)nullptr,
-                       (long long*)list, feat, c->sdata, raw, c->fb_list, c->counters, c->err, tg::GridSrc{},
-                       (double*)nullptr, (float*)nullptr, (tg::StepState*)nullptr, (long long*)nullptr,
-                       (const double*)nullptr);
+    with_rates(c, [&](auto t) {
+        hipLaunchKernelGGL((tg::surrogate_prepass_kernel<false, tg::PRE_ROUTE, decltype(t)::even>),
+                           dim3((unsigned)nb), dim3(256), 0, c->stream,
+                           t, c->tables, sc, (long long)n, const_cast<double*>(in), scratch, (unsigned char*)nullptr,
+                           (long long*)list, feat, c->sdata, raw, c->fb_list, c->counters, c->err, tg::GridSrc{},
+                           (double*)nullptr, (float*)nullptr, (tg::StepState*)nullptr, (long long*)nullptr,
+                           (const double*)nullptr);
+    });
     keep(hipGetLastError());
     if (e == hipSuccess) {
         hipLaunchKernelGGL(tg::surrogate_targets_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, c->counters,
@@ -1607,9 +1647,12 @@ static int grid_timestep_dev(torchgpu_ctx* ctx, torchgpu_cooling* c, const doubl
     hipLaunchKernelGGL(tg::set_u64_kernel, dim3(1), dim3(1), 0, c->stream, c->dtbits, 0x7fefffffffffffffull);
     long long nb = (n + 255) / 256;
     if (nb > (long long)c->nsm * 16) nb = (long long)c->nsm * 16;
-    hipLaunchKernelGGL(tg::thermo_timestep_kernel<true>, dim3((unsigned)nb), dim3(256), 0, c->stream, c->t,
-                       c->tables, n, (const double*)nullptr, c->dtbits, c->err, gs, cfl_st,
-                       keep_rate && *keep_rate ? c->rcache : (double*)nullptr);
+    with_rates(c, [&](auto t) {
+        hipLaunchKernelGGL((tg::thermo_timestep_kernel<true, decltype(t)::even>),
+                           dim3((unsigned)nb), dim3(256), 0, c->stream, t,
+                           c->tables, n, (const double*)nullptr, c->dtbits, c->err, gs, cfl_st,
+                           keep_rate && *keep_rate ? c->rcache : (double*)nullptr);
+    });
     HIP_OK(hipGetLastError());
     return TORCHGPU_OK;
 }

@@ -23,7 +23,16 @@ struct ThermoConsts {
     double icxhi;  // 1 / cxhi_damp
     double spl_k0; // 1 - 10 spl_x[0]: the spline piece at log10 T is 10 log10 T + spl_k0
     int subcycling;
-    int spl_even;  // the abscissae are spl_x[0] + k / 10 to 1e-9
+    int pad;
+};
+
+// The constants as the rate functions take them.  EVEN: the spline's abscissae
+// are spl_x[0] + k / 10 to 1e-9.  A kernel is built for both (chosen at
+// launch): the test and its uneven branch inside the rate took 3 % of a lone
+// wave's subcycle.
+template <bool EVEN>
+struct RateConsts : ThermoConsts {
+    static constexpr bool even = EVEN;
 };
 
 // ---------------------------------------------------------------------------
@@ -38,7 +47,7 @@ struct ThermoConsts {
 // chain (double-double); these take 16 and 17 and keep an error of 0.53 and
 // 0.51 ulp, and the spline's three divides go.  A subcycle (the integrator's
 // whole trip: rate, floors, bookkeeping) went from about 650 vector
-// instructions to 155, and 215 above ciec_minT (230 and 305 with the scalar and
+// instructions to 150, and 210 above ciec_minT (225 and 300 with the scalar and
 // LDS ones).
 // ---------------------------------------------------------------------------
 constexpr int TT_EXP = 0, TT_EXP_LO = 128, TT_C = 256, TT_LHI = 384, TT_LLO = 512, TT_SPL = 640, TT_NSPL = 27;
@@ -141,13 +150,14 @@ __device__ __forceinline__ double rcp_t(double x) {
 // where they are not that even.  The spline is steep (20 decades in 1.5 of T):
 // the offset from the knot is formed from both parts, or the rounding of log10
 // T alone would be 2e-14 of the rate.
-__device__ __forceinline__ double log_spline_t(const ThermoConsts& t, const double* tab, double hi, double lo) {
+template <bool EVEN>
+__device__ __forceinline__ double log_spline_t(const RateConsts<EVEN>& t, const double* tab, double hi, double lo) {
     const double x = hi * 0x1.bcb7b1526e50ep-2;
     const double xl = __builtin_fma(lo, 0x1.bcb7b1526e50ep-2,
                                     __builtin_fma(hi, 0x1.95355baaafad3p-57, __builtin_fma(hi, 0x1.bcb7b1526e50ep-2, -x)));
     int k = (int)__builtin_fma(x + xl, 10.0, t.spl_k0);  // 0 below the first knot, 26 from the last on
     k = k < 0 ? 0 : (k > TT_NSPL - 1 ? TT_NSPL - 1 : k);
-    if (__builtin_expect(!t.spl_even, 0)) {  // piece 0 starts at knot 0, piece j at knot j - 1
+    if (!EVEN) {  // piece 0 starts at knot 0, piece j at knot j - 1
         const double* knot = tab + TT_SPL + 1;
         const double v = x + xl;
         k = k < 1 ? 1 : (k > TT_NSPL - 2 ? TT_NSPL - 2 : k);
@@ -189,11 +199,10 @@ __device__ __forceinline__ double soft_landing(double rate, double T, double T_m
     if (rate < 0.0) {
         if (T <= T_min) result = 0;
         else if (T <= T_min + 200) {
-            // rate (T - T_min) / 200, rounded as the division rounds it; the
-            // correction of an infinite q is NaN
+            // rate (T - T_min) / 200, rounded as the division rounds it; an
+            // infinite product's remainder, NaN, is replaced by a finite value
             const double x = rate * (T - T_min), q = x * 0.005;
-            const double r = __builtin_fma(__builtin_fma(-200.0, q, x), 0.005, q);
-            result = r == r ? r : q;
+            result = __builtin_fma(fmin(__builtin_fma(-200.0, q, x), 1.0e300), 0.005, q);
         }
     }
     return result;
@@ -227,8 +236,9 @@ __device__ __forceinline__ CoolingCell cooling_cell(const ThermoConsts& t, const
 // reciprocal, a square or e^(1.63 ln T) leaves the double range and meets its
 // opposite as 0 x infinity.  Each term by its own exponential, whose exponent
 // is clamped where the result is 0 or infinity anyway.
-__device__ __forceinline__ double subtract_cooling_far(const ThermoConsts& t, const CoolingCell& c, const double* tab,
-                                                       double rate, double T) {
+template <bool EVEN>
+__device__ __forceinline__ double subtract_cooling_far(const RateConsts<EVEN>& t, const CoolingCell& c,
+                                                       const double* tab, double rate, double T) {
     if (!(T > 0.0)) return T == 0.0 ? rate : __builtin_nan("");  // all terms vanish towards 0; no rate below it, or of NaN
     if (T > 0x1.fffffffffffffp1023) return rate - c.imlc_k - c.nmlc_k - c.nmc_k * T;
     const double iT = 1.0 / T;
@@ -255,7 +265,8 @@ __device__ __forceinline__ double subtract_cooling_far(const ThermoConsts& t, co
 // ciec_minT) instead of ten libm calls.  The values differ from the
 // reference's by rounding of the exponents only (relative ~1e-15 on each
 // term).
-__device__ __forceinline__ double subtract_cooling(const ThermoConsts& t, const CoolingCell& c, const double* tab,
+template <bool EVEN>
+__device__ __forceinline__ double subtract_cooling(const RateConsts<EVEN>& t, const CoolingCell& c, const double* tab,
                                                    double rate, double T) {
     if (!(T >= 1e-100 && T <= 1e100)) return subtract_cooling_far(t, c, tab, rate, T);
     const double iT = rcp_t(T);
