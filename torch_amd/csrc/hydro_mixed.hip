@@ -28,7 +28,7 @@
 // stage and (corrector) its CFL term.  34 KB LDS, 128 VGPRs: four waves per
 // SIMD, four workgroups per CU (neither the registers nor the LDS allow a
 // fifth).  Bound by vector instructions: 1,360 (predictor) and 1,440 per cell and
-// stage, issued 0.80 and 0.85 of the time at 512^3, 0.71 and 0.76 at 256^3 (0.8
+// stage, issued 0.81 and 0.86 of the time at 512^3, 0.71 and 0.75 at 256^3 (0.9
 // ms per stage), and beside them the transcendentals' extra cycles.
 //
 // FP32 range: the float state is the FP64 state scaled by powers of two,
