@@ -104,6 +104,59 @@ def test_cooling_spline_takes_its_own_abscissae(gpu, orc, knots):
     assert err.max() < 1e-12, (err.max(), T[err.argmax()])
 
 
+def test_uneven_spline_in_every_kernel(gpu, orc):
+    """The kernels' instances for an uneven spline table: the integrator and the
+    subcycle counts on cells that subcycle, against the oracle; the grid's time
+    step and FP64 sub-step (inputs formed in the kernel) against the same on
+    gathered inputs (heating record on)."""
+    import torch
+
+    from torch_amd import cloud
+    from torch_amd import surrogate as sg
+
+    k = np.arange(26)
+    x = 3.5 + 0.1 * k + 0.04 * np.sin(2.1 * k)
+    c = orc.converter(1e-20, 1e-28, 1e11)
+    tc = lambda v, m, l, t: orc.to_code(c, v, m, l, t)  # noqa: E731
+    p = gpu.thermo_params()
+    t = orc.thermo_params(c, pfloor=p.pfloor)
+    for i in range(26):
+        t.spl_x[i] = p.spl_x[i] = x[i]
+    inp = cooling_inputs.to_code_inputs(cooling_inputs.sample_cgs(2048, seed=5), tc)
+    cool = gpu.Cooling(p)
+    cnt = sg.subcycles(cool, torch.from_numpy(np.ascontiguousarray(inp.T)).cuda()).cpu().numpy()
+    inp = np.ascontiguousarray(inp[(cnt >= 0) & (cnt <= 20000)])
+    ref = orc.thermo_batch(t, inp, nthreads=8)
+    dev = torch.from_numpy(np.ascontiguousarray(inp.T)).cuda()
+    np.testing.assert_array_equal(sg.subcycles(cool, dev).cpu().numpy(), ref[:, 3])
+    assert (ref[:, 3] > 8).sum() > 100
+    out, _ = cool.thermo_cells(dev)
+    rel = np.abs(out[4].cpu().numpy() - ref[:, 4]) / np.abs(ref[:, 4])
+    assert np.median(rel) < 1e-14 and rel.max() < 1e-6, np.quantile(rel, [0.5, 0.99, 1.0])
+    got = []
+    for track in (False, True):
+        gp, g, own, thermo = cloud.build(24, "fp64")
+        Q = cloud.setup(24, tc)[0].copy()
+        Q[1] *= 40.0    # 300 K to some 1e4 K, half ionised: the spline's term is the largest
+        Q[2] = 0.5
+        g.set_primitive(np.ascontiguousarray(Q))
+        if track:
+            g.heating_track(True)
+        grid_p = gpu.thermo_params()
+        grid_p.pfloor = gp.pfloor
+        for i in range(26):
+            grid_p.spl_x[i] = x[i]
+        gc = gpu.Cooling(grid_p)
+        dt = gc.grid_timestep(g, gp.dt_max, **thermo)
+        assert dt != own.grid_timestep(g, gp.dt_max, **thermo)   # the table matters on this state
+        gc.grid_substep(g, 100.0 * dt, **thermo)
+        g.synchronize()
+        got.append((dt, g.get_conserved()))
+        g.close()
+    assert got[0][0] == got[1][0]
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+
+
 def test_cooling_rate_of_extreme_temperatures(gpu, orc):
     """Pre-step rates of neutral, half and fully ionised cells from 1e-300 to
     1e290 K (and some at the operator's own temperatures) against the
